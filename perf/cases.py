@@ -289,8 +289,8 @@ def _block_inputs(case, seed):
     B, T = case["B"], case["T"]
     factor = _factors(g, B)
     layers = [(n, *_operands(g, B, T, i, o, factor, 4)) for n, i, o in _block_layers(case)]
-    norms = {f"{n}.weight": _randn(g, (B, case["d"]), factor[:, None] * (0.01 / math.sqrt(case["d"])))
-             for n in ("attn_norm", "mlp_norm")}
+    scale = factor[:, None] * (0.01 / math.sqrt(case["d"]))
+    norms = {f"{n}.weight": _randn(g, (B, case["d"]), scale) for n in ("attn_norm", "mlp_norm")}
     return {"layers": layers, "norms": norms}
 
 
@@ -463,8 +463,9 @@ def run(state):
 
 # About four times what the outputs differ by from the 64-bit result.  With 16-bit operands
 # that is the clip factor's safety margin (the rounding of 16-bit gradients that it allows
-# for, up to 0.5%, and a rounding bound of the norm, up to 1% at the longest sequences) where no noise covers it, and the outputs'
-# own rounding; with float32 it is the order of the sums (and the normals' own 1e-6).
+# for, up to 0.5%, and a rounding bound of the norm, up to 1% at the longest sequences) where
+# no noise covers it, and the outputs' own rounding; with float32 it is the order of the sums
+# (and the normals' own 1e-6).
 _TOLERANCE = {"linear": {"bf16": 2e-2, "fp32": 1e-5}, "block": 4e-2, "lora": 2e-2, "moe": 2e-2,
               "mlp": 1e-5, "leaves": {"bf16": 2e-2, "fp16": 4e-3, "fp32": 4e-6},
               "noise": {"bf16": 7e-3, "fp32": 4e-6}}
