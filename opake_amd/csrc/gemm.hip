@@ -3,7 +3,8 @@
 // as one GEMM over K = B * T with the normalisation and the Gaussian noise
 // fused into the epilogue.
 //
-// Fast path (bf16, T % 64 == 0, din % 8 == 0, dout % 8 == 0):
+// Fast path (bf16, T > 1; operands whose width is not a multiple of 8 are first
+// copied into rows padded to one):
 //   * 256 x 256 output tile per workgroup, 8 waves (2 per SIMD) of 128 x 64,
 //     bf16 MFMA 16x16x32 with fp32 accumulators (32 blocks per wave);
 //   * both operands are m- (n-) contiguous in HBM and are staged into LDS in
@@ -12,7 +13,8 @@
 //     need 8 consecutive k per lane, come out of LDS through the gfx950
 //     transposing read ds_read_b64_tr_b16 (two per fragment), so no data is
 //     transposed in registers; all LDS accesses are free of bank conflicts;
-//   * a K step is 64 deep and never straddles two examples, so the
+//   * a K step is 64 deep and never straddles two examples (with T % 64 != 0
+//     an example's last step is a partial one, kRagged), so the
 //     per-example scale is one scalar per step.  Dense mode applies it to the
 //     fp32 accumulators: they hold the partial sum divided by the current
 //     example's scale and are multiplied by scale_prev / scale_next where the
@@ -320,17 +322,22 @@ struct DenseProblem {
 };
 
 struct FastArgs {
-  const uint16_t* A;  // [B * T, N] (dense mode)
-  const uint16_t* G;  // [B * T, M]
+  const uint16_t* A;  // [B * T, lda] (dense mode)
+  const uint16_t* G;  // [B * T, ldg]
+  // Row lengths of A and G (kRagged, one layer): N and M, or the next
+  // multiples of 8 where the operand was copied into padded rows.
+  int lda, ldg;
   int T, B;
   const void* plan;
   const float* scale;
   Epilogue ep;
   GroupedTables grp;
   // Dense split-K: workgroup (split, tile) takes steps
-  // [split * n / splits, (split + 1) * n / splits) of the n steps and, for
-  // splits > 1, writes its raw fp32 tile to partial[split] ([M][N]); the
-  // reduce kernel adds the splits in order and applies the epilogue.
+  // [split * n / splits, (split + 1) * n / splits) of the n steps and, with
+  // `partial` (always given for splits > 1 and for an odd ep.N, which the
+  // kernel's own epilogue does not take), writes its raw fp32 tile to
+  // partial[split] ([ldg][lda]); the reduce kernel adds the splits in order
+  // and applies the epilogue.
   int splits;
   float* partial;
   // Dense multi-layer mode when nprob > 0 (splits is then 1; A, G and the
@@ -364,7 +371,14 @@ __shared__ __attribute__((aligned(16))) uint8_t lds_a1[kOperandBytes];
 // higher clock than 32x32x16 on the same data, and 8 waves measure faster
 // than 4 waves of 128 x 128 whose 256 accumulators per lane leave too few
 // registers for the pipeline.)
-template <bool kGrouped, bool kGdma, int kWaves, bool kHalfDma = false>
+//
+// kRagged (dense): T is not a multiple of 64, so an example's last step holds
+// fewer than 64 rows; the rows past its end are fetched out of range (zeros)
+// and the MFMAs of a sub-step that holds none are skipped, as in grouped mode.
+// [24, 197, 768 x 3072] takes 48 us (and 9 for its split-K sum) against 1067 in the generic kernel (15
+// TFLOP/s there: its 4 x 4 FMA blocks are bound by LDS reads); what is left
+// is the 36 tiles' split-K traffic and the 23% of the last steps' empty rows.
+template <bool kGrouped, bool kGdma, int kWaves, bool kHalfDma = false, bool kRagged = false>
 __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
   constexpr int kT = kWaves * 64;           // threads
   constexpr int kWavesN = kWaves / 2;       // waves along the tile columns
@@ -379,7 +393,12 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
   // kHalfDma's DMA waves step kWaves rows per instruction: the same swizzle
   // (row & 7) for every instruction needs kWaves % 8 == 0.
   static_assert(!kHalfDma || (!kGrouped && kWaves % 8 == 0), "half-wave DMAs: dense, 8k waves");
-  int M = args.ep.M, N = args.ep.N;
+  static_assert(!kRagged || (!kGrouped && !kHalfDma), "ragged steps: dense, all waves issue DMAs");
+  constexpr bool kPartial = kGrouped || kRagged;  // a step may hold fewer than kBK rows
+  // The operands' row lengths: the output's shape, except where kRagged reads
+  // padded copies (outputs past ep.M, ep.N are not stored).
+  int M = kRagged && args.nprob == 0 ? args.ldg : args.ep.M;
+  int N = kRagged && args.nprob == 0 ? args.lda : args.ep.N;
   const int T = args.T;
   int lin = xcd_linear_id(gridDim.x);
   Epilogue ep = args.ep;
@@ -426,8 +445,23 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
   const int wm = w / kWavesN, wn = w % kWavesN;  // wave tile: rows wm * 128, columns wn * kWC
 
   int total_rows, nsteps, step0 = 0, nactive = 0, nfast = 0, step_base = 0;
-  const int spe = T / kBK;
+  const int spe = kRagged ? (T + kBK - 1) / kBK : T / kBK;
   ClipPlanView plan = clip_plan_view(const_cast<void*>(args.plan), args.B);
+  // Rows past a step's `valid` are fetched out of range (zero in the G tile);
+  // the A tile starts from zeros so that whatever such a fetch leaves in LDS
+  // is finite.
+  auto zero_stages = [&]() __attribute__((always_inline)) {
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    for (int i = tid * 16; i < kOperandBytes; i += kT * 16) {
+      *reinterpret_cast<u32x4_t*>(lds_a0 + i) = zero;
+      *reinterpret_cast<u32x4_t*>(lds_a1 + i) = zero;
+      if constexpr (kGdma) {
+        *reinterpret_cast<u32x4_t*>(lds_g0 + i) = zero;
+        *reinterpret_cast<u32x4_t*>(lds_g1 + i) = zero;
+      }
+    }
+    __syncthreads();
+  };
   if (kGrouped) {
     // Table entries of the (uniform) problem, read into scalar registers: the
     // compiler loads them into vector registers, and a buffer resource built
@@ -446,20 +480,9 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
     if (args.grp.noise_ptrs) ep.noise = reinterpret_cast<const float*>(args.grp.noise_ptrs[grp]);
     ep.leaf = args.grp.leaf_ids[grp];
     ep.sigma = ep.noise_mode == DPC_NOISE_NONE ? 0.0f : args.grp.sigmas[grp];
-    // Rows past a step's `valid` are fetched out of range (zero in the G tile);
-    // the A tile starts from zeros so that whatever such a fetch leaves in LDS
-    // is finite.
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    for (int i = tid * 16; i < kOperandBytes; i += kT * 16) {
-      *reinterpret_cast<u32x4_t*>(lds_a0 + i) = zero;
-      *reinterpret_cast<u32x4_t*>(lds_a1 + i) = zero;
-      if constexpr (kGdma) {
-        *reinterpret_cast<u32x4_t*>(lds_g0 + i) = zero;
-        *reinterpret_cast<u32x4_t*>(lds_g1 + i) = zero;
-      }
-    }
-    __syncthreads();
+    zero_stages();
   } else {
+    if constexpr (kRagged) zero_stages();
     nactive = *plan.nactive;
     nfast = *plan.nfast;
     const long long all = (long long)nfast * spe;
@@ -506,7 +529,8 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         plan_sc = sl < nfast ? args.scale[plan_ex] : 0.0f;
       }
     };
-    // Dense: step t covers rows [active[t / spe] * T + (t % spe) * 64, +64).
+    // Dense: step t covers rows [active[t / spe] * T + (t % spe) * 64, +64),
+    // kRagged: those of them before the example's end.
     // Grouped: step t is table entry step0 + t.
     auto step_row0 = [&](int t, float* sc, int* valid) __attribute__((always_inline)) {
       t += step_base;  // dense split-K: this workgroup's first step
@@ -522,8 +546,9 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         *valid = __builtin_amdgcn_readlane(plan_pack, slot - plan_base) & 127;
         return ex;
       }
-      *valid = kBK;
-      return ex * T + (t % spe) * kBK;
+      const int r = (t % spe) * kBK;
+      *valid = kRagged ? min(kBK, T - r) : kBK;
+      return ex * T + r;
     };
 
     // G staging: chunk j (< kGC) of this thread is tile row r0 + kRowsPerPass j,
@@ -537,7 +562,7 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
     u32x4_t g[kGC];
     auto load_chunk = [&](int row0, int valid, int j) __attribute__((always_inline)) {
       const int row = row0 + r0;
-      const int bad = (kGrouped && r0 + kRowsPerPass * j >= valid) ? kOutOfRange : g_bad;
+      const int bad = (kPartial && r0 + kRowsPerPass * j >= valid) ? kOutOfRange : g_bad;
       g[j] = __builtin_amdgcn_raw_buffer_load_b128(g_rsrc, (row * M * 2 + g_voff) | bad,
                                                    j * kRowsPerPass * M * 2, 0);
     };
@@ -554,11 +579,11 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
     // instruction j only adds the uniform 2 kWaves j rows.
     // Grouped mode: rows past the step's `valid` and chunks whose columns lie
     // past the matrix are given an out-of-range offset (read as zero).  Dense
-    // mode: every row is valid, and a chunk past the matrix reads the row's
-    // last 8 columns instead -- they feed only output rows (columns) that are
-    // never stored -- so every transfer is in range, the per-lane offset is
-    // fixed, and the row offset of the step and instruction is the uniform
-    // soffset.
+    // mode: every row is valid (kRagged: rows past `valid` get an out-of-range
+    // offset), and a chunk past the matrix reads the row's last 8 columns
+    // instead -- they feed only output rows (columns) that are never stored --
+    // so every other transfer is in range, the per-lane offset is fixed, and
+    // the row offset of the step and instruction is the uniform soffset.
     const int dma_row = 2 * w + (lane >> 5);  // + 2 kWaves j
     const int dma_col = tile_slot_col(dma_row, lane & 31);
     const int dma_voff = dma_row * N * 2 + (kGrouped ? n0 + dma_col : min(n0 + dma_col, N - 8)) * 2;
@@ -596,7 +621,9 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         for (int j = 0; j < kDma; ++j) {
           auto* dst = (__attribute__((address_space(3))) void*)((lds_u8_t*)astage +
                                                                  (w + kWaves * j) * 1024);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, dst, 16, dma_voff,
+          const int voff =
+              kRagged && dma_row >= valid - 2 * kWaves * j ? kOutOfRange : dma_voff;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, dst, 16, voff,
                                                    (row0 + 2 * kWaves * j) * N * 2, 0, 0);
         }
       }
@@ -634,7 +661,9 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         for (int j = 0; j < kDma; ++j) {
           auto* dst = (__attribute__((address_space(3))) void*)((lds_u8_t*)gstage +
                                                                  (w + kWaves * j) * 1024);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(g_rsrc, dst, 16, gdma_voff,
+          const int voff =
+              kRagged && dma_row >= valid - 2 * kWaves * j ? kOutOfRange : gdma_voff;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(g_rsrc, dst, 16, voff,
                                                    (row0 + 2 * kWaves * j) * M * 2, 0, 0);
         }
       }
@@ -768,9 +797,9 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
       float sc_after;
       int valid2;
       const int row2 = step_row0(min(s + 2, nsteps - 1), &sc_after, &valid2);
-      // Grouped mode: a segment's last step may hold fewer than 64 rows; the
-      // MFMAs of a 32-row sub-step past them (all zeros) are skipped.
-      const int vcur = kGrouped ? valid_cur : kBK;
+      // A segment's (ragged example's) last step may hold fewer than 64 rows;
+      // the MFMAs of a 32-row sub-step past them (all zeros) are skipped.
+      const int vcur = kPartial ? valid_cur : kBK;
       auto stage_g = [&](int kk) __attribute__((always_inline)) {
         if constexpr (!kGdma) {
 #pragma unroll
@@ -885,10 +914,11 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
           rescale(m_cur / m);
           m_cur = m;
         }
-        const int rs = ex * T + (t % spe) * kBK;
-        dma_a(lds_a0, rs, kBK);
+        const int r = (t % spe) * kBK;
+        const int rs = ex * T + r, valid = kRagged ? min(kBK, T - r) : kBK;
+        dma_a(lds_a0, rs, valid);
 #pragma unroll
-        for (int j = 0; j < kGC; ++j) load_chunk(rs, kBK, j);
+        for (int j = 0; j < kGC; ++j) load_chunk(rs, valid, j);
         const float p2 = scale_pow2(sc);
 #pragma unroll
         for (int j = 0; j < kGC; ++j) store_chunk(g0, j, p2);
@@ -954,28 +984,16 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
       const float* qr = reinterpret_cast<const float*>(quarter(eq));
       const int mbase = m0 + (eq < 2 ? 0 : 128) + 64 * h + 32 * (eq & 1);
       const int n = n0 + cl;
-      if (!kGrouped && args.splits > 1) {
-        // Split-K: the raw fp32 tile; the reduce kernel finishes it.
-        auto* part = global_ptr<float>(args.partial + (size_t)split * M * N);
-#pragma unroll 4
-        for (int ml = 0; ml < 32; ++ml) {
-          const int m = mbase + ml;
-          if (m < M && n < N)
-            *reinterpret_cast<__attribute__((address_space(1))) f32x2_t*>(part + (size_t)m * N + n) =
-                *reinterpret_cast<const f32x2_t*>(qr + tile_off_epi(ml, cl));
-        }
-      } else {
-          with_epilogue_choices(ep, [&](auto BF, auto NB, auto NZ) __attribute__((always_inline)) {
+      with_epilogue_choices(ep, [&](auto BF, auto NB, auto NZ) __attribute__((always_inline)) {
 #pragma unroll 2
-          for (int ml = 0; ml < 32; ml += 2) {
-            const float2 t0 = *reinterpret_cast<const float2*>(qr + tile_off_epi(ml, cl));
-            const float2 t1 = *reinterpret_cast<const float2*>(qr + tile_off_epi(ml + 1, cl));
-            const float v[2][2] = {{t0.x, t0.y}, {t1.x, t1.y}};
-            emit_quad_t<decltype(BF)::value, decltype(NB)::value, decltype(NZ)::value>(
-                ep, mbase + ml, n, v);
-          }
-        });
-      }
+        for (int ml = 0; ml < 32; ml += 2) {
+          const float2 t0 = *reinterpret_cast<const float2*>(qr + tile_off_epi(ml, cl));
+          const float2 t1 = *reinterpret_cast<const float2*>(qr + tile_off_epi(ml + 1, cl));
+          const float v[2][2] = {{t0.x, t0.y}, {t1.x, t1.y}};
+          emit_quad_t<decltype(BF)::value, decltype(NB)::value, decltype(NZ)::value>(
+              ep, mbase + ml, n, v);
+        }
+      });
       __syncthreads();
     };
     half(std::integral_constant<int, 0>());
@@ -1011,7 +1029,7 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         __syncthreads();
         const int cl = 2 * (tid & 127);
         const int rr = (tid >> 7) * kEpiRows;
-        if (!decltype(Usual)::value && !kGrouped && args.splits > 1) {
+        if (!decltype(Usual)::value && args.partial) {
           // Split-K: the raw fp32 tile; the reduce kernel finishes it.
           auto* part = global_ptr<float>(args.partial + (size_t)split * M * N);
 #pragma unroll 2
@@ -1037,7 +1055,7 @@ __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
         __syncthreads();
       }
     };
-    if ((kGrouped || args.splits == 1) && ep.out_bf16 && !ep.apply_nb && ep.sigma != 0.0f)
+    if (!args.partial && ep.out_bf16 && !ep.apply_nb && ep.sigma != 0.0f)
       epilogue(std::true_type());
     else
       epilogue(std::false_type());
@@ -1067,7 +1085,7 @@ __device__ __forceinline__ bool grouped_scales_fit(const FastArgs& args) {
 // Dense mode: G by DMA.  Grouped mode: one launch in which each workgroup
 // takes the body that matches its problem's scales (both bodies share the
 // LDS arrays).
-template <bool kGrouped, bool kHalfDma = false>
+template <bool kGrouped, bool kHalfDma = false, bool kRagged = false>
 __global__ void __launch_bounds__(kFastWaves * 64, 1) clipped_sum_bf16_kernel(FastArgs args) {
   if constexpr (kGrouped) {
     if (grouped_scales_fit(args))
@@ -1075,7 +1093,7 @@ __global__ void __launch_bounds__(kFastWaves * 64, 1) clipped_sum_bf16_kernel(Fa
     else
       clipped_sum_tile<true, false, kFastWaves>(args);
   } else {
-    clipped_sum_tile<false, true, kFastWaves, kHalfDma>(args);
+    clipped_sum_tile<false, true, kFastWaves, kHalfDma, kRagged>(args);
   }
 }
 
@@ -1095,10 +1113,15 @@ int device_cus() {
 }
 
 // Dense launches of at most one workgroup per compute unit take the
-// half-wave DMA body (see clipped_sum_tile).
+// half-wave DMA body (see clipped_sum_tile); T % 64 != 0 and padded operands
+// take the ragged one.
 template <bool kGrouped>
 void launch_fast(dim3 grid, hipStream_t s, const FastArgs& args) {
-  if (!kGrouped && (int)grid.x <= device_cus())
+  const bool ragged = args.T % kBK != 0 || args.lda != args.ep.N || args.ldg != args.ep.M;
+  if (!kGrouped && ragged)
+    hipLaunchKernelGGL((clipped_sum_bf16_kernel<false, false, true>), grid, dim3(kFastWaves * 64),
+                       0, s, args);
+  else if (!kGrouped && (int)grid.x <= device_cus())
     hipLaunchKernelGGL((clipped_sum_bf16_kernel<false, true>), grid, dim3(kFastWaves * 64), 0, s,
                        args);
   else
@@ -1107,25 +1130,32 @@ void launch_fast(dim3 grid, hipStream_t s, const FastArgs& args) {
 }
 
 // Split-K finish: out = epilogue(sum over splits of partial[split], in
-// order).  One thread per (row pair, column pair); M and N are even.
+// order).  One thread per (row pair, column pair); a split's plane is rows x
+// ld values (rows >= M, ld >= N, both even).
 __global__ void __launch_bounds__(kThreads)
-split_reduce_kernel(const float* __restrict__ partial, int splits, Epilogue ep) {
-  const int half_n = ep.N / 2;
+split_reduce_kernel(const float* __restrict__ partial, int splits, int rows, int ld, Epilogue ep) {
+  const int half_n = (ep.N + 1) / 2;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long long)(ep.M / 2) * half_n) return;
+  if (idx >= (long long)((ep.M + 1) / 2) * half_n) return;
   const int m = 2 * (int)(idx / half_n), n = 2 * (int)(idx % half_n);
-  const size_t plane = (size_t)ep.M * ep.N;
+  const size_t plane = (size_t)rows * ld;
   float v[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
   for (int sp = 0; sp < splits; ++sp) {
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-      const float2 t = *reinterpret_cast<const float2*>(partial + sp * plane +
-                                                        (size_t)(m + r) * ep.N + n);
+      const float2 t =
+          *reinterpret_cast<const float2*>(partial + sp * plane + (size_t)(m + r) * ld + n);
       v[r][0] += t.x;
       v[r][1] += t.y;
     }
   }
-  emit_quad(ep, m, n, v);
+  if (ep.N & 1) {
+    // The rows start at any alignment: value by value.
+    emit_pair(ep, m, n, v[0][0], v[1][0]);
+    emit_pair(ep, m, n + 1, v[0][1], v[1][1]);
+  } else {
+    emit_quad(ep, m, n, v);
+  }
 }
 
 // Split-K factor of a dense fast-path launch: launches of fewer than 192
@@ -1135,7 +1165,7 @@ int fast_splits(int B, int T, int din, int dout) {
   const int ntiles = ceil_div(dout, kBM) * ceil_div(din, kBN);
   if (ntiles >= 192) return 1;
   int splits = 1;
-  const long long steps = (long long)B * (T / kBK);
+  const long long steps = (long long)B * ceil_div(T, kBK);
   while (splits < 8 && ntiles * splits * 2 <= 256 && steps >= 8LL * splits * 2) splits *= 2;
   return splits;
 }
@@ -1504,6 +1534,8 @@ extern "C" int dpc_grouped_clipped_sum(const int64_t* a_ptrs, const int64_t* g_p
     FastArgs args;
     args.A = nullptr;
     args.G = nullptr;
+    args.lda = din;
+    args.ldg = dout;
     args.nprob = 0;
     args.T = 0;
     args.B = 0;
@@ -1530,22 +1562,73 @@ extern "C" int dpc_grouped_clipped_sum(const int64_t* a_ptrs, const int64_t* g_p
 
 namespace {
 // Workspace layout: the bias split partials (kBiasSplits x dout floats), then,
-// 256-byte aligned, the split-K tiles of a dense fast-path launch.
+// each 256-byte aligned, the padded copies of the operands whose width is not
+// a multiple of 8 and the split-K tiles of a dense fast-path launch.
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 size_t bias_ws_bytes(int dout) {
-  return ((size_t)kBiasSplits * (size_t)dout * sizeof(float) + 255) & ~(size_t)255;
+  return align256((size_t)kBiasSplits * (size_t)dout * sizeof(float));
+}
+int padded_width(int d) { return (d + 7) & ~7; }
+// The bf16 MFMA path: any T of at least two tokens (T % 64 != 0: the ragged
+// body; its out-of-range offset must lie past the operands).  One token per
+// example leaves 63 of a step's 64 rows empty: those take the generic kernel,
+// which packs 16 examples into a chunk, and so do the calls of a few chunks
+// where the 512-thread kernel's start and finish (and the padding launches)
+// cost more than the chunks: B, T, din, dout = 4, 2, 64, 64 takes 16.3 us
+// there and 18.4 here, 2, 3, 9, 7 15.8 and 24.4; past the line 8, 20, 63, 65
+// takes 36.2 and 28.4 us, 64, 2, 1024, 1024 75 and 40, 16, 100, 1023, 511 254
+// and 38, 32, 197, 768, 768 368 and 42.
+bool few_chunks(int B, int T, int din, int dout) {
+  const bool aligned = din % 8 == 0 && dout % 8 == 0;
+  if (T % kBK == 0 && aligned) return false;
+  return (long long)B * ceil_div(T, 16) <= (aligned ? 4 : 8) &&
+         (long long)din * dout <= 512 * 512;
 }
 bool fast_shape(int B, int T, int din, int dout, int dtype) {
   const size_t rows = (size_t)B * (size_t)T;
-  const bool small = rows * (size_t)(din > dout ? din : dout) * 2 < ((size_t)1 << 31);
-  return dtype == DPC_BF16 && T % kBK == 0 && din % 8 == 0 && dout % 8 == 0 && B > 0 && small;
+  const size_t limit = T % kBK == 0 ? (size_t)1 << 31 : (size_t)kOutOfRange;
+  return dtype == DPC_BF16 && T > 1 && B > 0 && !few_chunks(B, T, din, dout) &&
+         rows * (size_t)padded_width(din > dout ? din : dout) * 2 < limit;
+}
+// Bytes of the padded operand copies (0 for widths that are multiples of 8).
+size_t pad_bytes(int B, int T, int d) {
+  return d % 8 == 0 ? 0 : align256((size_t)B * (size_t)T * (size_t)padded_width(d) * 2);
+}
+bool split_planes(int splits, int din) { return splits > 1 || din % 2 != 0; }
+size_t split_bytes(int splits, int din, int dout) {
+  if (!split_planes(splits, din)) return 0;
+  return (size_t)splits * (size_t)padded_width(dout) * (size_t)padded_width(din) * sizeof(float);
+}
+
+// dst[row] = src[row] (width elements) followed by zeros up to ld (a multiple
+// of 8); one thread per 16-byte chunk of dst.
+__global__ void __launch_bounds__(kThreads)
+pad_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, long long rows,
+                int width, int ld) {
+  const int chunks = ld / 8;
+  const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= rows * chunks) return;
+  const long long row = i / chunks;
+  const int c0 = (int)(i - row * chunks) * 8;
+  const uint16_t* p = src + row * width + c0;
+  u32x4_t v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t lo = c0 + 2 * k < width ? p[2 * k] : 0;
+    const uint32_t hi = c0 + 2 * k + 1 < width ? p[2 * k + 1] : 0;
+    v[k] = lo | (hi << 16);
+  }
+  *reinterpret_cast<u32x4_t*>(dst + i * 8) = v;
 }
 }  // namespace
 
 extern "C" size_t dpc_clipped_sum_workspace_bytes(int B, int T, int din, int dout, int dtype) {
   if (dout <= 0 || din <= 0 || T <= 0 || B < 0) return 0;
   size_t bytes = bias_ws_bytes(dout);
-  const int splits = fast_shape(B, T, din, dout, dtype) ? fast_splits(B, T, din, dout)
-                                                       : generic_splits(B, T, din, dout);
+  if (fast_shape(B, T, din, dout, dtype))
+    return bytes + pad_bytes(B, T, din) + pad_bytes(B, T, dout) +
+           split_bytes(fast_splits(B, T, din, dout), din, dout);
+  const int splits = generic_splits(B, T, din, dout);
   if (splits > 1) bytes += (size_t)splits * (size_t)dout * (size_t)din * sizeof(float);
   return bytes;
 }
@@ -1585,12 +1668,30 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
   ep.out_bf16 = out_dtype == DPC_BF16;
   ep.out = out;
 
-  // Buffer offsets are 32-bit: each operand must stay below 2 GiB.
-  const bool fast = fast_shape(B, T, din, dout, dtype) && plan != nullptr;
+  // Buffer offsets are 32-bit: each operand must stay below 2 GiB.  Operands
+  // whose rows are not 16-byte aligned are copied into padded rows first; a
+  // caller without the workspace for it gets the generic kernel.
+  const size_t pad_a = pad_bytes(B, T, din), pad_g = pad_bytes(B, T, dout);
+  const size_t pad_at = bias_ws_bytes(dout), split_at = pad_at + pad_a + pad_g;
+  const bool fast =
+      fast_shape(B, T, din, dout, dtype) && plan != nullptr &&
+      (pad_a + pad_g == 0 || (ws && ws_bytes >= split_at + split_bytes(1, din, dout)));
   if (fast) {
+    const long long rows = (long long)B * T;
+    auto padded = [&](const void* x, int d, size_t at) {
+      const int ld = padded_width(d);
+      if (ld == d) return (const uint16_t*)x;
+      uint16_t* dst = (uint16_t*)((uint8_t*)ws + at);
+      const long long chunks = rows * (ld / 8);
+      hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((chunks + kThreads - 1) / kThreads)),
+                         dim3(kThreads), 0, s, (const uint16_t*)x, dst, rows, d, ld);
+      return (const uint16_t*)dst;
+    };
     FastArgs args;
-    args.A = (const uint16_t*)A;
-    args.G = (const uint16_t*)G;
+    args.A = padded(A, din, pad_at);
+    args.G = padded(G, dout, pad_at + pad_a);
+    args.lda = padded_width(din);
+    args.ldg = padded_width(dout);
     args.nprob = 0;
     args.T = T;
     args.B = B;
@@ -1599,17 +1700,18 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
     args.ep = ep;
     // Split-K only with a workspace that holds the slices (else one pass).
     int splits = fast_splits(B, T, din, dout);
-    const size_t need = bias_ws_bytes(dout) + (size_t)splits * dout * (size_t)din * sizeof(float);
-    if (splits > 1 && (!ws || ws_bytes < need)) splits = 1;
+    if (splits > 1 && (!ws || ws_bytes < split_at + split_bytes(splits, din, dout))) splits = 1;
     args.splits = splits;
-    args.partial = splits > 1 ? (float*)((uint8_t*)ws + bias_ws_bytes(dout)) : nullptr;
+    args.partial = split_planes(splits, din) ? (float*)((uint8_t*)ws + split_at) : nullptr;
     const int ntiles = ceil_div(dout, kBM) * ceil_div(din, kBN);
+    DPC_HIP_CHECK(hipGetLastError());
     launch_fast<false>(dim3(ntiles * splits), s, args);
-    if (splits > 1) {
+    if (args.partial) {
       DPC_HIP_CHECK(hipGetLastError());
-      const long long quads = (long long)(dout / 2) * (din / 2);
+      const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
       hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
-                         dim3(kThreads), 0, s, (const float*)args.partial, splits, ep);
+                         dim3(kThreads), 0, s, (const float*)args.partial, splits, args.ldg,
+                         args.lda, ep);
     }
   } else {
     int splits = generic_splits(B, T, din, dout);
@@ -1631,7 +1733,7 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
       DPC_HIP_CHECK(hipGetLastError());
       const long long pairs = (long long)(dout / 2) * (din / 2);
       hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((pairs + kThreads - 1) / kThreads)),
-                         dim3(kThreads), 0, s, (const float*)partial, splits, ep);
+                         dim3(kThreads), 0, s, (const float*)partial, splits, dout, din, ep);
     }
   }
   DPC_HIP_CHECK(hipGetLastError());
@@ -1686,7 +1788,7 @@ extern "C" int dpc_clipped_sum_multi(int n, const void* const* A, const void* co
     if (sigmas[i] != 0.0 && noise_mode == DPC_NOISE_NONE) return DPC_EINVAL;
     if (sigmas[i] != 0.0 && noise_mode == DPC_NOISE_INJECTED && (!noise || !noise[i]))
       return DPC_EINVAL;
-    fast = fast && fast_shape(B, T, din[i], dout[i], dtype);
+    fast = fast && fast_shape(B, T, din[i], dout[i], dtype) && din[i] % 8 == 0 && dout[i] % 8 == 0;
   }
   hipStream_t s = (hipStream_t)stream;
   if (!fast) {
@@ -1705,6 +1807,8 @@ extern "C" int dpc_clipped_sum_multi(int n, const void* const* A, const void* co
     FastArgs args;
     args.A = nullptr;
     args.G = nullptr;
+    args.lda = 0;
+    args.ldg = 0;
     args.T = T;
     args.B = B;
     args.plan = plan;

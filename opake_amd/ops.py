@@ -478,7 +478,7 @@ def clipped_sum_multi(
     bf16 MFMA path the layers' output tiles share launches.  ``noises[i]``:
     layer i's noise (None: none); the specs must share one mode and seed.
     Returns one [dout, din] tensor per layer.  When every layer takes the
-    MFMA path (bf16, T % 64 == 0, widths % 8 == 0, a plan) each result equals
+    MFMA path (bf16, T > 1, widths % 8 == 0, a plan) each result equals
     its own ``clipped_sum`` call without a split-K workspace; otherwise the
     layers run as their own ``clipped_sum`` calls."""
     n = len(A_list)
@@ -503,9 +503,12 @@ def clipped_sum_multi(
     if any(sp.mode != mode or sp.seed != seed or sp.bias_noise is not None for sp in live):
         raise ConfigurationError("the layers' noise specs must share one mode and seed, no bias")
     out_dtype = out_dtype or dtype
-    mfma = plan is not None and B > 0 and dtype == torch.bfloat16 and T % 64 == 0 and all(
+    # The MFMA kernel's 32-bit buffer offsets (with T % 64 != 0 one of them
+    # marks the rows past an example's end).
+    limit = 2 ** 31 if T % 64 == 0 else 0x7FF00000
+    mfma = plan is not None and B > 0 and dtype == torch.bfloat16 and T > 1 and all(
         A.shape[2] % 8 == 0 and G.shape[2] % 8 == 0
-        and B * T * max(A.shape[2], G.shape[2]) * 2 < 2 ** 31 for A, G in zip(A_list, G_list))
+        and B * T * max(A.shape[2], G.shape[2]) * 2 < limit for A, G in zip(A_list, G_list))
     if not mfma:
         return [clipped_sum(A, G, scale, plan=plan, normalize_by=normalize_by, noise=sp,
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]

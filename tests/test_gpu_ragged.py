@@ -1,0 +1,98 @@
+"""The bf16 clipped sum at token counts that no 64-row step divides and at
+widths that are not multiples of 8 (GPU tests, called through the C ABI)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from opake_amd import _native as nat
+from opake_amd import ops
+from opake_amd.clipping import _numerics as num
+from opake_amd.clipping import guard_for_linear
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(B, T, din, dout, seed):
+    g = torch.Generator().manual_seed(seed)
+    A = torch.randn(B, T, din, generator=g).to(torch.bfloat16)
+    G = (torch.randn(B, T, dout, generator=g) * 0.01 *
+         torch.exp(torch.randn(B, 1, 1, generator=g))).to(torch.bfloat16)
+    return A, G
+
+
+def _factors(dev, A, G, C=1.0):
+    sq, err = ops.gram_sqnorms(A, G, return_error=True)
+    guard = guard_for_linear(A.dtype, A.shape[2], G.shape[2], False)
+    return ops.clip_factors(sq, num.conservative_bound(C), [guard], err=err,
+                            count_threshold=num.float32_of(C))
+
+
+def _exact(A, G, scale):
+    return sum(scale[b] * (G[b].double().t() @ A[b].double()) for b in range(A.shape[0]))
+
+
+def _rel(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+# Steps of 1, 2, 33, 63 and 65 rows; one and several tiles; split-K; padded
+# rows of A, of G and of both, odd (value by value) and even output rows.
+@pytest.mark.parametrize("B,T,din,dout", [
+    (3, 2, 16, 8), (1, 33, 8, 264), (2, 63, 64, 72), (5, 65, 264, 256), (24, 97, 256, 520),
+    (3, 64, 15, 24), (4, 100, 257, 1001), (2, 128, 1030, 9), (16, 130, 259, 250), (1, 7, 1, 3)])
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+def test_clipped_sum_ragged(dev, B, T, din, dout, out):
+    """fp32 sums of exact bf16 products: K = B T addends of one rounding each
+    stay within K 2^-24 of the sum of magnitudes, at random signs far below
+    1e-5 of the result; a bf16 output adds 2^-9 per entry."""
+    A, G = _operands(B, T, din, dout, B * 1000 + T + din)
+    A_d, G_d = A.to(dev), G.to(dev)
+    cf = _factors(dev, A_d, G_d)
+    w, _ = ops.clipped_sum(A_d, G_d, cf.scale[0], plan=cf.plan[0], out_dtype=out)
+    want = _exact(A, G, cf.scale[0].cpu().double())
+    assert _rel(w.cpu(), want) < (1e-5 if out == torch.float32 else 2.0**-8)
+
+
+@pytest.mark.parametrize("T,din", [(65, 264), (100, 33)])
+def test_clipped_sum_ragged_skips_a_nonfinite_neighbour(dev, T, din):
+    """The rows past an example's end belong to the next example: NaN there
+    (scale 0) must not reach the sum.  An example of the plan's slow list
+    (a scale below 2^-64) sums as the others do."""
+    A, G = _operands(4, T, din, 136, 5)
+    G[1] = float("nan")
+    A[1] = float("inf")
+    G[2] = (G[2].float() * 1e19).to(torch.bfloat16)
+    A_d, G_d = A.to(dev), G.to(dev)
+    cf = _factors(dev, A_d, G_d)
+    w, _ = ops.clipped_sum(A_d, G_d, cf.scale[0], plan=cf.plan[0], out_dtype=torch.float32)
+    scale = cf.scale[0].cpu().double()
+    assert scale[1] == 0 and 0 < scale[2] < 2.0**-64
+    keep = [0, 2, 3]
+    assert _rel(w.cpu(), _exact(A[keep], G[keep], scale[keep])) < 1e-5
+
+
+@pytest.mark.parametrize("din,dout", [(264, 72), (33, 17)])
+def test_clipped_sum_ragged_noise_matches_add_noise(dev, din, dout):
+    A, G = _operands(3, 70, din, dout, 9)
+    A_d, G_d = A.to(dev), G.to(dev)
+    cf = _factors(dev, A_d, G_d)
+    kw = dict(plan=cf.plan[0], normalize_by=2.0)
+    spec = ops.NoiseSpec(sigma=0.5, mode=nat.NOISE_PHILOX, seed=77, leaf_id=3)
+    plain, _ = ops.clipped_sum(A_d, G_d, cf.scale[0], **kw)
+    noised, _ = ops.clipped_sum(A_d, G_d, cf.scale[0], noise=spec, **kw)
+    assert torch.equal(noised, ops.add_noise(plain, 0.5, seed=77, leaf_id=3))
+
+
+def test_clipped_sum_multi_ragged_matches_single_layers(dev):
+    dims = [(256, 264), (320, 136), (8, 8)]
+    ops_ = [_operands(3, 70, din, dout, 20 + din) for din, dout in dims]
+    As, Gs = [a.to(dev) for a, _ in ops_], [g.to(dev) for _, g in ops_]
+    cf = _factors(dev, As[0], Gs[0])
+    kw = dict(plan=cf.plan[0], out_dtype=torch.float32)
+    got = ops.clipped_sum_multi(As, Gs, cf.scale[0], **kw)
+    for i, w in enumerate(got):
+        assert torch.equal(w, ops.clipped_sum_multi([As[i]], [Gs[i]], cf.scale[0], **kw)[0])
+        want = _exact(*ops_[i], cf.scale[0].cpu().double())
+        assert _rel(w.cpu(), want) < 1e-5
