@@ -30,6 +30,7 @@
 
 #include <algorithm>
 
+#include "bias_cols.h"
 #include "clip_block.h"
 #include "common.h"
 #include "lds_stage.h"
@@ -1826,12 +1827,13 @@ __device__ __forceinline__ double gram_bound_wave(const double* rec, int nt, dou
 
 // Dense finish, one wave per example: sqnorm[b] (+)= the fold of example b's
 // record inner products (+ the bias term), sqerr[b] (+)= its error bound (+
-// the bias term's).  bias (nullable): [B] squared norms then [B] error
-// bounds.
+// the bias term's).  bias (nullable): [B, n_slots] squared norms; their error
+// bound is 2^-21 relative (the fp64 sum of exact squares and the fp32 product
+// scale * column of the clipped sum).
 __global__ void __launch_bounds__(kGramThreads)
 gram_finish_kernel(const double* __restrict__ records, int B, int nt, int nlayers,
-                   int accumulate, const double* __restrict__ bias, double* __restrict__ sqnorm,
-                   double* __restrict__ sqerr) {
+                   int accumulate, const double* __restrict__ bias, int n_slots,
+                   double* __restrict__ sqnorm, double* __restrict__ sqerr) {
   const int b = blockIdx.x * (kGramThreads / 64) + (int)(threadIdx.x >> 6);
   if (b >= B) return;
   const size_t np = (size_t)nt * (nt + 1) / 2;
@@ -1846,13 +1848,15 @@ gram_finish_kernel(const double* __restrict__ records, int B, int nt, int nlayer
     v = first ? s : (L == 0 ? sqnorm[b] : v) + s;
     ev = first ? e : (L == 0 && sqerr ? sqerr[b] : ev) + e;
   }
-  if ((threadIdx.x & 63) != 0) return;
-  if (bias) v = v + bias[b];
-  sqnorm[b] = v;
-  if (sqerr) {
-    if (bias) ev = ev + bias[B + b];
-    sqerr[b] = ev;
+  if (bias) {
+    const int lane = threadIdx.x & 63;
+    const double t = wave_sum_all_f64(lane < n_slots ? bias[(size_t)b * n_slots + lane] : 0.0);
+    v = v + t;
+    ev = ev + t * 0x1.0p-21;
   }
+  if ((threadIdx.x & 63) != 0) return;
+  sqnorm[b] = v;
+  if (sqerr) sqerr[b] = ev;
 }
 
 // Grouped finish, one wave per segment: seg_sq[v] / seg_err[v] (nullable)
@@ -1875,29 +1879,25 @@ segment_finish_kernel(const double* __restrict__ records, const int32_t* __restr
   if (seg_err) seg_err[v] = e;
 }
 
-// ||sum_t G_i[t]||^2 for a bias: one workgroup per example, columns strided
-// over threads, column sums in fp32 (as the reference's per-example bias
-// gradient, and in the order bias_partial_kernel sums them, so the value
-// measured is the value summed), squares summed in fp64.  out[ex] = the
-// squared norm, out[B + ex] = its error bound: the fp64 sum of exact squares
-// and the fp32 product scale * column of the clipped sum, 2^-21 relative.
+// ||sum_t G_i[t]||^2 for a bias: workgroup (slot, ex) takes every n_slots-th
+// block of 128 columns of example ex (column sums in fp32, the values that the
+// clipped sum adds, see bias_cols.h) and writes the fp64 sum of their squares
+// to out[ex * n_slots + slot]; the finish kernel adds the slots.
 template <typename In>
-__global__ void __launch_bounds__(kGramThreads)
-bias_sqnorm_kernel(const In* __restrict__ G, int B, int T, int dout, double* __restrict__ out) {
-  __shared__ double red[kGramThreads / 64];
-  const int ex = blockIdx.x;
+__global__ void __launch_bounds__(kBiasThreads)
+bias_sqnorm_kernel(const In* __restrict__ G, int T, int dout, int n_slots,
+                   double* __restrict__ out) {
+  __shared__ float red[kBiasRedFloats];
+  __shared__ double fold[kBiasThreads / 64];
+  const int slot = blockIdx.x, ex = blockIdx.y;
   const In* g = G + (size_t)ex * T * dout;
   double s = 0.0;
-  for (int m = threadIdx.x; m < dout; m += blockDim.x) {
-    float col = 0.f;
-    for (int t = 0; t < T; ++t) col += load_as_f32(g + (size_t)t * dout + m);
+  for (int c0 = slot * kBiasCols; c0 < dout; c0 += n_slots * kBiasCols) {
+    const float col = bias_column_sum<In>(g, T, dout, c0, red);
     s += (double)col * (double)col;
   }
-  double total = block_sum_f64(s, red);
-  if (threadIdx.x == 0) {
-    out[ex] = total;
-    out[B + ex] = total * 0x1.0p-21;
-  }
+  const double total = block_sum_f64(s, fold);
+  if (threadIdx.x == 0) out[(size_t)ex * n_slots + slot] = total;
 }
 
 // Flat inputs: ||a||^2 ||g||^2 (+ ||g||^2 with a bias), each a fp64 sum of
@@ -1962,13 +1962,20 @@ size_t split_tickets_bytes(int B, int T) {
 }
 }  // namespace
 
-extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
-  if (B <= 0 || T <= 0) return 0;
+// The smallest workspace dpc_gram_sqnorms takes; with the kBiasSlots words per
+// example that dpc_gram_workspace_bytes adds, a bias norm's columns are shared
+// by several workgroups per example (without them by one).
+static size_t gram_min_bytes(int B, int T) {
   size_t n = align256(gram_records_bytes(B, T));
   if (split_shape(T))
     n += split_tickets_bytes(B, T) +
          (size_t)B * split_sets_per_example(ceil_div(T, kGramTile)) * 2 * kSplitSetBytes;
   return n;
+}
+
+extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
+  if (B <= 0 || T <= 0) return 0;
+  return align256(gram_min_bytes(B, T)) + (size_t)B * kBiasSlots * sizeof(double);
 }
 
 extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int dout,
@@ -1979,7 +1986,7 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
   if (!A || !G || !sqnorm || !ws) return DPC_EINVAL;
   if (dtype != DPC_F32 && dtype != DPC_BF16) return DPC_EINVAL;
   if (B > 65535) return DPC_ENOTSUP;
-  if (ws_bytes < dpc_gram_workspace_bytes(B, T)) return DPC_ENOSPC;
+  if (ws_bytes < gram_min_bytes(B, T)) return DPC_ENOSPC;
   hipStream_t s = (hipStream_t)stream;
   double* records = (double*)ws;
   int nt;
@@ -2034,21 +2041,27 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
   }
   DPC_HIP_CHECK(hipGetLastError());
   double* bias = nullptr;
+  int n_slots = 1;
   if (with_bias) {
-    const size_t np = (size_t)nt * (nt + 1) / 2;
-    bias = records + np * (size_t)B * DPC_GRAM_REC_WORDS;
-    if (dtype == DPC_BF16) {
-      hipLaunchKernelGGL(bias_sqnorm_kernel<uint16_t>, dim3(B), dim3(kGramThreads), 0, s,
-                         (const uint16_t*)G, B, T, dout, bias);
+    if (ws_bytes >= dpc_gram_workspace_bytes(B, T)) {
+      n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
+      bias = (double*)((uint8_t*)ws + align256(gram_min_bytes(B, T)));
     } else {
-      hipLaunchKernelGGL(bias_sqnorm_kernel<float>, dim3(B), dim3(kGramThreads), 0, s,
-                         (const float*)G, B, T, dout, bias);
+      bias = records + (size_t)nt * (nt + 1) / 2 * (size_t)B * DPC_GRAM_REC_WORDS;
+    }
+    const dim3 grid(n_slots, B);
+    if (dtype == DPC_BF16) {
+      hipLaunchKernelGGL(bias_sqnorm_kernel<uint16_t>, grid, dim3(kBiasThreads), 0, s,
+                         (const uint16_t*)G, T, dout, n_slots, bias);
+    } else {
+      hipLaunchKernelGGL(bias_sqnorm_kernel<float>, grid, dim3(kBiasThreads), 0, s,
+                         (const float*)G, T, dout, n_slots, bias);
     }
     DPC_HIP_CHECK(hipGetLastError());
   }
   hipLaunchKernelGGL(gram_finish_kernel, dim3(ceil_div(B, kGramThreads / 64)), dim3(kGramThreads), 0,
-                     s, (const double*)records, B, nt, 1, accumulate, (const double*)bias, sqnorm,
-                     sqerr);
+                     s, (const double*)records, B, nt, 1, accumulate, (const double*)bias, n_slots,
+                     sqnorm, sqerr);
   DPC_HIP_CHECK(hipGetLastError());
   return DPC_OK;
 }
@@ -2231,7 +2244,7 @@ extern "C" int dpc_gram_sqnorms_noalloc(const void* A, const void* G, int B, int
                                         double* sqnorm, double* sqerr, void* stream) {
   if (B < 0 || T <= 0 || din <= 0 || dout <= 0) return DPC_EINVAL;
   if (B == 0) return DPC_OK;
-  const size_t need = dpc_gram_workspace_bytes(B, T);
+  const size_t need = gram_min_bytes(B, T);
   if (need > (size_t)DPC_NOALLOC_SCRATCH_BYTES) return DPC_ENOSPC;
   void* ws = scratch_on_current_device();
   if (!ws) return DPC_EHIP;
@@ -2264,7 +2277,7 @@ size_t split_multi_bytes(int n, int B, int T) {
 extern "C" size_t dpc_gram_sqnorms_multi_workspace_bytes(int n, const int* din, const int* dout,
                                                         int B, int T, int dtype) {
   if (n <= 0 || B <= 0 || T <= 0 || !din || !dout) return 0;
-  const size_t one = dpc_gram_workspace_bytes(B, T);
+  const size_t one = gram_min_bytes(B, T);
   if (!split_multi_shape(n, din, dout, B, T, dtype)) return one;
   const size_t multi = split_multi_bytes(n, B, T);
   return multi > one ? multi : one;
@@ -2329,7 +2342,7 @@ extern "C" int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* c
                      nsets, nblocks, records, tickets, xbuf, SplitTail{});
   DPC_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(gram_finish_kernel, dim3(ceil_div(B, kGramThreads / 64)), dim3(kGramThreads), 0,
-                     s, (const double*)records, B, nt, n, accumulate, (const double*)nullptr,
+                     s, (const double*)records, B, nt, n, accumulate, (const double*)nullptr, 0,
                      sqnorm, sqerr);
   DPC_HIP_CHECK(hipGetLastError());
   return DPC_OK;
@@ -2372,7 +2385,7 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   if (!A || !G || !sqnorm || !ws) return DPC_EINVAL;
   if (dtype != DPC_F32 && dtype != DPC_BF16) return DPC_EINVAL;
   if (B > 65535) return DPC_ENOTSUP;
-  if (ws_bytes < dpc_gram_clip_workspace_bytes(B, T)) return DPC_ENOSPC;
+  if (ws_bytes < gram_min_bytes(B, T)) return DPC_ENOSPC;
   ClipJob job;
   int r = clip_job_from_args(C, kind, gamma, guard_rel, guard_abs, guard_mult, n_guards,
                              count_threshold, scale, scale64, norms_out, nclipped, plan, nonfinite,

@@ -96,3 +96,41 @@ def test_clipped_sum_multi_ragged_matches_single_layers(dev):
         assert torch.equal(w, ops.clipped_sum_multi([As[i]], [Gs[i]], cf.scale[0], **kw)[0])
         want = _exact(*ops_[i], cf.scale[0].cpu().double())
         assert _rel(w.cpu(), want) < 1e-5
+
+
+# Row groups of the bias column sums: fewer rows than groups, one more than a
+# full turn of them, the unrolled part and its remainder; 16-byte rows and
+# rows of any alignment; one and several column blocks and slots, and a
+# workspace without the slots.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,dout", [(3, 2, 8), (2, 7, 136), (2, 9, 1001), (40, 33, 264),
+                                      (2, 129, 130), (1, 300, 4104)])
+def test_bias_norm_and_sum(dev, dtype, B, T, dout):
+    g = torch.Generator().manual_seed(B + T + dout)
+    A = torch.randn(B, T, 16, generator=g).to(dtype)
+    G = (torch.randn(B, T, dout, generator=g) * 0.01 + 0.002).to(dtype)
+    cols = G.double().sum(dim=1)
+    exact_w = torch.stack([(G[b].double().t() @ A[b].double()).square().sum() for b in range(B)])
+    A_d, G_d = A.to(dev), G.to(dev)
+    sq, err = ops.gram_sqnorms(A_d, G_d, with_bias=True, return_error=True)
+    w_sq, w_err = ops.gram_sqnorms(A_d, G_d, return_error=True)
+    want = exact_w + cols.square().sum(dim=1)
+    # fp32 column sums of T addends: T 2^-24 of the magnitudes, twice in a
+    # square; the weight part is the bias-free call's own.
+    tol = 4 * T * 2.0**-24 * G.double().abs().sum(dim=1).square().sum(dim=1)
+    bias_sq = (sq - w_sq).cpu()
+    assert ((bias_sq - cols.square().sum(dim=1)).abs() <= tol + 1e-9 * want).all()
+    assert (err >= w_err).all()
+    small = nat.load().dpc_gram_workspace_bytes(B, T) - 32 * 8 * B
+    ws = torch.empty(small, dtype=torch.uint8, device=dev)
+    sq1 = torch.empty(B, dtype=torch.float64, device=dev)
+    nat.call("dpc_gram_sqnorms", nat.ptr(A_d), nat.ptr(G_d), B, T, 16, dout,
+             nat.dtype_code(dtype), 1, 0, nat.ptr(sq1), None, nat.ptr(ws), small,
+             nat.stream_handle(dev))
+    torch.testing.assert_close(sq1, sq, rtol=1e-12, atol=0)
+    scale = torch.rand(B, generator=g).to(dev)
+    scale[0] = 0.0 if B > 1 else 0.5
+    _, b = ops.clipped_sum(A_d, G_d, scale, with_bias=True, out_dtype=torch.float32)
+    want_b = scale.cpu().double() @ cols
+    bound = (T + B) * 2.0**-23 * (scale.cpu().double() @ G.double().abs().sum(dim=1))
+    assert ((b.cpu().double() - want_b).abs() <= bound).all()
