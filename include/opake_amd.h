@@ -115,7 +115,7 @@ int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* const* G, co
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): the
  * workspace is a static device array of DPC_NOALLOC_SCRATCH_BYTES per device,
  * held until the process ends.  Calls needing more
- * (dpc_gram_workspace_bytes(B, T) > DPC_NOALLOC_SCRATCH_BYTES) return
+ * (tile records and exchange past DPC_NOALLOC_SCRATCH_BYTES) return
  * DPC_ENOSPC.  Every call on a device shares that device's array, so calls
  * that overlap on one device (other streams, other threads) race. */
 #define DPC_NOALLOC_SCRATCH_BYTES (48u << 20)

@@ -27,6 +27,7 @@
 // tile pair on 4 waves.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include <algorithm>
 
@@ -1735,26 +1736,195 @@ __device__ __forceinline__ void generic_tile_stats(const double pa[4][4], const 
                        0.0, st);
 }
 
+// Dense fp64 Gram path (fp32 operands, and bf16 shapes off the bf16 MFMA
+// path): products of fp32 values are exact in fp64, and the 16x16x4 fp64 MFMA
+// sums them, so the error model is that of a fp64 chain.
+//
+// A workgroup computes one pair (p, q) of 32-row tiles of both Gram matrices:
+// waves 0, 1 the tile of A A^T, waves 2, 3 that of G G^T, as 2 x 2 blocks of
+// 16 x 16 (three on a diagonal pair), each wave over every other 32-deep chunk
+// of the depth.  A wave reads its fragments straight from memory, two chunks
+// ahead of the MFMAs: 32 MFMAs of 64 cycles need 8 KiB (fp32), and the
+// pair's waves and the workgroups of one example on an XCD find most of it in
+// their caches.  So the loop has no LDS round trip and no barrier: staged
+// through LDS with one barrier per chunk, [16, 256, 1024 x 1024] took 80 to 87
+// us against 61 here (375 in 4 x 4 FMA blocks; 28 at the matrix rate, of which
+// the uneven 2.25 tile pairs per CU cost a third), [16, 1024, 512 x 512] 370
+// (226; the loop's conversions and loads keep the MFMAs at 63% of their rate).
+// Lane l holds k = 8 (l / 16) .. + 7 of row l % 16 in two 16-byte loads (bf16:
+// one; at any element alignment, which global loads take: element by element
+// rows of odd width took twice as long), so a row's part of a chunk is one
+// 128-byte (64-byte) segment; the
+// order of k is permuted alike on both sides.  A last chunk that is not full is
+// read element by element, so no load reaches past a row's end.
+//
+// With `subs` = 2 (a workspace that holds only the records of 64-row tiles)
+// the pair's 32-row sub-pairs run one after the other.
+constexpr int kF64Threads = 256;
+constexpr int kF64Rows = 32;   // rows of a tile
+constexpr int kF64Depth = 32;  // depth of a chunk
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+// 16 bytes at any element boundary (global loads take every alignment).
+typedef u32x4_t u32x4_align2_t __attribute__((aligned(2)));
+typedef u32x4_t u32x4_align4_t __attribute__((aligned(4)));
+
+// One wave's 2 x 2 blocks (kDiag: without the lower left one) over the chunks
+// c0, c0 + 2, ... of the rows p0 .. + 31 and q0 .. + 31 of X [T, d].
+template <typename In, bool kDiag>
+__device__ __forceinline__ void gram_f64_blocks(const In* X, int T, int d, int p0, int q0, int c0,
+                                                f64x4_t (&acc)[2][2]) {
+  constexpr int kFrags = kDiag ? 2 : 4;              // p's two, then q's
+  constexpr int kWords = 8 * (int)sizeof(In) / 4;    // a lane's 8 values
+  using Chunk = std::conditional_t<sizeof(In) == 2, u32x4_align2_t, u32x4_align4_t>;
+  const int lane = threadIdx.x & 63, kl = 8 * (lane >> 4);
+  const int n = ceil_div(d, kF64Depth);
+  const bool full_rows = q0 + kF64Rows <= T && p0 + kF64Rows <= T;
+  // Rows past T read row 0; their words are zeroed before the product.
+  const In* ptr[kFrags];
+  bool ok[kFrags];
+#pragma unroll
+  for (int f = 0; f < kFrags; ++f) {
+    const int row = (f < 2 ? p0 : q0) + 16 * (f & 1) + (lane & 15);
+    ok[f] = row < T;
+    ptr[f] = X + (ok[f] ? (size_t)row * d : 0) + kl;
+  }
+  typedef uint32_t Raw[kFrags][kWords];
+  Raw raw0, raw1;
+  auto load = [&](int c, Raw& raw) __attribute__((always_inline)) {
+    const int k = c * kF64Depth;
+    if (k + kF64Depth <= d) {
+#pragma unroll
+      for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+        for (int h = 0; h < kWords / 4; ++h) {
+          const u32x4_t x = *global_ptr<const Chunk>(ptr[f] + k + 4 * h);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) raw[f][4 * h + i] = x[i];
+        }
+    } else {
+#pragma unroll
+      for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+        for (int i = 0; i < kWords; ++i) {
+          constexpr int kPer = 8 / kWords;  // values per word
+          uint32_t word = 0u;
+#pragma unroll
+          for (int j = 0; j < kPer; ++j) {
+            const int e = k + kPer * i + j;
+            if (kl + e < d) {
+              if constexpr (sizeof(In) == 2)
+                word |= (uint32_t)global_ptr<const uint16_t>(ptr[f])[e] << (16 * j);
+              else
+                word = global_ptr<const uint32_t>(ptr[f])[e];
+            }
+          }
+          raw[f][i] = word;
+        }
+    }
+  };
+  auto sum = [&](Raw& raw) __attribute__((always_inline)) {
+    if (!full_rows) {
+#pragma unroll
+      for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+        for (int i = 0; i < kWords; ++i) raw[f][i] = ok[f] ? raw[f][i] : 0u;
+    }
+    auto value = [&](int f, int i) __attribute__((always_inline)) {
+      if constexpr (kWords == 8) {
+        return (double)__builtin_bit_cast(float, raw[f][i]);
+      } else {
+        const uint32_t w = raw[f][i >> 1];
+        return (double)__builtin_bit_cast(float, i & 1 ? w & 0xffff0000u : w << 16);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      double v[kFrags];
+#pragma unroll
+      for (int f = 0; f < kFrags; ++f) v[f] = value(f, i);
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          if (!kDiag || s >= r)
+            acc[r][s] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[r], v[kDiag ? s : 2 + s], acc[r][s],
+                                                             0, 0, 0);
+    }
+  };
+  if (c0 < n) load(c0, raw0);
+  for (int c = c0; c < n; c += 4) {
+    if (c + 2 < n) load(c + 2, raw1);
+    sum(raw0);
+    if (c + 2 >= n) break;
+    if (c + 4 < n) load(c + 4, raw0);
+    sum(raw1);
+  }
+}
+
 template <typename In>
-__global__ void __launch_bounds__(kGramThreads)
-gram_generic_kernel(const In* __restrict__ A, const In* __restrict__ G, int T, int din, int dout,
-                    int npairs, double* __restrict__ records) {
-  __shared__ float sp[kGenK][kGenTile + 1];
-  __shared__ float sq[kGenK][kGenTile + 1];
-  __shared__ double red[kRecStat * (kGramThreads / 64)];
-  const int pair = blockIdx.x, ex = blockIdx.y;
-  int p, q;
-  pair_from_index(pair, &p, &q);
-  double pa[4][4], pg[4][4];
-  gram_tile_generic<In>(A + (size_t)ex * T * din, T, din, p, q, sp, sq, pa);
-  gram_tile_generic<In>(G + (size_t)ex * T * dout, T, dout, p, q, sp, sq, pg);
+__global__ void __launch_bounds__(kF64Threads, 2)
+gram_f64_kernel(const In* __restrict__ A, const In* __restrict__ G, int T, int din, int dout,
+                int npairs, int nblocks, int subs, double* __restrict__ records) {
+  __shared__ double xch[2 * 16 * 64];  // a wave's blocks per operand
+  __shared__ double red[kRecStat * (kF64Threads / 64)];
+  const int l = xcd_logical_block(gridDim.x, nblocks);
+  if (l < 0) return;  // padding workgroup: exits before any barrier
+  const int ex = l / npairs, pair = l - ex * npairs;
+  int P, Q;
+  pair_from_index(pair, &P, &Q);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int op = w >> 1, half = w & 1;
+  const int d = op ? dout : din;
+  const In* X = op ? G + (size_t)ex * T * dout : A + (size_t)ex * T * din;
+  // Chain lengths as in the grouped generic kernel (zero padding adds no error).
   const double gA = dpc_chain_gamma((double)ceil_div(din, kGenK) * kGenK, DPC_GRAM_U_FP64);
   const double gQ = dpc_chain_gamma((double)ceil_div(dout, kGenK) * kGenK, DPC_GRAM_U_FP64);
   double st[kRecStat] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  generic_tile_stats(pa, pg, p == q, gA, gQ, st);
-  if (p != q) st[0] *= 2.0;
-  write_gram_record(st, red, records + ((size_t)ex * npairs + pair) * DPC_GRAM_REC_WORDS, gA, gQ,
-                    T);
+  for (int sub = 0; sub < subs * subs; ++sub) {
+    const int p = subs * P + sub / subs, q = subs * Q + sub % subs;
+    const bool diag = p == q;
+    if (p > q || q * kF64Rows >= T) continue;  // a mirrored sub-pair, or no rows
+    f64x4_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+    if (diag)
+      gram_f64_blocks<In, true>(X, T, d, p * kF64Rows, q * kF64Rows, half, acc);
+    else
+      gram_f64_blocks<In, false>(X, T, d, p * kF64Rows, q * kF64Rows, half, acc);
+    // The second wave's blocks, then the G operand's sum, through LDS.
+    double* mine = xch + op * 16 * 64 + lane;
+    __syncthreads();  // the previous sub-pair's exchange is read
+    if (half == 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[64 * i] = acc[i >> 3][(i >> 2) & 1][i & 3];
+    }
+    __syncthreads();
+    if (half == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] += mine[64 * i];
+      if (op == 1) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mine[64 * i] = acc[i >> 3][(i >> 2) & 1][i & 3];
+      }
+    }
+    __syncthreads();
+    if (w == 0) {
+      // fp64 16x16 block: entry r of lane l is row 4 r + l / 16, column l % 16.
+      const double* other = xch + 16 * 64 + lane;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int br = i >> 3, bc = (i >> 2) & 1;
+        if (diag && br > bc) continue;  // mirrors block (0, 1)
+        const int row = 16 * br + 4 * (i & 3) + (lane >> 4), col = 16 * bc + (lane & 15);
+        const double a = acc[br][bc][i & 3], g = other[64 * i];
+        gram_entry_stats(a, g, diag && row == col, gA, 0.0, gQ, 0.0, 0.0, st);
+        if ((diag && br != bc) || (P == Q && !diag))
+          gram_entry_stats(a, g, false, gA, 0.0, gQ, 0.0, 0.0, st);  // its mirror entry
+      }
+    }
+  }
+  if (P != Q) st[0] *= 2.0;
+  write_gram_record(st, red, records + (size_t)l * DPC_GRAM_REC_WORDS, gA, gQ, T);
 }
 
 // Grouped generic path: one 128-row tile pair (P, Q) as its four 64-row
@@ -1962,9 +2132,11 @@ size_t split_tickets_bytes(int B, int T) {
 }
 }  // namespace
 
-// The smallest workspace dpc_gram_sqnorms takes; with the kBiasSlots words per
-// example that dpc_gram_workspace_bytes adds, a bias norm's columns are shared
-// by several workgroups per example (without them by one).
+// The smallest workspace dpc_gram_sqnorms takes.  What dpc_gram_workspace_bytes
+// adds: the records of 32-row tiles of the fp64 path (in place of the 64-row
+// ones; without the room that path keeps 64-row tiles), and kBiasSlots words
+// per example (a bias norm's columns shared by several workgroups per
+// example, without them by one).
 static size_t gram_min_bytes(int B, int T) {
   size_t n = align256(gram_records_bytes(B, T));
   if (split_shape(T))
@@ -1972,10 +2144,16 @@ static size_t gram_min_bytes(int B, int T) {
          (size_t)B * split_sets_per_example(ceil_div(T, kGramTile)) * 2 * kSplitSetBytes;
   return n;
 }
+static size_t gram_bias_slots_offset(int B, int T) {
+  size_t n = gram_min_bytes(B, T);
+  const size_t nt = ceil_div(T, kF64Rows);
+  const size_t fine = nt * (nt + 1) / 2 * B * DPC_GRAM_REC_WORDS * sizeof(double);
+  return align256(n > fine ? n : fine);
+}
 
 extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
   if (B <= 0 || T <= 0) return 0;
-  return align256(gram_min_bytes(B, T)) + (size_t)B * kBiasSlots * sizeof(double);
+  return gram_bias_slots_offset(B, T) + (size_t)B * kBiasSlots * sizeof(double);
 }
 
 extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int dout,
@@ -1988,6 +2166,7 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
   if (B > 65535) return DPC_ENOTSUP;
   if (ws_bytes < gram_min_bytes(B, T)) return DPC_ENOSPC;
   hipStream_t s = (hipStream_t)stream;
+  const bool full_ws = ws_bytes >= dpc_gram_workspace_bytes(B, T);
   double* records = (double*)ws;
   int nt;
   // Buffer offsets are 32-bit: one example's rows (plus a tile of padding)
@@ -2028,24 +2207,25 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
     hipLaunchKernelGGL(gram_mfma_bf16_kernel, dim3(padded), dim3(512), 0, s, (const uint16_t*)A,
                        (const uint16_t*)G, T, din, dout, npairs, items, nblocks, records);
   } else {
-    nt = ceil_div(T, kGenTile);
-    const int npairs = nt * (nt + 1) / 2;
+    const int subs = full_ws ? 1 : kGenTile / kF64Rows;
+    nt = ceil_div(T, kF64Rows * subs);
+    const int npairs = nt * (nt + 1) / 2, nblocks = npairs * B;
+    const dim3 grid(ceil_div(nblocks, kXcds) * kXcds), block(kF64Threads);
     if (dtype == DPC_BF16) {
-      hipLaunchKernelGGL(gram_generic_kernel<uint16_t>, dim3(npairs, B), dim3(kGramThreads), 0,
-                         s, (const uint16_t*)A, (const uint16_t*)G, T, din, dout, npairs,
-                         records);
+      hipLaunchKernelGGL(gram_f64_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)A,
+                         (const uint16_t*)G, T, din, dout, npairs, nblocks, subs, records);
     } else {
-      hipLaunchKernelGGL(gram_generic_kernel<float>, dim3(npairs, B), dim3(kGramThreads), 0, s,
-                         (const float*)A, (const float*)G, T, din, dout, npairs, records);
+      hipLaunchKernelGGL(gram_f64_kernel<float>, grid, block, 0, s, (const float*)A,
+                         (const float*)G, T, din, dout, npairs, nblocks, subs, records);
     }
   }
   DPC_HIP_CHECK(hipGetLastError());
   double* bias = nullptr;
   int n_slots = 1;
   if (with_bias) {
-    if (ws_bytes >= dpc_gram_workspace_bytes(B, T)) {
+    if (full_ws) {
       n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
-      bias = (double*)((uint8_t*)ws + align256(gram_min_bytes(B, T)));
+      bias = (double*)((uint8_t*)ws + gram_bias_slots_offset(B, T));
     } else {
       bias = records + (size_t)nt * (nt + 1) / 2 * (size_t)B * DPC_GRAM_REC_WORDS;
     }

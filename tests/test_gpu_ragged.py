@@ -121,16 +121,51 @@ def test_bias_norm_and_sum(dev, dtype, B, T, dout):
     bias_sq = (sq - w_sq).cpu()
     assert ((bias_sq - cols.square().sum(dim=1)).abs() <= tol + 1e-9 * want).all()
     assert (err >= w_err).all()
-    small = nat.load().dpc_gram_workspace_bytes(B, T) - 32 * 8 * B
-    ws = torch.empty(small, dtype=torch.uint8, device=dev)
-    sq1 = torch.empty(B, dtype=torch.float64, device=dev)
-    nat.call("dpc_gram_sqnorms", nat.ptr(A_d), nat.ptr(G_d), B, T, 16, dout,
-             nat.dtype_code(dtype), 1, 0, nat.ptr(sq1), None, nat.ptr(ws), small,
-             nat.stream_handle(dev))
-    torch.testing.assert_close(sq1, sq, rtol=1e-12, atol=0)
+    if (-(-T // 128)) % 2:
+        # The smallest workspace: the records of the 64-row tile pairs and two words
+        # per example (the workspace query adds finer tiles and shared columns).
+        pairs = (-(-T // 64)) * (-(-T // 64) + 1) // 2
+        small = -(-(pairs * 12 + 2) * B * 8 // 256) * 256
+        ws = torch.empty(small, dtype=torch.uint8, device=dev)
+        sq1 = torch.empty(B, dtype=torch.float64, device=dev)
+        nat.call("dpc_gram_sqnorms", nat.ptr(A_d), nat.ptr(G_d), B, T, 16, dout,
+                 nat.dtype_code(dtype), 1, 0, nat.ptr(sq1), None, nat.ptr(ws), small,
+                 nat.stream_handle(dev))
+        torch.testing.assert_close(sq1, sq, rtol=1e-12, atol=0)
     scale = torch.rand(B, generator=g).to(dev)
     scale[0] = 0.0 if B > 1 else 0.5
     _, b = ops.clipped_sum(A_d, G_d, scale, with_bias=True, out_dtype=torch.float32)
     want_b = scale.cpu().double() @ cols
     bound = (T + B) * 2.0**-23 * (scale.cpu().double() @ G.double().abs().sum(dim=1))
     assert ((b.cpu().double() - want_b).abs() <= bound).all()
+
+
+# The fp64 Gram path: 32-row tiles (few items) and 64-row ones (1024 items and
+# more), one, two and several tiles with ragged last ones, depths around the
+# 32-deep chunks, rows that 16-byte loads do not take, din != dout both ways.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,din,dout", [
+    (2, 2, 4, 8), (3, 31, 33, 9), (2, 32, 32, 31), (4, 65, 100, 36), (1, 130, 7, 260),
+    (2, 257, 64, 65), (1024, 40, 12, 20), (110, 200, 33, 68)])
+def test_gram_f64(dev, dtype, B, T, din, dout):
+    """Exact products in fp64: the error is within the kernel's own bound, and
+    far below what fp32 sums would leave (2^-24)."""
+    g = torch.Generator().manual_seed(B + T + din)
+    A = torch.randn(B, T, din, generator=g).to(dtype).to(dev)
+    G = torch.randn(B, T, dout, generator=g).to(dtype).to(dev)
+    if dtype == torch.bfloat16 and din % 8 == 0 and dout % 8 == 0:
+        pytest.skip("takes the bf16 MFMA kernels")
+    sq, err = ops.gram_sqnorms(A, G, return_error=True)
+    grads = torch.stack([G[b].double().t() @ A[b].double() for b in range(B)])
+    want = grads.square().sum(dim=(1, 2))
+    # The reference's own fp64 sums: T products per entry, at most 2^-53 each.
+    own = (T + 8) * 2.0**-52 * (G.double().abs().transpose(1, 2).contiguous()
+                                @ A.double().abs().contiguous()).square().sum(dim=(1, 2))
+    assert ((sq - want).abs() <= err + own).all()
+    assert ((sq - want).abs() <= 1e-11 * want).all()
+    # The bound's own size: by Cauchy-Schwarz over its tiles it is at most
+    # (gamma_A + gamma_G + (T^2 + 256) 2^-52) sum |a|^2 sum |g|^2, with gamma of
+    # a chain of d products padded to 16.
+    gammas = sum(1.125 * (-(-d // 16) * 16) * 2.0**-52 for d in (din, dout))
+    rows = A.double().square().sum(dim=(1, 2)) * G.double().square().sum(dim=(1, 2))
+    assert (err <= 1.001 * (gammas + (T * T + 256) * 2.0**-52) * rows).all()
