@@ -268,8 +268,8 @@ __device__ __forceinline__ u32x4_t scale_chunk(u32x4_t x, float s) {
 
 // Linear workgroup id -> (tile_m, tile_n) in GROUP_M order, so a group of
 // tile rows shares the activation tiles.
+template <int kGroupM = 4>
 __device__ __forceinline__ void tile_coords(int lin, int tiles_m, int tiles_n, int* tm, int* tn) {
-  constexpr int kGroupM = 4;
   const int per_group = kGroupM * tiles_n;
   const int group = lin / per_group;
   const int first_m = group * kGroupM;
@@ -1173,7 +1173,8 @@ int fast_splits(int B, int T, int din, int dout) {
 
 #undef DPC_WAIT_VMCNT
 
-// Generic path: any T, float32 or bf16 operands; 64 x 64 tiles with a 4 x 4
+// Generic path (calls without the workspace of the paths above and below, bf16
+// with one token or a few chunks): any T, float32 or bf16 operands; 64 x 64 tiles with a 4 x 4
 // FMA block per thread.  K is walked in chunks of at most 16 rows that never
 // straddle two examples: G is staged multiplied by the power of two of its
 // example's scale (exact) and the accumulators carry the mantissa (they hold
@@ -1319,6 +1320,258 @@ int generic_splits(int B, int T, int din, int dout) {
   long long splits = (512 + tiles - 1) / tiles;
   splits = splits < K / 64 ? splits : K / 64;
   return (int)(splits < 1 ? 1 : (splits > 32 ? 32 : splits));
+}
+
+// fp32 path: 64 x 64 output tiles on the 16x16x4 fp32 MFMA.  A wave sums the
+// whole tile over a slice of the K = B T rows, straight from memory: lane l
+// loads 16 bytes of row k0 + l / 16 of each operand, columns 4 (l % 16) .. + 3
+// (256-byte row segments), which are its entries of four fragments -- block i
+// of an operand holds the columns 4 j + i -- so two loads feed 16 MFMAs of 32
+// cycles, with no LDS and no barrier in the loop; 16 rows are in flight while
+// 16 are summed.  The four waves of a workgroup take consecutive slices and add
+// their tiles through LDS in order; `splits` workgroups per tile take
+// consecutive parts of K and write raw tiles, which split_reduce_kernel adds in
+// order and finishes.  Rows of any width are read (16-byte loads at 4-byte
+// alignment).
+//
+// The scale is applied as in the generic kernel: G times the power of two of
+// its example's scale (exact), the mantissa on the accumulators; with one
+// token per example (kFlat) row k times its own scale.
+//
+// The kernel is bound by the fp32 matrix rate (64 FLOP per cycle and SIMD) and,
+// for small outputs, by how K divides: [16, 256, 1024 x 1024] takes 92 us (55 at
+// that rate) against 488 in the 4 x 4 FMA blocks of the generic kernel, [4,
+// 1024, 2048 x 2048] 325 (222), [256, 1, 784 x 512] 11 against 18.8.  A branch
+// per load for the edge tiles cost 10 to 40%: the waits at its joins serialise
+// the loads, so edge tiles have a body of their own.
+constexpr int kF32Tile = 64;
+constexpr int kF32Rows = 16;  // rows of a chunk
+typedef f32x4_t f32x4_align4_t __attribute__((aligned(4)));
+
+struct F32Chunk {
+  f32x4_t g[4], a[4];  // rows 4 q + l / 16
+  float s[4];          // kFlat: those rows' scales
+};
+
+struct F32Args {
+  const float* A;      // [B * T, N]
+  const float* G;      // [B * T, M]
+  const float* scale;  // [B]
+  int B, T, M, N;
+  int splits;
+  long long per;  // rows of a wave's slice
+  int plane_rows, plane_ld;
+  float* partial;  // [splits][plane_rows][plane_ld]
+};
+
+// kEdge: a tile that the matrix does not fill.  Its 16-byte loads start at the
+// row's last 4 columns at most, and the values move to their places before the
+// product (the columns past the matrix, never stored, hold whatever comes).
+template <bool kFlat, bool kEdge>
+__device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0, int n0, int split,
+                                                     float* tile) {
+  const int M = args.M, N = args.N, T = args.T;
+  const float* scale = args.scale;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kq = lane >> 4, cl = 4 * (lane & 15);
+  const long long K = (long long)args.B * T;
+  const long long kb = min(K, (4LL * split + w) * args.per), ke = min(K, kb + args.per);
+  const int cg = kEdge ? min(m0 + cl, M - 4) : m0 + cl, ca = kEdge ? min(n0 + cl, N - 4) : n0 + cl;
+
+  // Rows k0 + 4 q + l / 16 of a chunk of `rows` rows; past them its first row.
+  auto load = [&](long long k0, int rows, F32Chunk& x) __attribute__((always_inline)) {
+    const float* gb = args.G + k0 * M;
+    const float* ab = args.A + k0 * N;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = 4 * q + kq;
+      const uint32_t rr = r < rows ? r : 0;
+      x.g[q] = *global_ptr<const f32x4_align4_t>(gb + (rr * (uint32_t)M + (uint32_t)cg));
+      x.a[q] = *global_ptr<const f32x4_align4_t>(ab + (rr * (uint32_t)N + (uint32_t)ca));
+      if (kFlat) x.s[q] = scale[k0 + rr];
+    }
+  };
+  auto place = [&](f32x4_t& v, int shift) __attribute__((always_inline)) {
+    if constexpr (kEdge) {
+      const f32x4_t x = v;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        float y = x[i];
+#pragma unroll
+        for (int sh = 1; i + sh < 4; ++sh) y = shift == sh ? x[i + sh] : y;
+        v[i] = y;
+      }
+    }
+  };
+
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto sum_rows = [&](int rows, float p2, F32Chunk& x, auto Full) __attribute__((always_inline)) {
+    constexpr bool kFull = decltype(Full)::value;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (!kFull && 4 * q >= rows) break;
+      f32x4_t g = x.g[q], a = x.a[q];
+      const float sc = kFlat ? x.s[q] : p2;
+      place(g, m0 + cl - cg);
+      place(a, n0 + cl - ca);
+      if (kFlat || !kFull) {
+        // Rows past the chunk, and examples with scale 0, add nothing (their
+        // values may be non-finite).
+        const bool on = (kFull || 4 * q + kq < rows) && (!kFlat || sc > 0.0f);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          g[i] = on ? g[i] : 0.0f;
+          a[i] = on ? a[i] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) g[i] *= sc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(g[i], a[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  auto sum = [&](int rows, float p2, F32Chunk& x) __attribute__((always_inline)) {
+    if (rows == kF32Rows)
+      sum_rows(rows, p2, x, std::true_type());
+    else
+      sum_rows(rows, p2, x, std::false_type());
+  };
+
+  // Chunks of at most 16 rows inside one example (kFlat: of 16 examples) of
+  // [kb, ke), without examples of scale 0.
+  long long next = kb;
+  int ex = kFlat ? 0 : (int)(kb / T);
+  long long ex_end = (long long)(ex + 1) * T;
+  auto advance = [&](long long& k0, int& rows, float& sc) __attribute__((always_inline)) {
+    rows = 0;
+    if constexpr (kFlat) {
+      k0 = next;
+      rows = (int)min((long long)kF32Rows, ke - next);
+      next += rows;
+      sc = 1.0f;
+    } else {
+      while (next < ke) {
+        if (next >= ex_end) {
+          ++ex;
+          ex_end += T;
+        }
+        sc = scale[ex];
+        if (sc > 0.0f) {
+          k0 = next;
+          rows = (int)min((long long)kF32Rows, min(ke, ex_end) - next);
+          next += rows;
+          return;
+        }
+        next = ex_end;
+      }
+    }
+  };
+  F32Chunk x0, x1;
+  long long k0 = 0;
+  int rows0 = 0, rows1 = 0;
+  float s0 = 0.0f, s1 = 0.0f, m_cur = 1.0f;
+  auto run = [&](int rows, float sc, F32Chunk& x) __attribute__((always_inline)) {
+    if constexpr (kFlat) {
+      sum(rows, 1.0f, x);
+    } else {
+      const float m = scale_mantissa(sc);
+      if (m != m_cur) {
+        const float r = m_cur / m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] *= r;
+        m_cur = m;
+      }
+      sum(rows, scale_pow2(sc), x);
+    }
+  };
+  advance(k0, rows0, s0);
+  if (rows0 > 0) load(k0, rows0, x0);
+  while (rows0 > 0) {
+    advance(k0, rows1, s1);
+    if (rows1 > 0) load(k0, rows1, x1);
+    run(rows0, s0, x0);
+    if (rows1 == 0) break;
+    advance(k0, rows0, s0);
+    if (rows0 > 0) load(k0, rows0, x0);
+    run(rows1, s1, x1);
+  }
+
+  // Block (i, j), entry r of lane l: row 16 (l / 16) + 4 r + i, column
+  // 4 (l % 16) + j of the tile.  In two halves (i): [wave][i, r, j][lane]
+  // through LDS, then each wave adds and stores a quarter.
+  const int plane_rows = args.plane_rows, plane_ld = args.plane_ld;
+  float* plane = args.partial + (size_t)split * plane_rows * plane_ld;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (h) __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 32; ++e) {
+      const int i = 2 * h + (e >> 4), r = (e >> 2) & 3, j = e & 3;
+      tile[(w * 32 + e) * 64 + lane] = acc[i][j][r] * m_cur;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e4 = 0; e4 < 2; ++e4) {
+      const int e = 8 * w + 4 * e4;
+      f32x4_t v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] = tile[(e + j) * 64 + lane];
+#pragma unroll
+        for (int u = 1; u < 4; ++u) v[j] += tile[(u * 32 + e + j) * 64 + lane];
+      }
+      const int m = m0 + 16 * kq + 4 * ((e >> 2) & 3) + 2 * h + (e >> 4), n = n0 + cl;
+      if (m < plane_rows && n < plane_ld)
+        *global_ptr<f32x4_t>(plane + (size_t)m * plane_ld + n) = v;
+    }
+  }
+}
+
+template <bool kFlat>
+__global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args args) {
+  __shared__ __attribute__((aligned(16))) float tile[4 * 32 * 64];
+  const int lin = xcd_linear_id(gridDim.x);
+  const int tiles_m = ceil_div(args.M, kF32Tile), tiles_n = ceil_div(args.N, kF32Tile);
+  const int split = __builtin_amdgcn_readfirstlane(lin / (tiles_m * tiles_n));
+  int tm, tn;
+  tile_coords<8>(lin - split * tiles_m * tiles_n, tiles_m, tiles_n, &tm, &tn);
+  const int m0 = __builtin_amdgcn_readfirstlane(tm) * kF32Tile;
+  const int n0 = __builtin_amdgcn_readfirstlane(tn) * kF32Tile;
+  if (m0 + kF32Tile <= args.M && n0 + kF32Tile <= args.N)
+    clipped_sum_f32_tile<kFlat, false>(args, m0, n0, split, tile);
+  else
+    clipped_sum_f32_tile<kFlat, true>(args, m0, n0, split, tile);
+}
+
+// The widths that its loads take (a row of at least 16 bytes, 16 rows within
+// 32-bit offsets).
+bool f32_shape(int B, int din, int dout) {
+  return B > 0 && din >= 4 && dout >= 4 && din < (1 << 26) && dout < (1 << 26);
+}
+
+// Workgroups per tile of the fp32 path: enough for two on every CU, each of a
+// wave's slices at least 64 rows.
+int f32_splits(int B, int T, int din, int dout) {
+  const long long tiles = (long long)ceil_div(din, kF32Tile) * ceil_div(dout, kF32Tile);
+  const long long K = (long long)B * T;
+  long long splits = (512 + tiles - 1) / tiles;
+  splits = splits < K / 256 ? splits : K / 256;
+  return (int)(splits < 1 ? 1 : (splits > 64 ? 64 : splits));
+}
+int f32_plane_rows(int dout) { return (dout + 1) & ~1; }
+int f32_plane_ld(int din) { return (din + 3) & ~3; }
+size_t f32_bytes(int B, int T, int din, int dout) {
+  return (size_t)f32_splits(B, T, din, dout) * (size_t)f32_plane_rows(dout) *
+         (size_t)f32_plane_ld(din) * sizeof(float);
 }
 
 // Bias: partial[split][m] = sum over examples e of the split of
@@ -1654,6 +1907,7 @@ extern "C" size_t dpc_clipped_sum_workspace_bytes(int B, int T, int din, int dou
   if (fast_shape(B, T, din, dout, dtype))
     return bytes + pad_bytes(B, T, din) + pad_bytes(B, T, dout) +
            split_bytes(fast_splits(B, T, din, dout), din, dout);
+  if (dtype == DPC_F32 && f32_shape(B, din, dout)) return bytes + f32_bytes(B, T, din, dout);
   const int splits = generic_splits(B, T, din, dout);
   if (splits > 1) bytes += (size_t)splits * (size_t)dout * (size_t)din * sizeof(float);
   return bytes;
@@ -1739,6 +1993,37 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
                          dim3(kThreads), 0, s, (const float*)args.partial, splits, args.ldg,
                          args.lda, ep);
     }
+  } else if (dtype == DPC_F32 && f32_shape(B, din, dout) && ws &&
+             ws_bytes >= pad_at + f32_bytes(B, T, din, dout)) {
+    const int splits = f32_splits(B, T, din, dout);
+    const long long K = (long long)B * T;
+    F32Args args;
+    args.A = (const float*)A;
+    args.G = (const float*)G;
+    args.scale = scale;
+    args.B = B;
+    args.T = T;
+    args.M = dout;
+    args.N = din;
+    args.splits = splits;
+    args.per = ((K + 4LL * splits - 1) / (4LL * splits) + kF32Rows - 1) / kF32Rows * kF32Rows;
+    args.plane_rows = f32_plane_rows(dout);
+    args.plane_ld = f32_plane_ld(din);
+    args.partial = (float*)((uint8_t*)ws + pad_at);
+    const long long blocks =
+        (long long)ceil_div(dout, kF32Tile) * ceil_div(din, kF32Tile) * splits;
+    if (blocks > 0x7fffffff) return DPC_ENOTSUP;
+    if (T == 1)
+      hipLaunchKernelGGL(clipped_sum_f32_kernel<true>, dim3((unsigned)blocks), dim3(kThreads), 0, s,
+                         args);
+    else
+      hipLaunchKernelGGL(clipped_sum_f32_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, s,
+                         args);
+    DPC_HIP_CHECK(hipGetLastError());
+    const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
+    hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, s, (const float*)args.partial, splits, args.plane_rows,
+                       args.plane_ld, ep);
   } else {
     int splits = generic_splits(B, T, din, dout);
     const size_t need = bias_ws_bytes(dout) + (size_t)splits * dout * (size_t)din * sizeof(float);

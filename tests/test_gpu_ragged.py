@@ -169,3 +169,33 @@ def test_gram_f64(dev, dtype, B, T, din, dout):
     gammas = sum(1.125 * (-(-d // 16) * 16) * 2.0**-52 for d in (din, dout))
     rows = A.double().square().sum(dim=(1, 2)) * G.double().square().sum(dim=(1, 2))
     assert (err <= 1.001 * (gammas + (T * T + 256) * 2.0**-52) * rows).all()
+
+
+# The fp32 MFMA path: chunks of 16 rows and their remainders, one token per
+# example (16 examples a chunk), 64-column tiles and their edges at any
+# alignment, one and several splits; a zero-scale example that holds NaN.
+@pytest.mark.parametrize("B,T,din,dout", [
+    (2, 2, 1, 1), (3, 5, 33, 17), (7, 19, 100, 67), (16, 130, 64, 64), (2, 300, 257, 66),
+    (40, 33, 512, 130), (2, 1, 7, 5), (40, 1, 65, 10), (300, 1, 64, 130), (1030, 1, 20, 64)])
+def test_clipped_sum_fp32(dev, B, T, din, dout):
+    g = torch.Generator().manual_seed(B + T + din)
+    A = torch.randn(B, T, din, generator=g)
+    G = torch.randn(B, T, dout, generator=g)
+    scale = torch.rand(B, generator=g) * torch.exp(3 * torch.randn(B, generator=g))
+    G[B // 2] = float("nan")
+    scale[B // 2] = 0.0
+    A_d, G_d, s_d = A.to(dev), G.to(dev), scale.to(dev)
+    got, _ = ops.clipped_sum(A_d, G_d, s_d)
+    keep = torch.arange(B) != B // 2
+    s64, A64, G64 = scale[keep].double(), A[keep].double(), G[keep].double()
+    want = _exact(A64, G64, s64)
+    # Sums of K = B T products in fp32, each partial sum rounded once (2^-24),
+    # the scaled operand or accumulator twice more.
+    mag = _exact(A64.abs(), G64.abs(), s64)
+    assert ((got.cpu().double() - want).abs() <= (B * T + 3) * 2.0**-24 * mag).all()
+    assert _rel(got.cpu(), want) < 2e-6
+    spec = ops.NoiseSpec(sigma=0.5, mode=nat.NOISE_PHILOX, seed=7, leaf_id=2)
+    half, _ = ops.clipped_sum(A_d, G_d, s_d, normalize_by=3.0, out_dtype=torch.bfloat16)
+    noised, _ = ops.clipped_sum(A_d, G_d, s_d, normalize_by=3.0, out_dtype=torch.bfloat16,
+                                noise=spec)
+    assert torch.equal(noised, ops.add_noise(half, 0.5, seed=7, leaf_id=2))
