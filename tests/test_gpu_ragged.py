@@ -199,3 +199,50 @@ def test_clipped_sum_fp32(dev, B, T, din, dout):
     noised, _ = ops.clipped_sum(A_d, G_d, s_d, normalize_by=3.0, out_dtype=torch.bfloat16,
                                 noise=spec)
     assert torch.equal(noised, ops.add_noise(half, 0.5, seed=7, leaf_id=2))
+
+
+# Materialised leaves whose rows start at any element boundary, leaves shorter
+# than 8 elements, tiles and waves that a leaf ends in, batches that 8 does not
+# divide; fp16 beside bf16 and fp32; diagnostics and the second moment.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B", [1, 7, 17])
+@pytest.mark.parametrize("out", [None, torch.float32])
+def test_leaves_unaligned_match_oracle(dev, dtype, B, out):
+    from opake_amd.clipping import leaves_clip_sum
+    from oracle import clip_oracle
+
+    g = torch.Generator().manual_seed(B)
+    shapes = [(1,), (7,), (9,), (511,), (513,), (2047,), (2049,), (3, 683), (4096,), (5, 1031)]
+    leaves = [(torch.randn(B, *s, generator=g) * 0.05).to(dtype) for s in shapes]
+    leaves[3][0, 5] = float("nan")
+    leaves[6][B - 1, 2048] = float("inf")
+    res = leaves_clip_sum([x.to(dev) for x in leaves], 1.0, with_postsq=True, second_moment=True,
+                          sum_dtypes=None if out is None else {dtype: (torch.float32, out)})
+    want = clip_oracle.stream_clip_and_sum(leaves, clip_oracle.conservative_bound(1.0),
+                                           second_moment=True,
+                                           reduce_dtype=None if out is None else {dtype: out})
+    torch.testing.assert_close(res.norms.cpu().double(), want.norms.double(), rtol=1e-6, atol=0)
+    scale = res.scales[dtype][0].cpu()
+    for got, sq, x in zip(res.reduced, res.squared, leaves):
+        # The reference's arithmetic on the device's scales: one rounding per
+        # product, fp32 sums in example order -- the same bits.
+        clean = torch.nan_to_num(x.float(), nan=0.0, posinf=0.0, neginf=0.0)
+        prod = clean * scale.view(B, *[1] * (x.dim() - 1))
+        stored = prod.to(dtype)
+        tiny = torch.finfo(dtype).smallest_normal
+        up = (stored.float().abs() <= tiny) & (stored.float().abs() > prod.abs())
+        if dtype != torch.float32:
+            stored = torch.where(up, torch.zeros_like(stored), stored)
+        acc, acc2 = torch.zeros(x.shape[1:]), torch.zeros(x.shape[1:])
+        for b in range(B):
+            acc = acc + stored[b].float()
+            acc2 = acc2 + (stored[b].float() ** 2).to(dtype).float()
+        assert torch.equal(got.cpu(), acc.to(out or dtype))
+        assert torch.equal(sq.cpu(), acc2.to(out or dtype))
+    post = torch.zeros(B, dtype=torch.float64)
+    for x in leaves:
+        clean = torch.nan_to_num(x.float(), nan=0.0, posinf=0.0, neginf=0.0)
+        s = (clean * scale.view(B, *[1] * (x.dim() - 1))).to(dtype).double()
+        post += (s.reshape(B, -1) ** 2).sum(dim=1)
+    # fp32 sums of 512 squares per wave (fp64 for fp16), then fp64.
+    torch.testing.assert_close(res.post_sq.cpu().double(), post, rtol=1e-4 * 2**-4, atol=0)
