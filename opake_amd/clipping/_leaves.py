@@ -256,7 +256,7 @@ class LeafBatch:
         stream = nat.stream_handle(self.device)
         reduced = [None] * self.L
         squared = [None] * self.L
-        post_sq = torch.zeros(B, dtype=torch.float64, device=self.device) if with_postsq else None
+        post_sq = None  # a batch holds at least one leaf, so one part
         for p, ptrs in zip(self.parts, self.ptr_tables):
             h, dtype = p.host, p.dtype
             acc, out_dtype = (sum_dtypes or {}).get(dtype, (_sum_dtype_of(dtype, None), dtype))
@@ -291,12 +291,12 @@ class LeafBatch:
                          nat.ptr(flat), nat.ptr(flat_sq), nat.dtype_code(out_dtype, wide=True),
                          nat.ptr(tile_sq), stream)
             if with_postsq:
-                post_sq += tile_sq.sum(dim=1, dtype=torch.float64)
-            for j, i in enumerate(h.members):
-                off, n = h.out_starts[j], h.numels[j]
-                reduced[i] = flat[off:off + n].view(self.leaves[i].shape[1:])
-                if second_moment:
-                    squared[i] = flat_sq[off:off + n].view(self.leaves[i].shape[1:])
+                part_sq = tile_sq.sum(dim=1, dtype=torch.float64)
+                post_sq = part_sq if post_sq is None else post_sq + part_sq
+            for sums, buf in ((reduced, flat), (squared, flat_sq)):
+                if buf is not None:
+                    for i, x in zip(h.members, buf.split(h.numels)):
+                        sums[i] = x.view(self.leaves[i].shape[1:])
         if second_moment:
             return reduced, post_sq, squared
         return reduced, post_sq
@@ -342,29 +342,28 @@ def leaves_clip_sum(leaves, clipping_norm, *, kind: str = "fixed", gamma: float 
         group_sq = torch.empty((n_groups, B), dtype=torch.float64, device=device)
         nat.call("dpc_group_sum_f64", nat.ptr(leaf_sq), B, L, L, 1, nat.ptr(col_group),
                  n_groups, nat.ptr(group_sq), 0, stream)
-        cfs = [ops.clip_factors(group_sq[k], bound_of(bounds[k]), guards,
-                                kind=scale_kind, gamma=gamma,
-                                count_threshold=num.float32_of(bounds[k]))
-               for k in range(n_groups)]
+        cf = ops.clip_factors_groups(group_sq, [bound_of(b) for b in bounds], guards,
+                                     kind=scale_kind, gamma=gamma,
+                                     count_thresholds=[num.float32_of(b) for b in bounds])
         # The clip kernel's norms are (float)sqrt(sq): the diagnostic when the
         # reduction dtype is float32 (_streaming.py:174-180).
-        if acc == torch.float32:
-            norms = torch.sqrt(sq).to(acc)
-            group_norms = torch.stack([cf.norms for cf in cfs])
-        else:
-            norms = torch.sqrt(sq).to(acc)
-            group_norms = torch.sqrt(group_sq).to(acc)
-        nclipped = torch.cat([cf.nclipped for cf in cfs])
+        norms = torch.sqrt(sq).to(acc)
+        group_norms = cf.norms if acc == torch.float32 else torch.sqrt(group_sq).to(acc)
+        nclipped = cf.nclipped
+        rows, rows64 = cf.scale, cf.scale64
     else:
-        cfs = [ops.clip_factors(sq, bound_of(bounds[0]), guards, kind=scale_kind,
-                                gamma=gamma, count_threshold=num.float32_of(bounds[0]))]
-        norms = cfs[0].norms if acc == torch.float32 else torch.sqrt(sq).to(acc)
-        group_norms, nclipped = None, cfs[0].nclipped
+        cf = ops.clip_factors(sq, bound_of(bounds[0]), guards, kind=scale_kind,
+                              gamma=gamma, count_threshold=num.float32_of(bounds[0]))
+        norms = cf.norms if acc == torch.float32 else torch.sqrt(sq).to(acc)
+        group_norms, nclipped = None, cf.nclipped
+        rows = cf.scale.unsqueeze(0)
+        rows64 = None if cf.scale64 is None else cf.scale64.unsqueeze(0)
+    # [G, guards, B] -> each storage dtype's [G, B] rows.
     scales, scales64 = {}, {}
     for gi, dtype in enumerate(batch.dtypes):
-        scales[dtype] = torch.stack([cf.scale[gi] for cf in cfs])
+        scales[dtype] = rows[:, gi].contiguous()
         if mults[dtype] == torch.float64:
-            scales64[dtype] = torch.stack([cf.scale64[gi] for cf in cfs])
+            scales64[dtype] = rows64[:, gi].contiguous()
     if sum_dtypes is None:
         sum_dtypes = {dt: (_sum_dtype_of(dt, compute_dtype), dt) for dt in batch.dtypes}
     out = batch.apply(scales, leaf_groups if grouped else None, sum_dtypes, with_postsq,

@@ -488,8 +488,13 @@ def ghost_clip_captured(
     buckets = {}
     for L in segmented:
         buckets.setdefault((L.A.shape[1], L.G.shape[1], L.A.dtype), []).append(L)
-    bucket_layouts = [(members, ops.SegmentLayout([L.cap.segments for L in members], device))
-                      for members in buckets.values()]
+    bucket_layouts, sum_layouts = [], {}
+    for members in buckets.values():
+        # Layers of several shapes over the same segments share their layout.
+        key = tuple(map(tuple, (L.cap.segments for L in members)))
+        if key not in sum_layouts:
+            sum_layouts[key] = ops.SegmentLayout(key, device, gram=False)
+        bucket_layouts.append((members, sum_layouts[key]))
 
     # Materialised per-example gradients: per-leaf squared norms, summed into
     # their groups in leaf order.

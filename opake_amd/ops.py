@@ -570,7 +570,9 @@ class SegmentLayout:
     Two Gram schedules are kept: tile-pair items for every segment (any
     dtype), and for the bf16 MFMA path the split kernel's items -- two per
     segment of 1 .. 320 rows (A and G) -- with tile-pair items for the
-    longer segments only.
+    longer segments only.  ``gram=False`` builds neither (a layout for
+    :func:`grouped_clipped_sum` alone: the schedules are most of the host work,
+    0.3 ms for 8 problems of 16 segments).
     """
 
     MAX_GRAM_PROBLEMS = 64
@@ -661,7 +663,7 @@ class SegmentLayout:
             out[x * per:x * per + n] = items[idx]
         return out
 
-    def __init__(self, lengths, device, gram_weights=None, gram_dims=None):
+    def __init__(self, lengths, device, gram_weights=None, gram_dims=None, gram=True):
         import numpy as np
 
         lens = np.asarray(lengths, dtype=np.int64)
@@ -674,10 +676,19 @@ class SegmentLayout:
         self.max_rows = int(self.rows.max()) if self.E else 0
         if self.max_rows >= 1 << 30:
             raise ConfigurationError("too many rows in one problem")
-        weights = np.ones(self.E) if gram_weights is None else np.asarray(gram_weights, float)
         flat = lens.reshape(-1)
         row0 = (np.cumsum(lens, axis=1) - lens).reshape(-1)
         group = np.repeat(np.arange(self.E, dtype=np.int64), self.K)
+        self.max_steps = int(((flat + _STEP_ROWS - 1) // _STEP_ROWS).sum())
+        self.device = torch.device(device)
+        self.has_gram = bool(gram)
+        if not gram:
+            self._buf = device_table(np.concatenate([row0, flat, group, self.rows]), np.int32,
+                                     device)
+            self.seg_row0, self.seg_len, self.seg_group, self.rows_dev = self._buf.split(
+                [self.S, self.S, self.S, self.E])
+            return
+        weights = np.ones(self.E) if gram_weights is None else np.asarray(gram_weights, float)
         nt = (flat + _GRAM_TILE - 1) // _GRAM_TILE
         npairs = nt * (nt + 1) // 2
         if npairs.size and npairs.max() >= 1 << 16:
@@ -721,7 +732,6 @@ class SegmentLayout:
         else:
             long_items = np.zeros((0, 4), dtype=np.int64)
         self.n_sets = int(short.sum())
-        self.max_steps = int(((flat + _STEP_ROWS - 1) // _STEP_ROWS).sum())
         # One int32 buffer: row0 [S] | len [S] | group [S] | rows [E] |
         # item_start [S + 1] | tile-pair items of every segment | tile-pair
         # items of the long segments | split items.
@@ -736,7 +746,6 @@ class SegmentLayout:
         self.n_long_items = len(long_items)
         self.n_set_items = len(set_items)
         self._buf = buf
-        self.device = torch.device(device)
 
 
 def _ptr_table(tensors, device) -> torch.Tensor:
@@ -774,6 +783,8 @@ def grouped_gram_sqnorms(A_list, G_list, layout: SegmentLayout, *, return_error:
     _, _, dtype = _check_grouped(A_list, G_list, layout, same_shape=False)
     if layout.E > SegmentLayout.MAX_GRAM_PROBLEMS:
         raise ConfigurationError("at most 64 problems per grouped Gram call")
+    if not layout.has_gram:
+        raise ConfigurationError("the layout was built without its Gram schedules (gram=False)")
     dims = (ctypes.c_int * (2 * layout.E))(
         *[v for A, G in zip(A_list, G_list) for v in (A.shape[1], G.shape[1])])
     seg_sq = torch.empty((layout.E, layout.K), dtype=torch.float64, device=dev)

@@ -85,3 +85,15 @@ def test_split_schedule_runs_expensive_items_first_per_xcd():
         blocks = np.where(part[:, 2] > 288, 55, np.where(part[:, 2] > 256, 45, 36))
         cost = k * blocks
         assert (np.diff(cost) <= 0).all(), x
+
+
+def test_sum_layout_has_the_full_layouts_tables():
+    """gram=False leaves the Gram schedules out and nothing else."""
+    lengths = [[3, 0, 65, 700], [64, 1, 0, 128]]
+    full = ops.SegmentLayout(lengths, "cpu")
+    part = ops.SegmentLayout(lengths, "cpu", gram=False)
+    for name in ("seg_row0", "seg_len", "seg_group", "rows_dev"):
+        assert getattr(part, name).tolist() == getattr(full, name).tolist()
+    assert (part.S, part.E, part.K, part.max_rows, part.max_steps) == (
+        full.S, full.E, full.K, full.max_rows, full.max_steps)
+    assert full.has_gram and not part.has_gram
