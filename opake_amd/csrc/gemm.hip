@@ -156,6 +156,16 @@ __device__ __forceinline__ void emit_quad(const Epilogue& ep, int m, int n, cons
   }
 }
 
+// emit_quad for any N: odd rows start at any alignment, so they go value by value.
+__device__ __forceinline__ void emit_rows(const Epilogue& ep, int m, int n, const float v[2][2]) {
+  if (ep.N & 1) {
+    emit_pair(ep, m, n, v[0][0], v[1][0]);
+    emit_pair(ep, m, n + 1, v[0][1], v[1][1]);
+  } else {
+    emit_quad(ep, m, n, v);
+  }
+}
+
 #pragma clang fp contract(off)
 // finish_value with the epilogue's workgroup-uniform choices fixed at compile
 // time (bf16 output, / normalize_by, noise added): the tile epilogues pick
@@ -1150,31 +1160,38 @@ split_reduce_kernel(const float* __restrict__ partial, int splits, int rows, int
       v[r][1] += t.y;
     }
   }
-  if (ep.N & 1) {
-    // The rows start at any alignment: value by value.
-    emit_pair(ep, m, n, v[0][0], v[1][0]);
-    emit_pair(ep, m, n + 1, v[0][1], v[1][1]);
-  } else {
-    emit_quad(ep, m, n, v);
-  }
+  emit_rows(ep, m, n, v);
 }
 
-// Split-K factor of a dense fast-path launch: launches of fewer than 192
-// output tiles (on 256 CUs) take their K steps in up to 8 slices so that the
-// grid fills the chip; the slices' fp32 tiles go through a workspace.
+// Split-K factor of a dense fast-path launch of one layer: launches of fewer
+// than 192 output tiles (on 256 CUs) take their K steps in slices, the slices'
+// fp32 tiles going through a workspace.  The factor with the least of a slice's
+// steps (1.7 us each, as measured) plus the slices' traffic (written and read
+// once, 5 bytes/ps), one workgroup per CU and at least four steps a slice:
+// [48, 1000, 512 x 512] in 48 slices 60 us with its launches (8, the former
+// limit: 132), [48, 1000, 256 x 256] 49 (130), [24, 197, 768 x 3072] in 6 52 (4,
+// by powers of two: 57).
 int fast_splits(int B, int T, int din, int dout) {
   const int ntiles = ceil_div(dout, kBM) * ceil_div(din, kBN);
   if (ntiles >= 192) return 1;
-  int splits = 1;
   const long long steps = (long long)B * ceil_div(T, kBK);
-  while (splits < 8 && ntiles * splits * 2 <= 256 && steps >= 8LL * splits * 2) splits *= 2;
-  return splits;
+  const double plane_us = 8e-6 * (double)din * (double)dout / 5.0;
+  int best = 1;
+  double best_us = 1.7 * (double)steps;
+  for (int sp = 2; sp <= 64 && ntiles * sp <= 256 && steps >= 4LL * sp; ++sp) {
+    const double us = 1.7 * (double)((steps + sp - 1) / sp) + sp * plane_us;
+    if (us < best_us) {
+      best = sp;
+      best_us = us;
+    }
+  }
+  return best;
 }
 
 #undef DPC_WAIT_VMCNT
 
-// Generic path (calls without the workspace of the paths above and below, bf16
-// with one token or a few chunks): any T, float32 or bf16 operands; 64 x 64 tiles with a 4 x 4
+// Generic path (calls without the workspace of the paths above and below, or
+// of widths below 4): any T, float32 or bf16 operands; 64 x 64 tiles with a 4 x 4
 // FMA block per thread.  K is walked in chunks of at most 16 rows that never
 // straddle two examples: G is staged multiplied by the power of two of its
 // example's scale (exact) and the accumulators carry the mantissa (they hold
@@ -1329,7 +1346,7 @@ int generic_splits(int B, int T, int din, int dout) {
 // of an operand holds the columns 4 j + i -- so two loads feed 16 MFMAs of 32
 // cycles, with no LDS and no barrier in the loop; 16 rows are in flight while
 // 16 are summed.  The four waves of a workgroup take consecutive slices and add
-// their tiles through LDS in order; `splits` workgroups per tile take
+// their tiles through LDS in order; `splits` > 1 workgroups per tile take
 // consecutive parts of K and write raw tiles, which split_reduce_kernel adds in
 // order and finishes.  Rows of any width are read (16-byte loads at 4-byte
 // alignment).
@@ -1346,30 +1363,56 @@ int generic_splits(int B, int T, int din, int dout) {
 // the loads, so edge tiles have a body of their own.
 constexpr int kF32Tile = 64;
 constexpr int kF32Rows = 16;  // rows of a chunk
-typedef f32x4_t f32x4_align4_t __attribute__((aligned(4)));
+constexpr double kF32MaxBf16Flops = 1.5e9;
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// Four elements of a row, at any element boundary.
+template <typename In>
+struct F32Quad;
+template <>
+struct F32Quad<float> {
+  typedef f32x4_t Raw;
+  typedef f32x4_t Load __attribute__((aligned(4)));
+};
+template <>
+struct F32Quad<uint16_t> {
+  typedef u32x2_t Raw;
+  typedef u32x2_t Load __attribute__((aligned(2)));
+};
+__device__ __forceinline__ f32x4_t quad_f32(f32x4_t x) { return x; }
+__device__ __forceinline__ f32x4_t quad_f32(u32x2_t x) {
+  const uint32_t lo = x[0], hi = x[1];
+  return f32x4_t{__builtin_bit_cast(float, lo << 16), __builtin_bit_cast(float, lo & 0xffff0000u),
+                 __builtin_bit_cast(float, hi << 16), __builtin_bit_cast(float, hi & 0xffff0000u)};
+}
 
+template <typename In>
 struct F32Chunk {
-  f32x4_t g[4], a[4];  // rows 4 q + l / 16
-  float s[4];          // kFlat: those rows' scales
+  typename F32Quad<In>::Raw g[4], a[4];  // rows 4 q + l / 16
+  float s[4];                            // kFlat: those rows' scales
 };
 
+template <typename In>
 struct F32Args {
-  const float* A;      // [B * T, N]
-  const float* G;      // [B * T, M]
+  const In* A;         // [B * T, N]
+  const In* G;         // [B * T, M]
   const float* scale;  // [B]
   int B, T, M, N;
   int splits;
   long long per;  // rows of a wave's slice
+  // splits > 1: raw tiles [splits][plane_rows][plane_ld]; else null, and the
+  // kernel finishes its tiles itself.
   int plane_rows, plane_ld;
-  float* partial;  // [splits][plane_rows][plane_ld]
+  float* partial;
+  Epilogue ep;
 };
 
 // kEdge: a tile that the matrix does not fill.  Its 16-byte loads start at the
 // row's last 4 columns at most, and the values move to their places before the
 // product (the columns past the matrix, never stored, hold whatever comes).
-template <bool kFlat, bool kEdge>
-__device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0, int n0, int split,
-                                                     float* tile) {
+template <typename In, bool kFlat, bool kEdge>
+__device__ __forceinline__ void clipped_sum_f32_tile(const F32Args<In>& args, int m0, int n0,
+                                                     int split, float* tile) {
+  using Load = typename F32Quad<In>::Load;
   const int M = args.M, N = args.N, T = args.T;
   const float* scale = args.scale;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1379,15 +1422,15 @@ __device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0
   const int cg = kEdge ? min(m0 + cl, M - 4) : m0 + cl, ca = kEdge ? min(n0 + cl, N - 4) : n0 + cl;
 
   // Rows k0 + 4 q + l / 16 of a chunk of `rows` rows; past them its first row.
-  auto load = [&](long long k0, int rows, F32Chunk& x) __attribute__((always_inline)) {
-    const float* gb = args.G + k0 * M;
-    const float* ab = args.A + k0 * N;
+  auto load = [&](long long k0, int rows, F32Chunk<In>& x) __attribute__((always_inline)) {
+    const In* gb = args.G + k0 * M;
+    const In* ab = args.A + k0 * N;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int r = 4 * q + kq;
       const uint32_t rr = r < rows ? r : 0;
-      x.g[q] = *global_ptr<const f32x4_align4_t>(gb + (rr * (uint32_t)M + (uint32_t)cg));
-      x.a[q] = *global_ptr<const f32x4_align4_t>(ab + (rr * (uint32_t)N + (uint32_t)ca));
+      x.g[q] = *global_ptr<const Load>(gb + (rr * (uint32_t)M + (uint32_t)cg));
+      x.a[q] = *global_ptr<const Load>(ab + (rr * (uint32_t)N + (uint32_t)ca));
       if (kFlat) x.s[q] = scale[k0 + rr];
     }
   };
@@ -1409,12 +1452,12 @@ __device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  auto sum_rows = [&](int rows, float p2, F32Chunk& x, auto Full) __attribute__((always_inline)) {
+  auto sum_rows = [&](int rows, float p2, F32Chunk<In>& x, auto Full) __attribute__((always_inline)) {
     constexpr bool kFull = decltype(Full)::value;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (!kFull && 4 * q >= rows) break;
-      f32x4_t g = x.g[q], a = x.a[q];
+      f32x4_t g = quad_f32(x.g[q]), a = quad_f32(x.a[q]);
       const float sc = kFlat ? x.s[q] : p2;
       place(g, m0 + cl - cg);
       place(a, n0 + cl - ca);
@@ -1437,7 +1480,7 @@ __device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(g[i], a[j], acc[i][j], 0, 0, 0);
     }
   };
-  auto sum = [&](int rows, float p2, F32Chunk& x) __attribute__((always_inline)) {
+  auto sum = [&](int rows, float p2, F32Chunk<In>& x) __attribute__((always_inline)) {
     if (rows == kF32Rows)
       sum_rows(rows, p2, x, std::true_type());
     else
@@ -1473,11 +1516,11 @@ __device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0
       }
     }
   };
-  F32Chunk x0, x1;
+  F32Chunk<In> x0, x1;
   long long k0 = 0;
   int rows0 = 0, rows1 = 0;
   float s0 = 0.0f, s1 = 0.0f, m_cur = 1.0f;
-  auto run = [&](int rows, float sc, F32Chunk& x) __attribute__((always_inline)) {
+  auto run = [&](int rows, float sc, F32Chunk<In>& x) __attribute__((always_inline)) {
     if constexpr (kFlat) {
       sum(rows, 1.0f, x);
     } else {
@@ -1506,39 +1549,41 @@ __device__ __forceinline__ void clipped_sum_f32_tile(const F32Args& args, int m0
   }
 
   // Block (i, j), entry r of lane l: row 16 (l / 16) + 4 r + i, column
-  // 4 (l % 16) + j of the tile.  In two halves (i): [wave][i, r, j][lane]
-  // through LDS, then each wave adds and stores a quarter.
-  const int plane_rows = args.plane_rows, plane_ld = args.plane_ld;
-  float* plane = args.partial + (size_t)split * plane_rows * plane_ld;
+  // 4 (l % 16) + j of the tile.  All four waves' entries [wave][i, r, j][lane] go
+  // through LDS; wave w then adds and finishes (or stores) the rows of r = w.
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (h) __syncthreads();
+  for (int e = 0; e < 64; ++e)
+    tile[(w * 64 + e) * 64 + lane] = acc[e >> 4][e & 3][(e >> 2) & 3] * m_cur;
+  __syncthreads();
+  auto value = [&](int i, int j) __attribute__((always_inline)) {
+    const float* p = tile + ((i * 4 + w) * 4 + j) * 64 + lane;
+    float v = p[0];
 #pragma unroll
-    for (int e = 0; e < 32; ++e) {
-      const int i = 2 * h + (e >> 4), r = (e >> 2) & 3, j = e & 3;
-      tile[(w * 32 + e) * 64 + lane] = acc[i][j][r] * m_cur;
+    for (int u = 1; u < 4; ++u) v += p[u * 64 * 64];
+    return v;
+  };
+  const int mr = m0 + 16 * kq + 4 * w, n = n0 + cl;
+  if (args.partial) {
+    float* plane = args.partial + (size_t)split * args.plane_rows * args.plane_ld;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (mr + i < args.plane_rows && n < args.plane_ld)
+        *global_ptr<f32x4_t>(plane + (size_t)(mr + i) * args.plane_ld + n) =
+            f32x4_t{value(i, 0), value(i, 1), value(i, 2), value(i, 3)};
     }
-    __syncthreads();
-#pragma unroll
-    for (int e4 = 0; e4 < 2; ++e4) {
-      const int e = 8 * w + 4 * e4;
-      f32x4_t v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = tile[(e + j) * 64 + lane];
-#pragma unroll
-        for (int u = 1; u < 4; ++u) v[j] += tile[(u * 32 + e + j) * 64 + lane];
-      }
-      const int m = m0 + 16 * kq + 4 * ((e >> 2) & 3) + 2 * h + (e >> 4), n = n0 + cl;
-      if (m < plane_rows && n < plane_ld)
-        *global_ptr<f32x4_t>(plane + (size_t)m * plane_ld + n) = v;
-    }
+    return;
+  }
+#pragma unroll 1
+  for (int it = 0; it < 4; ++it) {
+    const int i = it & 2, j = 2 * (it & 1);
+    const float v[2][2] = {{value(i, j), value(i, j + 1)}, {value(i + 1, j), value(i + 1, j + 1)}};
+    emit_rows(args.ep, mr + i, n + j, v);
   }
 }
 
-template <bool kFlat>
-__global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args args) {
-  __shared__ __attribute__((aligned(16))) float tile[4 * 32 * 64];
+template <typename In, bool kFlat>
+__global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args<In> args) {
+  __shared__ __attribute__((aligned(16))) float tile[4 * 64 * 64];
   const int lin = xcd_linear_id(gridDim.x);
   const int tiles_m = ceil_div(args.M, kF32Tile), tiles_n = ceil_div(args.N, kF32Tile);
   const int split = __builtin_amdgcn_readfirstlane(lin / (tiles_m * tiles_n));
@@ -1547,15 +1592,25 @@ __global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args ar
   const int m0 = __builtin_amdgcn_readfirstlane(tm) * kF32Tile;
   const int n0 = __builtin_amdgcn_readfirstlane(tn) * kF32Tile;
   if (m0 + kF32Tile <= args.M && n0 + kF32Tile <= args.N)
-    clipped_sum_f32_tile<kFlat, false>(args, m0, n0, split, tile);
+    clipped_sum_f32_tile<In, kFlat, false>(args, m0, n0, split, tile);
   else
-    clipped_sum_f32_tile<kFlat, true>(args, m0, n0, split, tile);
+    clipped_sum_f32_tile<In, kFlat, true>(args, m0, n0, split, tile);
 }
 
-// The widths that its loads take (a row of at least 16 bytes, 16 rows within
-// 32-bit offsets).
-bool f32_shape(int B, int din, int dout) {
-  return B > 0 && din >= 4 && dout >= 4 && din < (1 << 26) && dout < (1 << 26);
+// The calls it takes: every float32 one of widths that its loads take (a row
+// of at least four elements, 16 rows within 32-bit offsets), and bf16 ones of
+// one token per example (63 of the 64 rows of a bf16 kernel's step would be
+// empty) or of less work than the bf16 kernel's start, finish, padding and
+// split-K are worth (its matrix rate is 16 times higher): B, T, din, dout = 4,
+// 24, 64, 96 takes 10 us here and 20 there (both with their launches), 8, 20,
+// 63, 65 12 and 28, 64, 2, 1024, 1024 22 and 40, 16, 128, 512, 512 (1.1 GFLOP)
+// 24 and 26, 16, 100, 1023, 511 (1.7) 33 and 38, but 32, 100, 768, 768 (3.8) 66
+// and 35; 256 tokens of one example each, 512 x 512, 18, and 1024 of 2048 x 2048
+// 101 (15 and 580 in the generic kernel).
+bool f32_shape(int B, int T, int din, int dout, int dtype) {
+  if (B <= 0 || din < 4 || dout < 4 || din >= (1 << 26) || dout >= (1 << 26)) return false;
+  if (dtype == DPC_F32 || T == 1) return true;
+  return 2.0 * B * T * (double)din * dout < kF32MaxBf16Flops;
 }
 
 // Workgroups per tile of the fp32 path: enough for two on every CU, each of a
@@ -1570,8 +1625,9 @@ int f32_splits(int B, int T, int din, int dout) {
 int f32_plane_rows(int dout) { return (dout + 1) & ~1; }
 int f32_plane_ld(int din) { return (din + 3) & ~3; }
 size_t f32_bytes(int B, int T, int din, int dout) {
-  return (size_t)f32_splits(B, T, din, dout) * (size_t)f32_plane_rows(dout) *
-         (size_t)f32_plane_ld(din) * sizeof(float);
+  const int splits = f32_splits(B, T, din, dout);
+  if (splits == 1) return 0;
+  return (size_t)splits * (size_t)f32_plane_rows(dout) * (size_t)f32_plane_ld(din) * sizeof(float);
 }
 
 // Bias: partial[split][m] = sum over examples e of the split of
@@ -1849,24 +1905,11 @@ size_t bias_ws_bytes(int dout) {
 }
 int padded_width(int d) { return (d + 7) & ~7; }
 // The bf16 MFMA path: any T of at least two tokens (T % 64 != 0: the ragged
-// body; its out-of-range offset must lie past the operands).  One token per
-// example leaves 63 of a step's 64 rows empty: those take the generic kernel,
-// which packs 16 examples into a chunk, and so do the calls of a few chunks
-// where the 512-thread kernel's start and finish (and the padding launches)
-// cost more than the chunks: B, T, din, dout = 4, 2, 64, 64 takes 16.3 us
-// there and 18.4 here, 2, 3, 9, 7 15.8 and 24.4; past the line 8, 20, 63, 65
-// takes 36.2 and 28.4 us, 64, 2, 1024, 1024 75 and 40, 16, 100, 1023, 511 254
-// and 38, 32, 197, 768, 768 368 and 42.
-bool few_chunks(int B, int T, int din, int dout) {
-  const bool aligned = din % 8 == 0 && dout % 8 == 0;
-  if (T % kBK == 0 && aligned) return false;
-  return (long long)B * ceil_div(T, 16) <= (aligned ? 4 : 8) &&
-         (long long)din * dout <= 512 * 512;
-}
+// body; its out-of-range offset must lie past the operands).
 bool fast_shape(int B, int T, int din, int dout, int dtype) {
   const size_t rows = (size_t)B * (size_t)T;
   const size_t limit = T % kBK == 0 ? (size_t)1 << 31 : (size_t)kOutOfRange;
-  return dtype == DPC_BF16 && T > 1 && B > 0 && !few_chunks(B, T, din, dout) &&
+  return dtype == DPC_BF16 && T > 1 && B > 0 &&
          rows * (size_t)padded_width(din > dout ? din : dout) * 2 < limit;
 }
 // Bytes of the padded operand copies (0 for widths that are multiples of 8).
@@ -1904,10 +1947,10 @@ pad_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, lo
 extern "C" size_t dpc_clipped_sum_workspace_bytes(int B, int T, int din, int dout, int dtype) {
   if (dout <= 0 || din <= 0 || T <= 0 || B < 0) return 0;
   size_t bytes = bias_ws_bytes(dout);
+  if (f32_shape(B, T, din, dout, dtype)) return bytes + f32_bytes(B, T, din, dout);
   if (fast_shape(B, T, din, dout, dtype))
     return bytes + pad_bytes(B, T, din) + pad_bytes(B, T, dout) +
            split_bytes(fast_splits(B, T, din, dout), din, dout);
-  if (dtype == DPC_F32 && f32_shape(B, din, dout)) return bytes + f32_bytes(B, T, din, dout);
   const int splits = generic_splits(B, T, din, dout);
   if (splits > 1) bytes += (size_t)splits * (size_t)dout * (size_t)din * sizeof(float);
   return bytes;
@@ -1953,8 +1996,11 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
   // caller without the workspace for it gets the generic kernel.
   const size_t pad_a = pad_bytes(B, T, din), pad_g = pad_bytes(B, T, dout);
   const size_t pad_at = bias_ws_bytes(dout), split_at = pad_at + pad_a + pad_g;
+  const size_t f32_ws = f32_bytes(B, T, din, dout);
+  const bool f32 = f32_shape(B, T, din, dout, dtype) &&
+                   (f32_ws == 0 || (ws && ws_bytes >= pad_at + f32_ws));
   const bool fast =
-      fast_shape(B, T, din, dout, dtype) && plan != nullptr &&
+      !f32 && fast_shape(B, T, din, dout, dtype) && plan != nullptr &&
       (pad_a + pad_g == 0 || (ws && ws_bytes >= split_at + split_bytes(1, din, dout)));
   if (fast) {
     const long long rows = (long long)B * T;
@@ -1993,37 +2039,46 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
                          dim3(kThreads), 0, s, (const float*)args.partial, splits, args.ldg,
                          args.lda, ep);
     }
-  } else if (dtype == DPC_F32 && f32_shape(B, din, dout) && ws &&
-             ws_bytes >= pad_at + f32_bytes(B, T, din, dout)) {
+  } else if (f32) {
     const int splits = f32_splits(B, T, din, dout);
-    const long long K = (long long)B * T;
-    F32Args args;
-    args.A = (const float*)A;
-    args.G = (const float*)G;
-    args.scale = scale;
-    args.B = B;
-    args.T = T;
-    args.M = dout;
-    args.N = din;
-    args.splits = splits;
-    args.per = ((K + 4LL * splits - 1) / (4LL * splits) + kF32Rows - 1) / kF32Rows * kF32Rows;
-    args.plane_rows = f32_plane_rows(dout);
-    args.plane_ld = f32_plane_ld(din);
-    args.partial = (float*)((uint8_t*)ws + pad_at);
+    const int prows = f32_plane_rows(dout), pld = f32_plane_ld(din);
+    float* partial = splits > 1 ? (float*)((uint8_t*)ws + pad_at) : nullptr;
     const long long blocks =
         (long long)ceil_div(dout, kF32Tile) * ceil_div(din, kF32Tile) * splits;
     if (blocks > 0x7fffffff) return DPC_ENOTSUP;
-    if (T == 1)
-      hipLaunchKernelGGL(clipped_sum_f32_kernel<true>, dim3((unsigned)blocks), dim3(kThreads), 0, s,
-                         args);
+    auto run = [&](auto* a, auto* g) {
+      using In = std::remove_const_t<std::remove_pointer_t<decltype(a)>>;
+      const long long K = (long long)B * T;
+      F32Args<In> args;
+      args.A = a;
+      args.G = g;
+      args.scale = scale;
+      args.B = B;
+      args.T = T;
+      args.M = dout;
+      args.N = din;
+      args.splits = splits;
+      args.per = ((K + 4LL * splits - 1) / (4LL * splits) + kF32Rows - 1) / kF32Rows * kF32Rows;
+      args.plane_rows = prows;
+      args.plane_ld = pld;
+      args.partial = partial;
+      args.ep = ep;
+      const dim3 grid((unsigned)blocks), block(kThreads);
+      if (T == 1)
+        hipLaunchKernelGGL((clipped_sum_f32_kernel<In, true>), grid, block, 0, s, args);
+      else
+        hipLaunchKernelGGL((clipped_sum_f32_kernel<In, false>), grid, block, 0, s, args);
+    };
+    if (dtype == DPC_BF16)
+      run((const uint16_t*)A, (const uint16_t*)G);
     else
-      hipLaunchKernelGGL(clipped_sum_f32_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, s,
-                         args);
-    DPC_HIP_CHECK(hipGetLastError());
-    const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
-    hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, s, (const float*)args.partial, splits, args.plane_rows,
-                       args.plane_ld, ep);
+      run((const float*)A, (const float*)G);
+    if (splits > 1) {
+      DPC_HIP_CHECK(hipGetLastError());
+      const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
+      hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
+                         dim3(kThreads), 0, s, (const float*)partial, splits, prows, pld, ep);
+    }
   } else {
     int splits = generic_splits(B, T, din, dout);
     const size_t need = bias_ws_bytes(dout) + (size_t)splits * dout * (size_t)din * sizeof(float);

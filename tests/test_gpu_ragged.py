@@ -41,7 +41,10 @@ def _rel(got, want):
 # rows of A, of G and of both, odd (value by value) and even output rows.
 @pytest.mark.parametrize("B,T,din,dout", [
     (3, 2, 16, 8), (1, 33, 8, 264), (2, 63, 64, 72), (5, 65, 264, 256), (24, 97, 256, 520),
-    (3, 64, 15, 24), (4, 100, 257, 1001), (2, 128, 1030, 9), (16, 130, 259, 250), (1, 7, 1, 3)])
+    (3, 64, 15, 24), (4, 100, 257, 1001), (2, 128, 1030, 9), (16, 130, 259, 250), (1, 7, 1, 3),
+    # 1.5 GFLOP and more (below, layers on their own take the fp32 MFMA kernel): ragged steps,
+    # padded A, G and both, T % 64 == 0 with padding, many K slices
+    (24, 97, 520, 640), (16, 100, 1023, 511), (16, 64, 1000, 801), (100, 130, 248, 257)])
 @pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
 def test_clipped_sum_ragged(dev, B, T, din, dout, out):
     """fp32 sums of exact bf16 products: K = B T addends of one rounding each
@@ -52,7 +55,11 @@ def test_clipped_sum_ragged(dev, B, T, din, dout, out):
     cf = _factors(dev, A_d, G_d)
     w, _ = ops.clipped_sum(A_d, G_d, cf.scale[0], plan=cf.plan[0], out_dtype=out)
     want = _exact(A, G, cf.scale[0].cpu().double())
-    assert _rel(w.cpu(), want) < (1e-5 if out == torch.float32 else 2.0**-8)
+    tol = 1e-5 if out == torch.float32 else 2.0**-8
+    assert _rel(w.cpu(), want) < tol
+    if din % 8 == 0 and dout % 8 == 0:  # the bf16 kernel at any size
+        m, = ops.clipped_sum_multi([A_d], [G_d], cf.scale[0], plan=cf.plan[0], out_dtype=out)
+        assert _rel(m.cpu(), want) < tol
 
 
 @pytest.mark.parametrize("T,din", [(65, 264), (100, 33)])
@@ -70,10 +77,20 @@ def test_clipped_sum_ragged_skips_a_nonfinite_neighbour(dev, T, din):
     scale = cf.scale[0].cpu().double()
     assert scale[1] == 0 and 0 < scale[2] < 2.0**-64
     keep = [0, 2, 3]
-    assert _rel(w.cpu(), _exact(A[keep], G[keep], scale[keep])) < 1e-5
+    want = _exact(A[keep], G[keep], scale[keep])
+    assert _rel(w.cpu(), want) < 1e-5
+    if din % 8 == 0:
+        # The bf16 kernel; an entry of the plan between its two lists is not read.
+        plan = cf.plan[0].clone()
+        words = plan.view(torch.int32)
+        assert words[:2].tolist() == [3, 2]
+        words[4 + 2] = 1 << 28
+        m, = ops.clipped_sum_multi([A_d], [G_d], cf.scale[0], plan=plan, out_dtype=torch.float32)
+        assert _rel(m.cpu(), want) < 1e-5
 
 
-@pytest.mark.parametrize("din,dout", [(264, 72), (33, 17)])
+# fp32 MFMA kernel, even and odd rows; the bf16 kernel with and without padding.
+@pytest.mark.parametrize("din,dout", [(264, 72), (33, 17), (3000, 1200), (2999, 1201)])
 def test_clipped_sum_ragged_noise_matches_add_noise(dev, din, dout):
     A, G = _operands(3, 70, din, dout, 9)
     A_d, G_d = A.to(dev), G.to(dev)
