@@ -1008,8 +1008,22 @@ struct SplitTail {
   int32_t* ex_done;  // [B]: sets (of all layers) written per example
   double* sqnorm;
   double* sqerr;
+  const double* bias;  // nullable: [B, n_slots] squared norms (gram_add_bias)
+  int n_slots;
   ClipJob job;
 };
+
+// A wave adds example ex's bias norm (the sum of its n_slots words, in a fixed
+// order) to its squared norm, and that norm's error bound, 2^-21 relative (the
+// fp64 sum of exact squares and the fp32 product scale * column of the clipped
+// sum).
+__device__ __forceinline__ void gram_add_bias(const double* bias, int n_slots, int ex, double& v,
+                                              double& ev) {
+  const int lane = threadIdx.x & 63;
+  const double t = wave_sum_all_f64(lane < n_slots ? bias[(size_t)ex * n_slots + lane] : 0.0);
+  v = v + t;
+  ev = ev + t * 0x1.0p-21;
+}
 
 __device__ __forceinline__ double gram_bound_wave(const double* rec, int nt, double* sum);
 
@@ -1076,6 +1090,7 @@ __device__ void split_tail(const SplitTail& tail, const double* __restrict__ rec
       v = L == 0 ? sm : v + sm;
       ev = L == 0 ? e : ev + e;
     }
+    if (tail.bias) gram_add_bias(tail.bias, tail.n_slots, ex, v, ev);
     if (lane == 0) {
       const ClipExample e = clip_example_eval(v, ev, tail.sqerr != nullptr, B, tail.job);
       // The flags replace the example's set count; they are at memory before
@@ -1995,38 +2010,67 @@ __device__ __forceinline__ double gram_bound_wave(const double* rec, int nt, dou
   return err * (1.0 + 0x1.0p-40);
 }
 
+// One wave folds example b's record inner products (+ the bias term) into v
+// and its error bounds into ev, added to the caller's (accumulate) values.
+__device__ __forceinline__ void gram_finish_example(const double* records, int B, int nt,
+                                                    int nlayers, bool accumulate,
+                                                    const double* bias, int n_slots, int b,
+                                                    double& v, double& ev) {
+  const size_t np = (size_t)nt * (nt + 1) / 2;
+  // Layers' records one after the other (B examples each), added in layer
+  // order as consecutive accumulating calls would.
+  for (int L = 0; L < nlayers; ++L) {
+    double s;
+    const double e = gram_bound_wave(
+        records + ((size_t)L * B + (size_t)b) * np * DPC_GRAM_REC_WORDS, nt, &s);
+    const bool first = L == 0 && !accumulate;
+    v = first ? s : v + s;
+    ev = first ? e : ev + e;
+  }
+  if (bias) gram_add_bias(bias, n_slots, b, v, ev);
+}
+
 // Dense finish, one wave per example: sqnorm[b] (+)= the fold of example b's
 // record inner products (+ the bias term), sqerr[b] (+)= its error bound (+
-// the bias term's).  bias (nullable): [B, n_slots] squared norms; their error
-// bound is 2^-21 relative (the fp64 sum of exact squares and the fp32 product
-// scale * column of the clipped sum).
+// the bias term's).  bias (nullable): [B, n_slots] squared norms.
 __global__ void __launch_bounds__(kGramThreads)
 gram_finish_kernel(const double* __restrict__ records, int B, int nt, int nlayers,
                    int accumulate, const double* __restrict__ bias, int n_slots,
                    double* __restrict__ sqnorm, double* __restrict__ sqerr) {
   const int b = blockIdx.x * (kGramThreads / 64) + (int)(threadIdx.x >> 6);
   if (b >= B) return;
-  const size_t np = (size_t)nt * (nt + 1) / 2;
-  // Layers' records one after the other (B examples each), added in layer
-  // order as consecutive accumulating calls would.
-  double v = 0.0, ev = 0.0;
-  for (int L = 0; L < nlayers; ++L) {
-    double s;
-    const double e = gram_bound_wave(
-        records + ((size_t)L * B + (size_t)b) * np * DPC_GRAM_REC_WORDS, nt, &s);
-    const bool first = L == 0 && !accumulate;
-    v = first ? s : (L == 0 ? sqnorm[b] : v) + s;
-    ev = first ? e : (L == 0 && sqerr ? sqerr[b] : ev) + e;
-  }
-  if (bias) {
-    const int lane = threadIdx.x & 63;
-    const double t = wave_sum_all_f64(lane < n_slots ? bias[(size_t)b * n_slots + lane] : 0.0);
-    v = v + t;
-    ev = ev + t * 0x1.0p-21;
-  }
+  double v = accumulate ? sqnorm[b] : 0.0, ev = accumulate && sqerr ? sqerr[b] : 0.0;
+  gram_finish_example(records, B, nt, nlayers, accumulate != 0, bias, n_slots, b, v, ev);
   if ((threadIdx.x & 63) != 0) return;
   sqnorm[b] = v;
   if (sqerr) sqerr[b] = ev;
+}
+
+// The finish and the clip factors of a small batch by one workgroup, the same
+// bits as the two launches (4.3 us against 3.4 + 3.3 and the gap between
+// them).  Up to two examples a wave: more would wait for each other's folds
+// longer than that.
+constexpr int kFinishClipThreads = 1024;
+constexpr int kFinishClipMaxB = 2 * kFinishClipThreads / 64;
+
+__global__ void __launch_bounds__(kFinishClipThreads)
+gram_finish_clip_kernel(const double* __restrict__ records, int B, int nt,
+                        const double* __restrict__ bias, int n_slots, double* __restrict__ sqnorm,
+                        double* __restrict__ sqerr, const ClipJob job) {
+  __shared__ double sq[kFinishClipMaxB], err[kFinishClipMaxB];
+  __shared__ int shm[clip_block_lds_ints(kFinishClipThreads / 64)];
+  for (int b = threadIdx.x >> 6; b < B; b += kFinishClipThreads / 64) {
+    double v = 0.0, ev = 0.0;
+    gram_finish_example(records, B, nt, 1, false, bias, n_slots, b, v, ev);
+    if ((threadIdx.x & 63) == 0) {
+      sq[b] = v;
+      err[b] = ev;
+      sqnorm[b] = v;
+      if (sqerr) sqerr[b] = ev;
+    }
+  }
+  __syncthreads();
+  clip_factors_block(sq, sqerr ? err : nullptr, B, job, shm);
 }
 
 // Grouped finish, one wave per segment: seg_sq[v] / seg_err[v] (nullable)
@@ -2156,9 +2200,27 @@ extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
   return gram_bias_slots_offset(B, T) + (size_t)B * kBiasSlots * sizeof(double);
 }
 
-extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int dout,
-                                int dtype, int with_bias, int accumulate, double* sqnorm,
-                                double* sqerr, void* ws, size_t ws_bytes, void* stream) {
+// The column norms of a bias into `out` ([B, n_slots] words).
+static int launch_bias_sqnorm(const void* G, int B, int T, int dout, int dtype, int n_slots,
+                              double* out, hipStream_t s) {
+  const dim3 grid(n_slots, B);
+  if (dtype == DPC_BF16) {
+    hipLaunchKernelGGL(bias_sqnorm_kernel<uint16_t>, grid, dim3(kBiasThreads), 0, s,
+                       (const uint16_t*)G, T, dout, n_slots, out);
+  } else {
+    hipLaunchKernelGGL(bias_sqnorm_kernel<float>, grid, dim3(kBiasThreads), 0, s, (const float*)G, T,
+                       dout, n_slots, out);
+  }
+  DPC_HIP_CHECK(hipGetLastError());
+  return DPC_OK;
+}
+
+// dpc_gram_sqnorms; with `clip` (accumulate == 0, B <= kFinishClipMaxB) the
+// last launch computes the clip factors too.
+static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din, int dout,
+                            int dtype, int with_bias, int accumulate, double* sqnorm,
+                            double* sqerr, const ClipJob* clip, void* ws, size_t ws_bytes,
+                            void* stream) {
   if (B < 0 || T <= 0 || din <= 0 || dout <= 0) return DPC_EINVAL;
   if (B == 0) return DPC_OK;
   if (!A || !G || !sqnorm || !ws) return DPC_EINVAL;
@@ -2229,21 +2291,27 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
     } else {
       bias = records + (size_t)nt * (nt + 1) / 2 * (size_t)B * DPC_GRAM_REC_WORDS;
     }
-    const dim3 grid(n_slots, B);
-    if (dtype == DPC_BF16) {
-      hipLaunchKernelGGL(bias_sqnorm_kernel<uint16_t>, grid, dim3(kBiasThreads), 0, s,
-                         (const uint16_t*)G, T, dout, n_slots, bias);
-    } else {
-      hipLaunchKernelGGL(bias_sqnorm_kernel<float>, grid, dim3(kBiasThreads), 0, s,
-                         (const float*)G, T, dout, n_slots, bias);
-    }
-    DPC_HIP_CHECK(hipGetLastError());
+    const int r = launch_bias_sqnorm(G, B, T, dout, dtype, n_slots, bias, s);
+    if (r != DPC_OK) return r;
   }
-  hipLaunchKernelGGL(gram_finish_kernel, dim3(ceil_div(B, kGramThreads / 64)), dim3(kGramThreads), 0,
-                     s, (const double*)records, B, nt, 1, accumulate, (const double*)bias, n_slots,
-                     sqnorm, sqerr);
+  if (clip) {
+    hipLaunchKernelGGL(gram_finish_clip_kernel, dim3(1), dim3(kFinishClipThreads), 0, s,
+                       (const double*)records, B, nt, (const double*)bias, n_slots, sqnorm, sqerr,
+                       *clip);
+  } else {
+    hipLaunchKernelGGL(gram_finish_kernel, dim3(ceil_div(B, kGramThreads / 64)),
+                       dim3(kGramThreads), 0, s, (const double*)records, B, nt, 1, accumulate,
+                       (const double*)bias, n_slots, sqnorm, sqerr);
+  }
   DPC_HIP_CHECK(hipGetLastError());
   return DPC_OK;
+}
+
+extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int dout,
+                                int dtype, int with_bias, int accumulate, double* sqnorm,
+                                double* sqerr, void* ws, size_t ws_bytes, void* stream) {
+  return gram_sqnorms_run(A, G, B, T, din, dout, dtype, with_bias, accumulate, sqnorm, sqerr,
+                          nullptr, ws, ws_bytes, stream);
 }
 
 // Workspace of dpc_grouped_gram_sqnorms: the records, the split kernel's
@@ -2529,12 +2597,12 @@ extern "C" int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* c
 }
 
 namespace {
-bool gram_clip_one_launch(int B, int T, int din, int dout, int dtype, int with_bias) {
+bool gram_clip_one_launch(int B, int T, int din, int dout, int dtype) {
   const size_t dmax = (size_t)(din > dout ? din : dout);
   // The tail's LDS holds one example's records, then B flag words.
   const size_t nt = (size_t)ceil_div(T, kGramTile), np = nt * (nt + 1) / 2;
   const size_t lds_doubles = (size_t)(4 * 3 * kGTileBytes) / sizeof(double);
-  return dtype == DPC_BF16 && !with_bias && din % 8 == 0 && dout % 8 == 0 && split_shape(T) &&
+  return dtype == DPC_BF16 && din % 8 == 0 && dout % 8 == 0 && split_shape(T) &&
          B <= kSplitTailMaxB && ((size_t)T + kGramTile) * dmax * 2 < ((size_t)1 << 31) &&
          np * DPC_GRAM_REC_WORDS <= lds_doubles && (size_t)B <= 2 * lds_doubles;
 }
@@ -2571,12 +2639,19 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
                              count_threshold, scale, scale64, norms_out, nclipped, plan, nonfinite,
                              &job);
   if (r != DPC_OK) return r;
-  if (!gram_clip_one_launch(B, T, din, dout, dtype, with_bias)) {
-    // The norms and the clip factors as separate launches (the counters
-    // are not used).
-    r = dpc_gram_sqnorms(A, G, B, T, din, dout, dtype, with_bias, 0, sqnorm, sqerr, ws, ws_bytes,
-                         stream);
-    if (r != DPC_OK) return r;
+  // A bias goes with the one launch (it saves the ticket reset, the finish and
+  // the clip pass: [24, 197, 768 x 3072] 120 -> 112 us in all) when the
+  // workspace holds its column norms and, as it did not need them before, when
+  // there are counters.
+  const bool bias_fits = !with_bias || (ws_bytes >= dpc_gram_workspace_bytes(B, T) && counters &&
+                                        counter_bytes >= dpc_gram_clip_counter_bytes(B, T));
+  if (!gram_clip_one_launch(B, T, din, dout, dtype) || !bias_fits) {
+    // The norms, then (in their last launch, for a small batch) the clip
+    // factors; the counters are not used.
+    const bool together = B <= kFinishClipMaxB;
+    r = gram_sqnorms_run(A, G, B, T, din, dout, dtype, with_bias, 0, sqnorm, sqerr,
+                         together ? &job : nullptr, ws, ws_bytes, stream);
+    if (r != DPC_OK || together) return r;
     return dpc_clip_factors(sqnorm, sqerr, B, C, kind, gamma, guard_rel, guard_abs, guard_mult,
                             n_guards, count_threshold, scale, scale64, norms_out, nclipped, plan,
                             nonfinite, stream);
@@ -2610,7 +2685,16 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   tail.done = tail.ex_done + B;
   tail.sqnorm = sqnorm;
   tail.sqerr = sqerr;
+  tail.bias = nullptr;
+  tail.n_slots = 0;
   tail.job = job;
+  if (with_bias) {
+    tail.n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
+    double* slots = (double*)(base + gram_bias_slots_offset(B, T));
+    tail.bias = slots;
+    r = launch_bias_sqnorm(G, B, T, dout, dtype, tail.n_slots, slots, s);
+    if (r != DPC_OK) return r;
+  }
   hipLaunchKernelGGL(gram_split_bf16_kernel, dim3(padded), dim3(512), 0, s, lay, B, T, npairs,
                      nsets, nblocks, records, counters, xbuf, tail);
   DPC_HIP_CHECK(hipGetLastError());

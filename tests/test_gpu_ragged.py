@@ -263,3 +263,29 @@ def test_leaves_unaligned_match_oracle(dev, dtype, B, out):
         post += (s.reshape(B, -1) ** 2).sum(dim=1)
     # fp32 sums of 512 squares per wave (fp64 for fp16), then fp64.
     torch.testing.assert_close(res.post_sq.cpu().double(), post, rtol=1e-4 * 2**-4, atol=0)
+
+
+# Norms and clip factors: finished together for up to 32 examples (one and two
+# a wave), by two launches past that; a bias inside the one-launch path (an even
+# number of 128-row blocks) and beside it; call after call on one counter buffer.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T", [(1, 24), (16, 40), (17, 70), (32, 33), (33, 20), (9, 200), (40, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_clip_factors_with_the_norms(dev, dtype, B, T, bias):
+    A, G = (x.to(dev, dtype) for x in _operands(B, T, 64, 264, B + T))
+    G[B // 2, 0, 0] = float("nan")
+    guards = [guard_for_linear(dtype, 64, 264, bias)]
+    kw = dict(with_bias=bias)
+    for _ in range(2):
+        sq, err, cf = ops.gram_clip_factors(A, G, 1.0, guards, count_threshold=1.0, **kw)
+        wsq, werr = ops.gram_sqnorms(A, G, return_error=True, **kw)
+        want = ops.clip_factors(wsq, 1.0, guards, err=werr, count_threshold=1.0)
+        for x, y in ((sq, wsq), (err, werr), (cf.scale, want.scale), (cf.norms, want.norms),
+                     (cf.nclipped, want.nclipped)):
+            assert torch.equal(torch.nan_to_num(x, nan=-1.0), torch.nan_to_num(y, nan=-1.0))
+        n = int(cf.plan[0].view(torch.int32)[0])
+        assert n == B - 1
+        assert torch.equal(cf.plan[0].view(torch.int32)[:4 + n][:2],
+                           want.plan[0].view(torch.int32)[:2])
+        assert torch.equal(cf.plan[0].view(torch.int32)[4:4 + n],
+                           want.plan[0].view(torch.int32)[4:4 + n])
