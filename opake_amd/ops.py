@@ -8,7 +8,7 @@ None of them synchronises the host.
 from __future__ import annotations
 
 import ctypes
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import torch
 
@@ -478,9 +478,9 @@ def clipped_sum_multi(
     bf16 MFMA path the layers' output tiles share launches.  ``noises[i]``:
     layer i's noise (None: none); the specs must share one mode and seed.
     Returns one [dout, din] tensor per layer.  When every layer takes the
-    MFMA path (bf16, T > 1, widths % 8 == 0, a plan) each result equals
-    its own ``clipped_sum`` call without a split-K workspace; otherwise the
-    layers run as their own ``clipped_sum`` calls."""
+    MFMA path (bf16, T > 1, widths % 8 == 0, a plan) and their tiles fill
+    launches, each result equals its own ``clipped_sum`` call without a split-K
+    workspace; otherwise the layers run as their own ``clipped_sum`` calls."""
     n = len(A_list)
     if n == 0 or len(G_list) != n:
         raise ConfigurationError("expected matching, non-empty lists of A and G")
@@ -509,6 +509,20 @@ def clipped_sum_multi(
     mfma = plan is not None and B > 0 and dtype == torch.bfloat16 and T > 1 and all(
         A.shape[2] % 8 == 0 and G.shape[2] % 8 == 0
         and B * T * max(A.shape[2], G.shape[2]) * 2 < limit for A, G in zip(A_list, G_list))
+    # Layers of few output tiles (256 x 256) and a long K leave most CUs idle for
+    # the whole of it in a shared launch, which does not split K. Their own calls
+    # do, for some 25 us more a layer; a K step is about 1.6 us. A transformer
+    # block's seven layers, norms and sums: width 256 at [24, 900] (360 steps)
+    # 830 -> 490 us, width 512 at [24, 1000] (384) 989 -> 700 us; at the line,
+    # 82 tiles at [23, 640] (230) 614 -> 549 us and 96 tiles at [112, 100] (224)
+    # 628 -> 558 us; width 384 at [22, 192] (66) would lose, 261 -> 319 us, and
+    # stays shared.
+    tiles = sum(-(-A.shape[2] // 256) * -(-G.shape[2] // 256) for A, G in zip(A_list, G_list))
+    if mfma and n > 1 and tiles <= 96 and B * -(-T // 64) >= 32 * n:
+        mfma = False
+        noises = [None if sp is None or sp.sigma == 0.0
+                  else replace(sp, noise=None if sp.noise is None else _contig(sp.noise))
+                  for sp in noises]
     if not mfma:
         return [clipped_sum(A, G, scale, plan=plan, normalize_by=normalize_by, noise=sp,
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]

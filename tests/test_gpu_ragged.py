@@ -289,3 +289,20 @@ def test_clip_factors_with_the_norms(dev, dtype, B, T, bias):
                            want.plan[0].view(torch.int32)[:2])
         assert torch.equal(cf.plan[0].view(torch.int32)[4:4 + n],
                            want.plan[0].view(torch.int32)[4:4 + n])
+
+
+def test_clipped_sum_multi_few_tiles_long_k(dev):
+    """Few output tiles and a long K: the layers' own split-K calls, with noise
+    tensors of any strides, noise specs without noise, and none at all."""
+    dims = [(64, 264), (520, 256), (64, 72)]
+    pairs = [_operands(40, 130, din, dout, din + dout) for din, dout in dims]
+    As, Gs = [a.to(dev) for a, _ in pairs], [g.to(dev) for _, g in pairs]
+    cf = _factors(dev, As[0], Gs[0])
+    z = torch.randn(64, 264, device=dev).t()
+    noises = [ops.NoiseSpec(0.5, ops.nat.NOISE_INJECTED, noise=z),
+              ops.NoiseSpec(0.0, ops.nat.NOISE_INJECTED), None]
+    kw = dict(plan=cf.plan[0], out_dtype=torch.float32)
+    got = ops.clipped_sum_multi(As, Gs, cf.scale[0], noises=noises, **kw)
+    for w, a, g, pair, noise in zip(got, As, Gs, pairs, (0.5 * z, 0, 0)):
+        assert torch.equal(w, ops.clipped_sum(a, g, cf.scale[0], **kw)[0] + noise)
+        assert _rel((w - noise).cpu(), _exact(*pair, cf.scale[0].cpu().double())) < 1e-5
