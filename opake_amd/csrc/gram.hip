@@ -2269,16 +2269,31 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
     hipLaunchKernelGGL(gram_mfma_bf16_kernel, dim3(padded), dim3(512), 0, s, (const uint16_t*)A,
                        (const uint16_t*)G, T, din, dout, npairs, items, nblocks, records);
   } else {
-    const int subs = full_ws ? 1 : kGenTile / kF64Rows;
+    // A launch holds less than 2^32 threads: more tile pairs go out as several
+    // launches of whole examples, an example of more than that in 64-row tiles.
+    constexpr size_t kMaxBlocks = ((size_t)1 << 32) / kF64Threads - 2 * kXcds;
+    const size_t fine = ceil_div(T, kF64Rows);
+    const bool coarse = !full_ws || fine * (fine + 1) / 2 > kMaxBlocks;
+    const int subs = coarse ? kGenTile / kF64Rows : 1;
     nt = ceil_div(T, kF64Rows * subs);
-    const int npairs = nt * (nt + 1) / 2, nblocks = npairs * B;
-    const dim3 grid(ceil_div(nblocks, kXcds) * kXcds), block(kF64Threads);
-    if (dtype == DPC_BF16) {
-      hipLaunchKernelGGL(gram_f64_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)A,
-                         (const uint16_t*)G, T, din, dout, npairs, nblocks, subs, records);
-    } else {
-      hipLaunchKernelGGL(gram_f64_kernel<float>, grid, block, 0, s, (const float*)A,
-                         (const float*)G, T, din, dout, npairs, nblocks, subs, records);
+    const size_t np = (size_t)nt * (nt + 1) / 2;
+    if (np > kMaxBlocks) return DPC_ENOTSUP;
+    const int npairs = (int)np;
+    const int per_launch = (int)(kMaxBlocks / np < (size_t)B ? kMaxBlocks / np : (size_t)B);
+    for (int e0 = 0; e0 < B; e0 += per_launch) {
+      const int nblocks = npairs * min(per_launch, B - e0);
+      const dim3 grid(ceil_div(nblocks, kXcds) * kXcds), block(kF64Threads);
+      const size_t row0 = (size_t)e0 * T;
+      double* rec = records + (size_t)e0 * np * DPC_GRAM_REC_WORDS;
+      if (dtype == DPC_BF16) {
+        hipLaunchKernelGGL(gram_f64_kernel<uint16_t>, grid, block, 0, s,
+                           (const uint16_t*)A + row0 * din, (const uint16_t*)G + row0 * dout, T,
+                           din, dout, npairs, nblocks, subs, rec);
+      } else {
+        hipLaunchKernelGGL(gram_f64_kernel<float>, grid, block, 0, s, (const float*)A + row0 * din,
+                           (const float*)G + row0 * dout, T, din, dout, npairs, nblocks, subs, rec);
+      }
+      DPC_HIP_CHECK(hipGetLastError());
     }
   }
   DPC_HIP_CHECK(hipGetLastError());

@@ -157,13 +157,14 @@ def test_bias_norm_and_sum(dev, dtype, B, T, dout):
     assert ((b.cpu().double() - want_b).abs() <= bound).all()
 
 
-# The fp64 Gram path: 32-row tiles (few items) and 64-row ones (1024 items and
-# more), one, two and several tiles with ragged last ones, depths around the
-# 32-deep chunks, rows that 16-byte loads do not take, din != dout both ways.
+# The fp64 Gram path: one, two and several 32-row tiles with ragged last ones,
+# depths around the 32-deep chunks, rows that 16-byte loads do not take, din !=
+# dout both ways; 16.8 million tile pairs, more than one launch holds (2^32 threads).
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,din,dout", [
     (2, 2, 4, 8), (3, 31, 33, 9), (2, 32, 32, 31), (4, 65, 100, 36), (1, 130, 7, 260),
-    (2, 257, 64, 65), (1024, 40, 12, 20), (110, 200, 33, 68)])
+    (2, 257, 64, 65), (1024, 40, 12, 20), (110, 200, 33, 68),
+    (2040, 4096, 4, 4)])
 def test_gram_f64(dev, dtype, B, T, din, dout):
     """Exact products in fp64: the error is within the kernel's own bound, and
     far below what fp32 sums would leave (2^-24)."""
