@@ -231,8 +231,9 @@ int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, i
  * z comes from `noise` (float32 [dout, din], mode INJECTED; bit-exact with a
  * host-drawn tensor) or from the Philox stream (mode PHILOX) keyed by
  * (seed, leaf_id).  `plan` is the dpc_clip_factors plan built from the same
- * `scale` (nullable: the generic kernel then scans every example).  On the
- * bf16 MFMA path (T % 64 == 0, din and dout multiples of 8) the products of
+ * `scale` (nullable: bf16 layers of 1.5 GFLOP and more then take the generic kernel,
+ * which scans every example).  On the bf16 MFMA path (T > 1; widths that are
+ * not multiples of 8 are copied into padded rows in ws) the products of
  * the given bf16 values are summed in fp32 and each example's scale is
  * applied to the fp32 accumulators (the plan's first list); examples of the
  * plan's second list have G multiplied by the power of two of their scale
@@ -240,9 +241,10 @@ int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, i
  * with_bias, bias_out[m] = same recipe over
  * sum_i scale[i] * sum_t G[i, t, m], its noise keyed by (seed, bias_leaf_id)
  * under the [dout, 1] view.  ws (dpc_clipped_sum_workspace_bytes) holds the
- * bias partials and, on the MFMA path for layers of fewer than 192 256 x 256
- * output tiles, the fp32 K-slices of a split-K launch (summed in a fixed
- * order); with a smaller ws (or none, without bias) the launch is one pass.
+ * bias partials, the padded operand copies and, for layers of few output
+ * tiles, the fp32 K-slices of a split-K launch (summed in a fixed order); with
+ * a smaller ws (or none, without bias) the layer takes one pass or the generic
+ * kernel.
  * -------------------------------------------------------------------------*/
 size_t dpc_clipped_sum_workspace_bytes(int B, int T, int din, int dout, int dtype);
 int dpc_clipped_sum(const void* A, const void* G, const float* scale, const void* plan, int B,
