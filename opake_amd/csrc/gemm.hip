@@ -1140,13 +1140,47 @@ void launch_fast(dim3 grid, hipStream_t s, const FastArgs& args) {
                        args);
 }
 
+// A bias's finish: adds the nsplit partial sums of each column in order and
+// applies the epilogue, a pair of columns per thread; `blocks` workgroups (0:
+// no bias).
+struct BiasFinish {
+  const float* partial;
+  int nsplit;
+  int blocks;
+  Epilogue ep;
+};
+
+__device__ __forceinline__ void bias_finish_block(const BiasFinish& bias, int block) {
+  // Rows are handled in even/odd pairs so the Philox pairing matches the
+  // [M, 1] view of the bias leaf.
+  const int M = bias.ep.M;
+  const int m = 2 * (block * kThreads + (int)threadIdx.x);
+  if (m >= M) return;
+  const int m1 = min(m + 1, M - 1);
+  float v0 = 0.f, v1 = 0.f;
+#pragma unroll 8
+  for (int s = 0; s < bias.nsplit; ++s) {
+    v0 += bias.partial[(size_t)s * M + m];
+    v1 += bias.partial[(size_t)s * M + m1];
+  }
+  emit_pair(bias.ep, m, 0, v0, v1);
+}
+
 // Split-K finish: out = epilogue(sum over splits of partial[split], in
 // order).  One thread per (row pair, column pair); a split's plane is rows x
-// ld values (rows >= M, ld >= N, both even).
+// ld values (rows >= M, ld >= N, both even).  The first workgroups finish the
+// layer's bias, which as a launch of its own took 3.9 us: [24, 197, 768 x 3072]
+// with a bias 111.9 -> 107.3 us in all, [16, 256, 1024 x 1024] fp32 166 -> 162.
 __global__ void __launch_bounds__(kThreads)
-split_reduce_kernel(const float* __restrict__ partial, int splits, int rows, int ld, Epilogue ep) {
+split_reduce_kernel(const float* __restrict__ partial, int splits, int rows, int ld, Epilogue ep,
+                    BiasFinish bias) {
+  const int block = (int)blockIdx.x - bias.blocks;
+  if (block < 0) {
+    bias_finish_block(bias, blockIdx.x);
+    return;
+  }
   const int half_n = (ep.N + 1) / 2;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long idx = (long long)block * blockDim.x + threadIdx.x;
   if (idx >= (long long)((ep.M + 1) / 2) * half_n) return;
   const int m = 2 * (int)(idx / half_n), n = 2 * (int)(idx % half_n);
   const size_t plane = (size_t)rows * ld;
@@ -1677,20 +1711,8 @@ bias_partial_cols_kernel(const In* __restrict__ G, const float* __restrict__ sca
     partial[(size_t)split * M + c0 + threadIdx.x] = acc;
 }
 
-__global__ void __launch_bounds__(kThreads)
-bias_finish_kernel(const float* __restrict__ partial, int nsplit, Epilogue ep) {
-  // Rows are handled in even/odd pairs so the Philox pairing matches the
-  // [M, 1] view of the bias leaf.
-  const int m = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-  if (m >= ep.M) return;
-  const int m1 = min(m + 1, ep.M - 1);
-  float v0 = 0.f, v1 = 0.f;
-#pragma unroll 8
-  for (int s = 0; s < nsplit; ++s) {
-    v0 += partial[(size_t)s * ep.M + m];
-    v1 += partial[(size_t)s * ep.M + m1];
-  }
-  emit_pair(ep, m, 0, v0, v1);
+__global__ void __launch_bounds__(kThreads) bias_finish_kernel(BiasFinish bias) {
+  bias_finish_block(bias, blockIdx.x);
 }
 
 // Grouped generic path (float32, or bf16 of any shape): problem blockIdx.z,
@@ -1991,6 +2013,43 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
   ep.out_bf16 = out_dtype == DPC_BF16;
   ep.out = out;
 
+  // The bias's partial sums; its finish goes with the split-K sum's launch, if
+  // there is one.
+  BiasFinish bias = {nullptr, 0, 0, ep};
+  if (with_bias) {
+    const int nsplit = B > 0 ? min(B, kBiasSplits) : 1;
+    float* partial = (float*)ws;
+    dim3 grid(ceil_div(dout, kThreads), nsplit);
+    if (B > 0 && T >= kBiasColsMinT) {
+      const dim3 cols(ceil_div(dout, kBiasCols), nsplit);
+      if (dtype == DPC_BF16) {
+        hipLaunchKernelGGL(bias_partial_cols_kernel<uint16_t>, cols, dim3(kBiasThreads), 0, s,
+                           (const uint16_t*)G, scale, B, T, dout, nsplit, partial);
+      } else {
+        hipLaunchKernelGGL(bias_partial_cols_kernel<float>, cols, dim3(kBiasThreads), 0, s,
+                           (const float*)G, scale, B, T, dout, nsplit, partial);
+      }
+      DPC_HIP_CHECK(hipGetLastError());
+    } else if (B > 0) {
+      if (dtype == DPC_BF16) {
+        hipLaunchKernelGGL(bias_partial_kernel<uint16_t>, grid, dim3(kThreads), 0, s,
+                           (const uint16_t*)G, scale, B, T, dout, nsplit, partial);
+      } else {
+        hipLaunchKernelGGL(bias_partial_kernel<float>, grid, dim3(kThreads), 0, s,
+                           (const float*)G, scale, B, T, dout, nsplit, partial);
+      }
+      DPC_HIP_CHECK(hipGetLastError());
+    }
+    bias.partial = partial;
+    bias.nsplit = B > 0 ? nsplit : 0;
+    bias.blocks = ceil_div(ceil_div(dout, 2), kThreads);
+    bias.ep.M = dout;
+    bias.ep.N = 1;
+    bias.ep.noise = bias_noise;
+    bias.ep.leaf = bias_leaf_id;
+    bias.ep.out = bias_out;
+  }
+
   // Buffer offsets are 32-bit: each operand must stay below 2 GiB.  Operands
   // whose rows are not 16-byte aligned are copied into padded rows first; a
   // caller without the workspace for it gets the generic kernel.
@@ -2035,9 +2094,11 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
     if (args.partial) {
       DPC_HIP_CHECK(hipGetLastError());
       const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
-      hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
+      hipLaunchKernelGGL(split_reduce_kernel,
+                         dim3((unsigned)(bias.blocks + (quads + kThreads - 1) / kThreads)),
                          dim3(kThreads), 0, s, (const float*)args.partial, splits, args.ldg,
-                         args.lda, ep);
+                         args.lda, ep, bias);
+      bias.blocks = 0;
     }
   } else if (f32) {
     const int splits = f32_splits(B, T, din, dout);
@@ -2076,8 +2137,11 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
     if (splits > 1) {
       DPC_HIP_CHECK(hipGetLastError());
       const long long quads = (long long)ceil_div(dout, 2) * ceil_div(din, 2);
-      hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + kThreads - 1) / kThreads)),
-                         dim3(kThreads), 0, s, (const float*)partial, splits, prows, pld, ep);
+      hipLaunchKernelGGL(split_reduce_kernel,
+                         dim3((unsigned)(bias.blocks + (quads + kThreads - 1) / kThreads)),
+                         dim3(kThreads), 0, s, (const float*)partial, splits, prows, pld, ep,
+                         bias);
+      bias.blocks = 0;
     }
   } else {
     int splits = generic_splits(B, T, din, dout);
@@ -2098,44 +2162,17 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
     if (splits > 1) {
       DPC_HIP_CHECK(hipGetLastError());
       const long long pairs = (long long)(dout / 2) * (din / 2);
-      hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((pairs + kThreads - 1) / kThreads)),
-                         dim3(kThreads), 0, s, (const float*)partial, splits, dout, din, ep);
+      hipLaunchKernelGGL(split_reduce_kernel,
+                         dim3((unsigned)(bias.blocks + (pairs + kThreads - 1) / kThreads)),
+                         dim3(kThreads), 0, s, (const float*)partial, splits, dout, din, ep,
+                         bias);
+      bias.blocks = 0;
     }
   }
   DPC_HIP_CHECK(hipGetLastError());
 
-  if (with_bias) {
-    const int nsplit = B > 0 ? min(B, kBiasSplits) : 1;
-    float* partial = (float*)ws;
-    dim3 grid(ceil_div(dout, kThreads), nsplit);
-    if (B > 0 && T >= kBiasColsMinT) {
-      const dim3 cols(ceil_div(dout, kBiasCols), nsplit);
-      if (dtype == DPC_BF16) {
-        hipLaunchKernelGGL(bias_partial_cols_kernel<uint16_t>, cols, dim3(kBiasThreads), 0, s,
-                           (const uint16_t*)G, scale, B, T, dout, nsplit, partial);
-      } else {
-        hipLaunchKernelGGL(bias_partial_cols_kernel<float>, cols, dim3(kBiasThreads), 0, s,
-                           (const float*)G, scale, B, T, dout, nsplit, partial);
-      }
-      DPC_HIP_CHECK(hipGetLastError());
-    } else if (B > 0) {
-      if (dtype == DPC_BF16) {
-        hipLaunchKernelGGL(bias_partial_kernel<uint16_t>, grid, dim3(kThreads), 0, s,
-                           (const uint16_t*)G, scale, B, T, dout, nsplit, partial);
-      } else {
-        hipLaunchKernelGGL(bias_partial_kernel<float>, grid, dim3(kThreads), 0, s,
-                           (const float*)G, scale, B, T, dout, nsplit, partial);
-      }
-      DPC_HIP_CHECK(hipGetLastError());
-    }
-    Epilogue eb = ep;
-    eb.M = dout;
-    eb.N = 1;
-    eb.noise = bias_noise;
-    eb.leaf = bias_leaf_id;
-    eb.out = bias_out;
-    hipLaunchKernelGGL(bias_finish_kernel, dim3(ceil_div(ceil_div(dout, 2), kThreads)),
-                       dim3(kThreads), 0, s, (const float*)partial, B > 0 ? nsplit : 0, eb);
+  if (bias.blocks > 0) {
+    hipLaunchKernelGGL(bias_finish_kernel, dim3(bias.blocks), dim3(kThreads), 0, s, bias);
     DPC_HIP_CHECK(hipGetLastError());
   }
   return DPC_OK;

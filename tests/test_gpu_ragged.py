@@ -157,6 +157,29 @@ def test_bias_norm_and_sum(dev, dtype, B, T, dout):
     assert ((b.cpu().double() - want_b).abs() <= bound).all()
 
 
+# One workgroup of bias columns and several, an odd last column; the sums behind
+# them split over K (fp32 MFMA with din 16; bf16 MFMA with padded rows) and not.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,dout", [(40, 264), (40, 1001), (5, 513)])
+def test_bias_finish_with_the_split_sums(dev, dtype, T, dout):
+    """The bias finished in the split-K sum's launch and in one of its own: the
+    same bits, with noise and normalisation."""
+    g = torch.Generator().manual_seed(T + dout)
+    B, bias = 40, []
+    G = (torch.randn(B, T, dout, generator=g) * 0.01).to(dtype).to(dev)
+    sq = (4 * torch.rand(B, dtype=torch.float64, generator=g)).to(dev)
+    cf = ops.clip_factors(sq, 1.0, [guard_for_linear(dtype, 16, dout, True)], count_threshold=1.0)
+    scale, plan = cf.scale[0], cf.plan[0]
+    for din in (16, 1001, 8192):
+        A = torch.randn(B, T, din, generator=g).to(dtype).to(dev)
+        spec = ops.NoiseSpec(sigma=0.5, seed=77, leaf_id=3, bias_leaf_id=4)
+        _, b = ops.clipped_sum(A, G, scale, plan=plan, with_bias=True, noise=spec, normalize_by=2.0)
+        _, plain = ops.clipped_sum(A, G, scale, plan=plan, with_bias=True, normalize_by=2.0)
+        assert torch.equal(b, ops.add_noise(plain, 0.5, seed=77, leaf_id=4))
+        bias.append(b)
+    assert torch.equal(bias[0], bias[1]) and torch.equal(bias[0], bias[2])
+
+
 # The fp64 Gram path: one, two and several 32-row tiles with ragged last ones,
 # depths around the 32-deep chunks, rows that 16-byte loads do not take, din !=
 # dout both ways; 16.8 million tile pairs, more than one launch holds (2^32 threads).
