@@ -1945,24 +1945,32 @@ size_t split_bytes(int splits, int din, int dout) {
 }
 
 // dst[row] = src[row] (width elements) followed by zeros up to ld (a multiple
-// of 8); one thread per 16-byte chunk of dst.
+// of 8); one thread per 16-byte chunk of dst, read in one load at any element
+// alignment (global loads take it) except the row's last, which goes value by
+// value.  rows * ld / 8 is below 2^28 (fast_shape).
+// Bound by memory: [6144 x 1001] 5.9 us (4.2 TB/s) against 11.4 in 2-byte loads
+// with a 64-bit division.
+typedef u32x4_t u32x4_align2_t __attribute__((aligned(2)));
 __global__ void __launch_bounds__(kThreads)
-pad_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, long long rows,
-                int width, int ld) {
-  const int chunks = ld / 8;
-  const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
+pad_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, uint32_t rows,
+                uint32_t width, uint32_t ld) {
+  const uint32_t chunks = ld / 8;
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= rows * chunks) return;
-  const long long row = i / chunks;
-  const int c0 = (int)(i - row * chunks) * 8;
-  const uint16_t* p = src + row * width + c0;
+  const uint32_t row = i / chunks, c0 = (i - row * chunks) * 8;
+  const auto* p = global_ptr<const uint16_t>(src) + (size_t)row * width + c0;
   u32x4_t v;
+  if (c0 + 8 <= width) {
+    v = *(const __attribute__((address_space(1))) u32x4_align2_t*)p;
+  } else {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const uint32_t lo = c0 + 2 * k < width ? p[2 * k] : 0;
-    const uint32_t hi = c0 + 2 * k + 1 < width ? p[2 * k + 1] : 0;
-    v[k] = lo | (hi << 16);
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t lo = c0 + 2 * k < width ? p[2 * k] : 0;
+      const uint32_t hi = c0 + 2 * k + 1 < width ? p[2 * k + 1] : 0;
+      v[k] = lo | (hi << 16);
+    }
   }
-  *reinterpret_cast<u32x4_t*>(dst + i * 8) = v;
+  *reinterpret_cast<u32x4_t*>(dst + (size_t)i * 8) = v;
 }
 }  // namespace
 
@@ -2069,7 +2077,8 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
       uint16_t* dst = (uint16_t*)((uint8_t*)ws + at);
       const long long chunks = rows * (ld / 8);
       hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((chunks + kThreads - 1) / kThreads)),
-                         dim3(kThreads), 0, s, (const uint16_t*)x, dst, rows, d, ld);
+                         dim3(kThreads), 0, s, (const uint16_t*)x, dst, (uint32_t)rows,
+                         (uint32_t)d, (uint32_t)ld);
       return (const uint16_t*)dst;
     };
     FastArgs args;
