@@ -386,9 +386,10 @@ __shared__ __attribute__((aligned(16))) uint8_t lds_a1[kOperandBytes];
 // kRagged (dense): T is not a multiple of 64, so an example's last step holds
 // fewer than 64 rows; the rows past its end are fetched out of range (zeros)
 // and the MFMAs of a sub-step that holds none are skipped, as in grouped mode.
-// [24, 197, 768 x 3072] takes 48 us (and 9 for its split-K sum) against 1067 in the generic kernel (15
-// TFLOP/s there: its 4 x 4 FMA blocks are bound by LDS reads); what is left
-// is the 36 tiles' split-K traffic and the 23% of the last steps' empty rows.
+// [24, 197, 768 x 3072] takes 41 us (and 12 for its split-K sum) against 1067
+// in the generic kernel (15 TFLOP/s there: its 4 x 4 FMA blocks are bound by LDS
+// reads); what is left is the 36 tiles' split-K traffic and the 23% of the last
+// steps' empty rows.
 template <bool kGrouped, bool kGdma, int kWaves, bool kHalfDma = false, bool kRagged = false>
 __device__ __forceinline__ void clipped_sum_tile(const FastArgs& args) {
   constexpr int kT = kWaves * 64;           // threads
