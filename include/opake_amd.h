@@ -198,15 +198,17 @@ int dpc_clip_factors_groups(const double* sqnorm, const double* sqerr, int n_gro
  *                    guard_mult, n_guards, count_threshold, scale, scale64,
  *                    norms_out, nclipped, plan, stream)
  * (the same bits), in ONE launch when the split Gram kernel applies (bf16,
- * T an even number of 128-row blocks, din and dout multiples of 8, no bias,
- * B <= 2048): its last work item folds the records and computes the clip
- * factors.  ws: dpc_gram_clip_workspace_bytes(B, T) bytes of scratch (any
- * content).  counters: dpc_gram_clip_counter_bytes(B, T) bytes that must be
- * zero before the first call on them; every call leaves them zero again, so
- * one zero-filled buffer (as large as the largest call needs) serves call
- * after call of any shape on one stream -- calls that overlap on one
- * counter buffer race; the separate-launch shapes do not touch it.  sqnorm
- * is required. */
+ * T an even number of 128-row blocks up to 44, din and dout multiples of 8,
+ * B <= 1024, no bias): its last work item folds the records and computes the
+ * clip factors.  With a bias these shapes take two launches, the column norms
+ * before the rest.  ws:
+ * dpc_gram_clip_workspace_bytes(B, T) bytes of scratch (any content).
+ * counters: dpc_gram_clip_counter_bytes(B, T) bytes that must be zero before
+ * the first call on them; every call leaves them zero again, so one
+ * zero-filled buffer (as large as the largest call needs) serves call after
+ * call of any shape on one stream -- calls that overlap on one counter buffer
+ * race; calls with a bias (their counters are words of ws) and the
+ * separate-launch shapes neither need nor touch it.  sqnorm is required. */
 size_t dpc_gram_clip_workspace_bytes(int B, int T);
 size_t dpc_gram_clip_counter_bytes(int B, int T);
 int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, int dout,

@@ -2096,14 +2096,18 @@ segment_finish_kernel(const double* __restrict__ records, const int32_t* __restr
 // ||sum_t G_i[t]||^2 for a bias: workgroup (slot, ex) takes every n_slots-th
 // block of 128 columns of example ex (column sums in fp32, the values that the
 // clipped sum adds, see bias_cols.h) and writes the fp64 sum of their squares
-// to out[ex * n_slots + slot]; the finish kernel adds the slots.
+// to out[ex * n_slots + slot]; the finish kernel adds the slots.  The launch
+// also clears the n_zero words at `zero` (the counters of the launch after it).
 template <typename In>
 __global__ void __launch_bounds__(kBiasThreads)
 bias_sqnorm_kernel(const In* __restrict__ G, int T, int dout, int n_slots,
-                   double* __restrict__ out) {
+                   double* __restrict__ out, int32_t* __restrict__ zero, int n_zero) {
   __shared__ float red[kBiasRedFloats];
   __shared__ double fold[kBiasThreads / 64];
   const int slot = blockIdx.x, ex = blockIdx.y;
+  for (int i = (ex * n_slots + slot) * kBiasThreads + (int)threadIdx.x; i < n_zero;
+       i += (int)gridDim.y * n_slots * kBiasThreads)
+    zero[i] = 0;
   const In* g = G + (size_t)ex * T * dout;
   double s = 0.0;
   for (int c0 = slot * kBiasCols; c0 < dout; c0 += n_slots * kBiasCols) {
@@ -2200,16 +2204,17 @@ extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
   return gram_bias_slots_offset(B, T) + (size_t)B * kBiasSlots * sizeof(double);
 }
 
-// The column norms of a bias into `out` ([B, n_slots] words).
+// The column norms of a bias into `out` ([B, n_slots] words); clears n_zero
+// words at `zero`.
 static int launch_bias_sqnorm(const void* G, int B, int T, int dout, int dtype, int n_slots,
-                              double* out, hipStream_t s) {
+                              double* out, int32_t* zero, int n_zero, hipStream_t s) {
   const dim3 grid(n_slots, B);
   if (dtype == DPC_BF16) {
     hipLaunchKernelGGL(bias_sqnorm_kernel<uint16_t>, grid, dim3(kBiasThreads), 0, s,
-                       (const uint16_t*)G, T, dout, n_slots, out);
+                       (const uint16_t*)G, T, dout, n_slots, out, zero, n_zero);
   } else {
     hipLaunchKernelGGL(bias_sqnorm_kernel<float>, grid, dim3(kBiasThreads), 0, s, (const float*)G, T,
-                       dout, n_slots, out);
+                       dout, n_slots, out, zero, n_zero);
   }
   DPC_HIP_CHECK(hipGetLastError());
   return DPC_OK;
@@ -2306,7 +2311,7 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
     } else {
       bias = records + (size_t)nt * (nt + 1) / 2 * (size_t)B * DPC_GRAM_REC_WORDS;
     }
-    const int r = launch_bias_sqnorm(G, B, T, dout, dtype, n_slots, bias, s);
+    const int r = launch_bias_sqnorm(G, B, T, dout, dtype, n_slots, bias, nullptr, 0, s);
     if (r != DPC_OK) return r;
   }
   if (clip) {
@@ -2623,15 +2628,17 @@ bool gram_clip_one_launch(int B, int T, int din, int dout, int dtype) {
 }
 }  // namespace
 
-extern "C" size_t dpc_gram_clip_workspace_bytes(int B, int T) {
-  return dpc_gram_workspace_bytes(B, T);
-}
-
 extern "C" size_t dpc_gram_clip_counter_bytes(int B, int T) {
   if (B <= 0 || T <= 0) return 0;
   const int nsets = split_shape(T) ? split_sets_per_example(ceil_div(T, kGramTile)) : 0;
   // The split kernel's tickets, one counter per example, the example counter.
   return (size_t)(3 * (size_t)B * nsets + (size_t)B + 1) * sizeof(int32_t);
+}
+
+// The norms' workspace and a biased layer's own counters.
+extern "C" size_t dpc_gram_clip_workspace_bytes(int B, int T) {
+  if (B <= 0 || T <= 0) return 0;
+  return align256(dpc_gram_workspace_bytes(B, T)) + dpc_gram_clip_counter_bytes(B, T);
 }
 
 extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din,
@@ -2656,10 +2663,10 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   if (r != DPC_OK) return r;
   // A bias goes with the one launch (it saves the ticket reset, the finish and
   // the clip pass: [24, 197, 768 x 3072] 120 -> 112 us in all) when the
-  // workspace holds its column norms and, as it did not need them before, when
-  // there are counters.
-  const bool bias_fits = !with_bias || (ws_bytes >= dpc_gram_workspace_bytes(B, T) && counters &&
-                                        counter_bytes >= dpc_gram_clip_counter_bytes(B, T));
+  // workspace holds its column norms and the counters, which the column norms'
+  // launch clears: a biased call does not touch the caller's counter buffer, so
+  // it may overlap with a call that uses it.
+  const bool bias_fits = !with_bias || ws_bytes >= dpc_gram_clip_workspace_bytes(B, T);
   if (!gram_clip_one_launch(B, T, din, dout, dtype) || !bias_fits) {
     // The norms, then (in their last launch, for a small batch) the clip
     // factors; the counters are not used.
@@ -2671,15 +2678,19 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
                             n_guards, count_threshold, scale, scale64, norms_out, nclipped, plan,
                             nonfinite, stream);
   }
-  if (!counters) return DPC_EINVAL;
-  if (counter_bytes < dpc_gram_clip_counter_bytes(B, T)) return DPC_ENOSPC;
+  uint8_t* base = (uint8_t*)ws;
+  if (with_bias) {
+    counters = (int32_t*)(base + align256(dpc_gram_workspace_bytes(B, T)));
+  } else {
+    if (!counters) return DPC_EINVAL;
+    if (counter_bytes < dpc_gram_clip_counter_bytes(B, T)) return DPC_ENOSPC;
+  }
   hipStream_t s = (hipStream_t)stream;
   const int nt = ceil_div(T, kGramTile);
   const int npairs = nt * (nt + 1) / 2;
   const int nsets = split_sets_per_example(nt);
   const int nblocks = 2 * nsets * B;
   const int padded = ceil_div(nblocks, kXcds) * kXcds;
-  uint8_t* base = (uint8_t*)ws;
   double* records = (double*)base;
   // The exchange area where dpc_gram_sqnorms keeps it (after the records
   // and its own ticket words, unused here).
@@ -2707,7 +2718,8 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
     tail.n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
     double* slots = (double*)(base + gram_bias_slots_offset(B, T));
     tail.bias = slots;
-    r = launch_bias_sqnorm(G, B, T, dout, dtype, tail.n_slots, slots, s);
+    r = launch_bias_sqnorm(G, B, T, dout, dtype, tail.n_slots, slots, counters,
+                           (int)(dpc_gram_clip_counter_bytes(B, T) / sizeof(int32_t)), s);
     if (r != DPC_OK) return r;
   }
   hipLaunchKernelGGL(gram_split_bf16_kernel, dim3(padded), dim3(512), 0, s, lay, B, T, npairs,

@@ -10,6 +10,8 @@ blocks, float32) interleaved with one-launch calls.
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -88,3 +90,29 @@ def test_gram_clip_factors_leaves_counters_zero(dev):
         counters = ops._GRAM_CLIP_COUNTERS[(str(dev), nat.stream_handle(dev).value or 0)]
         assert counters.numel() * 4 >= nat.load().dpc_gram_clip_counter_bytes(B, T)
         assert torch.count_nonzero(counters).item() == 0, (B, T)
+
+
+@pytest.mark.parametrize("T", [256, 384])  # the split kernel, and separate launches
+def test_a_biased_call_leaves_the_counter_buffer_alone(dev, T):
+    """A bias needs no counters and does not touch any it is given (another
+    stream's call may be using them): none, and words that are no counters."""
+    B, din, dout = 6, 128, 264
+    A, G = _inputs(dev, B, T, din, dout, torch.bfloat16, T)
+    guard = guard_for_linear(torch.bfloat16, din, dout, True)
+    sq, err, cf = _two_calls(A, G, 1.0, [guard], True, nat.SCALE_FIXED, 0.0)
+    lib = nat.load()
+    ws_bytes = lib.dpc_gram_clip_workspace_bytes(B, T)
+    n = lib.dpc_gram_clip_counter_bytes(B, T) // 4
+    rel, abs_ = (ctypes.c_double * 1)(guard[0]), (ctypes.c_double * 1)(guard[1])
+    for counters in (None, torch.full((n,), 0x5A5A5A5A, dtype=torch.int32, device=dev)):
+        ws = torch.full((ws_bytes,), 0xA5, dtype=torch.uint8, device=dev)
+        got_sq, got_err = torch.empty_like(sq), torch.empty_like(err)
+        scale = torch.empty_like(cf.scale)
+        nat.call("dpc_gram_clip_factors", nat.ptr(A), nat.ptr(G), B, T, din, dout,
+                 nat.dtype_code(A.dtype), 1, 1.0, nat.SCALE_FIXED, 0.0, rel, abs_, None, 1, 1.0,
+                 nat.ptr(got_sq), nat.ptr(got_err), nat.ptr(scale), None, None, None, None, None,
+                 nat.ptr(ws), ws_bytes, nat.ptr(counters), 4 * n if counters is not None else 0,
+                 nat.stream_handle(dev))
+        assert torch.equal(got_sq, sq) and torch.equal(got_err, err)
+        assert torch.equal(scale, cf.scale)
+        assert counters is None or bool((counters == 0x5A5A5A5A).all())
