@@ -1751,8 +1751,32 @@ __device__ __forceinline__ void generic_tile_stats(const double pa[4][4], const 
                        0.0, st);
 }
 
-// Dense fp64 Gram path (fp32 operands, and bf16 shapes off the bf16 MFMA
-// path): products of fp32 values are exact in fp64, and the 16x16x4 fp64 MFMA
+// Dense generic path, one 64-row tile pair a workgroup: the layers that
+// gram_f64_route leaves to it.
+template <typename In>
+__global__ void __launch_bounds__(kGramThreads)
+gram_generic_kernel(const In* __restrict__ A, const In* __restrict__ G, int T, int din, int dout,
+                    int npairs, double* __restrict__ records) {
+  __shared__ float sp[kGenK][kGenTile + 1];
+  __shared__ float sq[kGenK][kGenTile + 1];
+  __shared__ double red[kRecStat * (kGramThreads / 64)];
+  const int pair = blockIdx.x, ex = blockIdx.y;
+  int p, q;
+  pair_from_index(pair, &p, &q);
+  double pa[4][4], pg[4][4];
+  gram_tile_generic<In>(A + (size_t)ex * T * din, T, din, p, q, sp, sq, pa);
+  gram_tile_generic<In>(G + (size_t)ex * T * dout, T, dout, p, q, sp, sq, pg);
+  const double gA = dpc_chain_gamma((double)ceil_div(din, kGenK) * kGenK, DPC_GRAM_U_FP64);
+  const double gQ = dpc_chain_gamma((double)ceil_div(dout, kGenK) * kGenK, DPC_GRAM_U_FP64);
+  double st[kRecStat] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  generic_tile_stats(pa, pg, p == q, gA, gQ, st);
+  if (p != q) st[0] *= 2.0;
+  write_gram_record(st, red, records + ((size_t)ex * npairs + pair) * DPC_GRAM_REC_WORDS, gA, gQ,
+                    T);
+}
+
+// Dense fp64 MFMA path (fp32 operands, and bf16 shapes off the bf16 MFMA path,
+// where gram_f64_route takes it): products of fp32 values are exact in fp64, and the 16x16x4 fp64 MFMA
 // sums them, so the error model is that of a fp64 chain.
 //
 // A workgroup computes one pair (p, q) of 32-row tiles of both Gram matrices:
@@ -1773,8 +1797,8 @@ __device__ __forceinline__ void generic_tile_stats(const double pa[4][4], const 
 // order of k is permuted alike on both sides.  A last chunk that is not full is
 // read element by element, so no load reaches past a row's end.
 //
-// With `subs` = 2 (a workspace that holds only the records of 64-row tiles)
-// the pair's 32-row sub-pairs run one after the other.
+// With `subs` = 2 the pair is one of 64-row tiles, whose 32-row sub-pairs run one
+// after the other into one record.
 constexpr int kF64Threads = 256;
 constexpr int kF64Rows = 32;   // rows of a tile
 constexpr int kF64Depth = 32;  // depth of a chunk
@@ -2180,6 +2204,46 @@ size_t split_tickets_bytes(int B, int T) {
 }
 }  // namespace
 
+// Kernel and tile rows of a dense layer off the bf16 MFMA path.  The FMA kernel
+// takes one operand's chunks after the other's; the MFMA kernel's waves take both
+// side by side, so it costs what the deeper one does, but more to start and to
+// take its statistics, which one wave of four does; and 32-row tiles leave four
+// times the records, which one wave an example folds at some 0.04 us each.  So
+// the FMA kernel keeps the narrow layers, the more so the longer the sequence and
+// the narrower one operand is beside the other, and 32-row tiles are for calls of
+// few tile pairs, which they spread over the chip, and for layers deep enough to pay
+// for the fold.  The lines lie where the times cross, within some 10%.
+// gram_sqnorms in us, FMA / 64-row MFMA / 32-row MFMA:
+//   fp32 [1, 512, 28 x 28] 16 / 22 / 16         [1, 512, 516 x 516] 159 / 58 / 23
+//        [32, 256, 28 x 28] 20 / 25 / 25        [32, 256, 100 x 100] 56 / 34 / 29
+//        [32, 1024, 12 x 12] 64 / 166 / 222     [32, 1024, 516 x 516] 1276 / 709 / 721
+//        [32, 1024, 60 x 60] 168 / 182 / 257    [32, 1024, 12 x 300] 410 / 408 / 439
+//        [4, 4096, 100 x 100] 554 / 541 / 1130  [4, 4096, 12 x 300] 769 / 886 / 1409
+//        [1, 2048, 2052 x 2052] 1004 / 466 / 405, [2, 4096, same] 5104 / 2506 / 2837
+//   bf16 [66, 312, 27 x 99] 51 / 65 / 60        [66, 312, 59 x 299] 126 / 118 / 94
+//        [32, 1024, 11 x 99] 170 / 201 / 248    [32, 1024, 11 x 299] 402 / 362 / 396
+enum class F64Route { kFma, kMfma64, kMfma32 };
+constexpr int kF64FineMaxT = 2048;  // kMfma32 holds no longer example
+static F64Route gram_f64_route(int B, int T, int din, int dout, int dtype) {
+  const int lo = din < dout ? din : dout, hi = din < dout ? dout : din;
+  const size_t nt = ceil_div(T, kGenTile), pairs = nt * (nt + 1) / 2 * (size_t)B;
+  bool narrow;
+  if (T <= kF64Rows)
+    narrow = false;  // one 32-row tile: [156, 2, 39 x 10] 10 us, the FMA kernel 14
+  else if (pairs < 512)
+    narrow = lo + hi <= 60;  // a round of workgroups: the FMA kernel's is its chunks
+  else if (T < 1024)
+    narrow = lo + hi / 2 < (T <= 256 ? 65 : 80);
+  else if (dtype == DPC_BF16)
+    narrow = lo + hi / 3 < 85;
+  else
+    narrow = lo + hi / 6 < (T < 2048 ? 80 : 100);
+  if (narrow) return F64Route::kFma;
+  if (T > kF64FineMaxT) return F64Route::kMfma64;
+  const int depth = T / (pairs >= 1024 || T > 1024 ? 2 : pairs >= 512 ? 3 : 4);
+  return pairs <= 128 || hi >= depth ? F64Route::kMfma32 : F64Route::kMfma64;
+}
+
 // The smallest workspace dpc_gram_sqnorms takes.  What dpc_gram_workspace_bytes
 // adds: the records of 32-row tiles of the fp64 path (in place of the 64-row
 // ones; without the room that path keeps 64-row tiles), and kBiasSlots words
@@ -2194,6 +2258,7 @@ static size_t gram_min_bytes(int B, int T) {
 }
 static size_t gram_bias_slots_offset(int B, int T) {
   size_t n = gram_min_bytes(B, T);
+  if (T > kF64FineMaxT) return align256(n);
   const size_t nt = ceil_div(T, kF64Rows);
   const size_t fine = nt * (nt + 1) / 2 * B * DPC_GRAM_REC_WORDS * sizeof(double);
   return align256(n > fine ? n : fine);
@@ -2274,18 +2339,29 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
     hipLaunchKernelGGL(gram_mfma_bf16_kernel, dim3(padded), dim3(512), 0, s, (const uint16_t*)A,
                        (const uint16_t*)G, T, din, dout, npairs, items, nblocks, records);
   } else {
-    // A launch holds less than 2^32 threads: more tile pairs go out as several
-    // launches of whole examples, an example of more than that in 64-row tiles.
-    constexpr size_t kMaxBlocks = ((size_t)1 << 32) / kF64Threads - 2 * kXcds;
-    const size_t fine = ceil_div(T, kF64Rows);
-    const bool coarse = !full_ws || fine * (fine + 1) / 2 > kMaxBlocks;
-    const int subs = coarse ? kGenTile / kF64Rows : 1;
+    F64Route route = gram_f64_route(B, T, din, dout, dtype);
+    if (route == F64Route::kMfma32 && !full_ws) route = F64Route::kMfma64;
+    const int subs = route == F64Route::kMfma32 ? 1 : kGenTile / kF64Rows;
     nt = ceil_div(T, kF64Rows * subs);
+    // A launch holds less than 2^32 threads: more tile pairs of the MFMA kernel
+    // go out as several launches of whole examples.
+    constexpr size_t kMaxBlocks = ((size_t)1 << 32) / kF64Threads - 2 * kXcds;
     const size_t np = (size_t)nt * (nt + 1) / 2;
     if (np > kMaxBlocks) return DPC_ENOTSUP;
     const int npairs = (int)np;
+    if (route == F64Route::kFma) {
+      const dim3 grid(npairs, B), block(kGramThreads);
+      if (dtype == DPC_BF16) {
+        hipLaunchKernelGGL(gram_generic_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)A,
+                           (const uint16_t*)G, T, din, dout, npairs, records);
+      } else {
+        hipLaunchKernelGGL(gram_generic_kernel<float>, grid, block, 0, s, (const float*)A,
+                           (const float*)G, T, din, dout, npairs, records);
+      }
+      DPC_HIP_CHECK(hipGetLastError());
+    }
     const int per_launch = (int)(kMaxBlocks / np < (size_t)B ? kMaxBlocks / np : (size_t)B);
-    for (int e0 = 0; e0 < B; e0 += per_launch) {
+    for (int e0 = 0; route != F64Route::kFma && e0 < B; e0 += per_launch) {
       const int nblocks = npairs * min(per_launch, B - e0);
       const dim3 grid(ceil_div(nblocks, kXcds) * kXcds), block(kF64Threads);
       const size_t row0 = (size_t)e0 * T;

@@ -180,14 +180,19 @@ def test_bias_finish_with_the_split_sums(dev, dtype, T, dout):
     assert torch.equal(bias[0], bias[1]) and torch.equal(bias[0], bias[2])
 
 
-# The fp64 Gram path: one, two and several 32-row tiles with ragged last ones,
-# depths around the 32-deep chunks, rows that 16-byte loads do not take, din !=
-# dout both ways; 16.8 million tile pairs, more than one launch holds (2^32 threads).
+# The fp64 Gram paths.  FMA kernel: narrow layers, at long sequences one wide
+# operand beside a narrow one.  MFMA kernel: one, two and several 32-row tiles with
+# ragged last ones, depths around the 32-deep chunks, rows that 16-byte loads do
+# not take, din != dout both ways; 64-row tiles (many tile pairs of shallow layers, more
+# than 2048 rows); 16.8 million tile pairs, more than one launch holds (2^32 threads).
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,din,dout", [
     (2, 2, 4, 8), (3, 31, 33, 9), (2, 32, 32, 31), (4, 65, 100, 36), (1, 130, 7, 260),
     (2, 257, 64, 65), (1024, 40, 12, 20), (110, 200, 33, 68),
-    (2040, 4096, 4, 4)])
+    (2040, 4096, 4, 4),
+    (5, 200, 29, 31), (5, 200, 30, 31), (100, 200, 43, 43), (100, 200, 44, 43), (100, 300, 52, 53),
+    (2, 1024, 63, 100), (2, 1100, 65, 127), (2, 2048, 31, 300), (2, 2050, 33, 900), (9, 1000, 131, 335),
+    (520, 16256, 65, 65)])
 def test_gram_f64(dev, dtype, B, T, din, dout):
     """Exact products in fp64: the error is within the kernel's own bound, and
     far below what fp32 sums would leave (2^-24)."""
@@ -210,6 +215,28 @@ def test_gram_f64(dev, dtype, B, T, din, dout):
     gammas = sum(1.125 * (-(-d // 16) * 16) * 2.0**-52 for d in (din, dout))
     rows = A.double().square().sum(dim=(1, 2)) * G.double().square().sum(dim=(1, 2))
     assert (err <= 1.001 * (gammas + (T * T + 256) * 2.0**-52) * rows).all()
+
+
+def _kernels(fn):
+    fn()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    cuda = torch.autograd.DeviceType.CUDA
+    return [e.name for e in prof.events() if e.device_type == cuda]
+
+
+# Narrow layers, where the fp64 MFMA kernel takes up to five times as long, keep the
+# FMA kernel; deep ones and single tiles do not.
+@pytest.mark.parametrize("B,T,din,dout,kernel", [
+    (32, 1024, 12, 12, "gram_generic_kernel"), (4, 4096, 12, 300, "gram_generic_kernel"),
+    (66, 312, 27, 59, "gram_generic_kernel"), (16, 256, 516, 516, "gram_f64_kernel"),
+    (156, 30, 39, 10, "gram_f64_kernel")])
+def test_gram_f64_kernel_of_narrow_layers(dev, B, T, din, dout, kernel):
+    A = torch.randn(B, T, din, device=dev)
+    G = torch.randn(B, T, dout, device=dev)
+    assert any(kernel in n for n in _kernels(lambda: ops.gram_sqnorms(A, G)))
 
 
 # The fp32 MFMA path: chunks of 16 rows and their remainders, one token per
