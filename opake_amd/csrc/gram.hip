@@ -2071,11 +2071,19 @@ gram_finish_kernel(const double* __restrict__ records, int B, int nt, int nlayer
 }
 
 // The finish and the clip factors of a small batch by one workgroup, the same
-// bits as the two launches (4.3 us against 3.4 + 3.3 and the gap between
-// them).  Up to two examples a wave: more would wait for each other's folds
-// longer than that.
+// bits as the two launches.  Up to two examples a wave, of one record a lane, or
+// few records in all: one CU folds more of them longer than the launch it saves
+// takes, while the finish launch has B / 4 CUs.  us in one launch / two, by records
+// an example: 1 at B = 1 3.5 / 7.5, at B = 32 6 / 7.5; 55 at 32 8.1 / 8.2; 78 at 16
+// 7.5 / 8.0, at 32 12 / 8; 136 at 8 8.3 / 9.5, at 32 16 / 10; 528 at 1 15 / 18, at
+// 8 21 / 20, at 32 48 / 20.
 constexpr int kFinishClipThreads = 1024;
 constexpr int kFinishClipMaxB = 2 * kFinishClipThreads / 64;
+constexpr size_t kFinishClipMaxRecords = 1300;
+static bool finish_with_clip(int B, int nt) {
+  const size_t np = (size_t)nt * (nt + 1) / 2;
+  return B <= kFinishClipMaxB && (np <= 64 || np * (size_t)B <= kFinishClipMaxRecords);
+}
 
 __global__ void __launch_bounds__(kFinishClipThreads)
 gram_finish_clip_kernel(const double* __restrict__ records, int B, int nt,
@@ -2285,12 +2293,12 @@ static int launch_bias_sqnorm(const void* G, int B, int T, int dout, int dtype, 
   return DPC_OK;
 }
 
-// dpc_gram_sqnorms; with `clip` (accumulate == 0, B <= kFinishClipMaxB) the
-// last launch computes the clip factors too.
+// dpc_gram_sqnorms; with `clip` (accumulate == 0), where finish_with_clip takes
+// them, the last launch computes the clip factors too and *clipped is set.
 static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din, int dout,
                             int dtype, int with_bias, int accumulate, double* sqnorm,
-                            double* sqerr, const ClipJob* clip, void* ws, size_t ws_bytes,
-                            void* stream) {
+                            double* sqerr, const ClipJob* clip, bool* clipped, void* ws,
+                            size_t ws_bytes, void* stream) {
   if (B < 0 || T <= 0 || din <= 0 || dout <= 0) return DPC_EINVAL;
   if (B == 0) return DPC_OK;
   if (!A || !G || !sqnorm || !ws) return DPC_EINVAL;
@@ -2390,7 +2398,8 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
     const int r = launch_bias_sqnorm(G, B, T, dout, dtype, n_slots, bias, nullptr, 0, s);
     if (r != DPC_OK) return r;
   }
-  if (clip) {
+  if (clip && finish_with_clip(B, nt)) {
+    *clipped = true;
     hipLaunchKernelGGL(gram_finish_clip_kernel, dim3(1), dim3(kFinishClipThreads), 0, s,
                        (const double*)records, B, nt, (const double*)bias, n_slots, sqnorm, sqerr,
                        *clip);
@@ -2407,7 +2416,7 @@ extern "C" int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int 
                                 int dtype, int with_bias, int accumulate, double* sqnorm,
                                 double* sqerr, void* ws, size_t ws_bytes, void* stream) {
   return gram_sqnorms_run(A, G, B, T, din, dout, dtype, with_bias, accumulate, sqnorm, sqerr,
-                          nullptr, ws, ws_bytes, stream);
+                          nullptr, nullptr, ws, ws_bytes, stream);
 }
 
 // Workspace of dpc_grouped_gram_sqnorms: the records, the split kernel's
@@ -2746,10 +2755,10 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   if (!gram_clip_one_launch(B, T, din, dout, dtype) || !bias_fits) {
     // The norms, then (in their last launch, for a small batch) the clip
     // factors; the counters are not used.
-    const bool together = B <= kFinishClipMaxB;
-    r = gram_sqnorms_run(A, G, B, T, din, dout, dtype, with_bias, 0, sqnorm, sqerr,
-                         together ? &job : nullptr, ws, ws_bytes, stream);
-    if (r != DPC_OK || together) return r;
+    bool clipped = false;
+    r = gram_sqnorms_run(A, G, B, T, din, dout, dtype, with_bias, 0, sqnorm, sqerr, &job, &clipped,
+                         ws, ws_bytes, stream);
+    if (r != DPC_OK || clipped) return r;
     return dpc_clip_factors(sqnorm, sqerr, B, C, kind, gamma, guard_rel, guard_abs, guard_mult,
                             n_guards, count_threshold, scale, scale64, norms_out, nclipped, plan,
                             nonfinite, stream);

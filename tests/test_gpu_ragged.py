@@ -317,10 +317,11 @@ def test_leaves_unaligned_match_oracle(dev, dtype, B, out):
 
 
 # Norms and clip factors: finished together for up to 32 examples (one and two
-# a wave), by two launches past that; a bias inside the one-launch path (an even
+# a wave) of few records, by two launches past that; a bias inside the one-launch path (an even
 # number of 128-row blocks) and beside it; call after call on one counter buffer.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("B,T", [(1, 24), (16, 40), (17, 70), (32, 33), (33, 20), (9, 200), (40, 256)])
+@pytest.mark.parametrize("B,T", [(1, 24), (16, 40), (17, 70), (32, 33), (33, 20), (9, 200), (40, 256),
+                                 (16, 1152), (32, 1152), (32, 1408)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_clip_factors_with_the_norms(dev, dtype, B, T, bias):
     A, G = (x.to(dev, dtype) for x in _operands(B, T, 64, 264, B + T))
@@ -357,3 +358,12 @@ def test_clipped_sum_multi_few_tiles_long_k(dev):
     for w, a, g, pair, noise in zip(got, As, Gs, pairs, (0.5 * z, 0, 0)):
         assert torch.equal(w, ops.clipped_sum(a, g, cf.scale[0], **kw)[0] + noise)
         assert _rel((w - noise).cpu(), _exact(*pair, cf.scale[0].cpu().double())) < 1e-5
+
+
+# bf16 tile pairs of 128 rows: 45 and 66 records an example.
+@pytest.mark.parametrize("B,T,one", [(32, 1152, True), (16, 1408, True), (32, 1408, False)])
+def test_one_workgroup_finishes_few_records_only(dev, B, T, one):
+    A, G = (x.to(dev) for x in _operands(B, T, 16, 8, 1))
+    guards = [guard_for_linear(torch.bfloat16, 16, 8, False)]
+    names = _kernels(lambda: ops.gram_clip_factors(A, G, 1.0, guards, count_threshold=1.0))
+    assert any("gram_finish_clip_kernel" in n for n in names) == one
