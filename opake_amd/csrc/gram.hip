@@ -2228,10 +2228,11 @@ size_t split_tickets_bytes(int B, int T) {
 //        [32, 1024, 60 x 60] 168 / 182 / 257    [32, 1024, 12 x 300] 410 / 408 / 439
 //        [4, 4096, 100 x 100] 554 / 541 / 1130  [4, 4096, 12 x 300] 769 / 886 / 1409
 //        [1, 2048, 2052 x 2052] 1004 / 466 / 405, [2, 4096, same] 5104 / 2506 / 2837
+//        [5, 2198, 3328 x 1256] - / 2821 / 2437 (6.2 rounds of 64-row pairs: 7)
 //   bf16 [66, 312, 27 x 99] 51 / 65 / 60        [66, 312, 59 x 299] 126 / 118 / 94
 //        [32, 1024, 11 x 99] 170 / 201 / 248    [32, 1024, 11 x 299] 402 / 362 / 396
 enum class F64Route { kFma, kMfma64, kMfma32 };
-constexpr int kF64FineMaxT = 2048;  // kMfma32 holds no longer example
+constexpr int kF64FineMaxT = 4096;  // kMfma32 holds no longer example
 static F64Route gram_f64_route(int B, int T, int din, int dout, int dtype) {
   const int lo = din < dout ? din : dout, hi = din < dout ? dout : din;
   const size_t nt = ceil_div(T, kGenTile), pairs = nt * (nt + 1) / 2 * (size_t)B;
@@ -2239,7 +2240,7 @@ static F64Route gram_f64_route(int B, int T, int din, int dout, int dtype) {
   if (T <= kF64Rows)
     narrow = false;  // one 32-row tile: [156, 2, 39 x 10] 10 us, the FMA kernel 14
   else if (pairs < 512)
-    narrow = lo + hi <= 60;  // a round of workgroups: the FMA kernel's is its chunks
+    narrow = lo + hi <= (pairs <= 128 ? 32 : pairs <= 256 ? 60 : 70);  // a round of workgroups
   else if (T < 1024)
     narrow = lo + hi / 2 < (T <= 256 ? 65 : 80);
   else if (dtype == DPC_BF16)
@@ -2248,7 +2249,10 @@ static F64Route gram_f64_route(int B, int T, int din, int dout, int dtype) {
     narrow = lo + hi / 6 < (T < 2048 ? 80 : 100);
   if (narrow) return F64Route::kFma;
   if (T > kF64FineMaxT) return F64Route::kMfma64;
-  const int depth = T / (pairs >= 1024 || T > 1024 ? 2 : pairs >= 512 ? 3 : 4);
+  const int depth = T > 3072                    ? T
+                    : pairs >= 1024 || T > 1024 ? T / 2
+                    : pairs >= 512              ? T / 3
+                                                : T / 4;
   return pairs <= 128 || hi >= depth ? F64Route::kMfma32 : F64Route::kMfma64;
 }
 
