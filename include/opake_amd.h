@@ -86,7 +86,8 @@ int dpc_write_words(void* dst, const uint32_t* host_words, int n, void* stream);
  * rounding or truncation of at most one fp32 ulp per addend of an MFMA
  * instruction, and flushed subnormals; generic path: fp64) and the fp64
  * inner product.  A layer bias adds ||sum_t G_i[t]||^2 (and its bound) when
- * with_bias != 0.  Examples whose A_i or G_i hold NaN/Inf produce a
+ * with_bias != 0.  ws: dpc_gram_workspace_bytes(B, T) bytes; less is taken
+ * down to the records of 64-row tiles, DPC_ENOSPC below that.  Examples whose A_i or G_i hold NaN/Inf produce a
  * non-finite value (their clip factor becomes 0).
  * -------------------------------------------------------------------------*/
 size_t dpc_gram_workspace_bytes(int B, int T);
@@ -101,7 +102,9 @@ int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int do
  * With bf16 operands, T an even number of 128-row blocks, B a multiple of 8
  * and up to 8 layers, all layers share one launch (the work items of every
  * layer spread over all XCDs); otherwise the layers run one by one.  ws:
- * dpc_gram_sqnorms_multi_workspace_bytes. */
+ * dpc_gram_sqnorms_multi_workspace_bytes (as in dpc_gram_sqnorms, fp32 and
+ * odd-width layers may take 64-row tiles where 32-row ones do not fit a smaller
+ * ws: norms that differ in their last bits, with their own bounds). */
 size_t dpc_gram_sqnorms_multi_workspace_bytes(int n, const int* din, const int* dout, int B,
                                               int T, int dtype);
 int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* const* G, const int* din,
@@ -110,8 +113,8 @@ int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* const* G, co
                            void* stream);
 
 /* dpc_gram_sqnorms_noalloc: no counterpart in the reference.  The same
- * computation as dpc_gram_sqnorms with no workspace argument and no
- * allocation, for callers that cannot allocate device memory (code under HIP
+ * computation as dpc_gram_sqnorms (the same bits where its workspace fits the
+ * scratch) with no workspace argument and no allocation, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): the
  * workspace is a static device array of DPC_NOALLOC_SCRATCH_BYTES per device,
  * held until the process ends.  Calls needing more

@@ -2268,17 +2268,30 @@ static size_t gram_min_bytes(int B, int T) {
          (size_t)B * split_sets_per_example(ceil_div(T, kGramTile)) * 2 * kSplitSetBytes;
   return n;
 }
-static size_t gram_bias_slots_offset(int B, int T) {
-  size_t n = gram_min_bytes(B, T);
-  if (T > kF64FineMaxT) return align256(n);
+// Where the bias words start; `fine`: after the records of 32-row tiles.
+static size_t gram_slots_at(int B, int T, bool fine) {
+  const size_t n = gram_min_bytes(B, T);
+  if (!fine) return align256(n);
   const size_t nt = ceil_div(T, kF64Rows);
-  const size_t fine = nt * (nt + 1) / 2 * B * DPC_GRAM_REC_WORDS * sizeof(double);
-  return align256(n > fine ? n : fine);
+  const size_t records = nt * (nt + 1) / 2 * B * DPC_GRAM_REC_WORDS * sizeof(double);
+  return align256(n > records ? n : records);
+}
+// The bf16 MFMA path.  Buffer offsets are 32-bit: one example's rows (plus a tile
+// of padding) must stay below 2 GiB.
+static bool gram_mfma_shape(int T, int din, int dout, int dtype) {
+  const size_t dmax = (size_t)(din > dout ? din : dout);
+  return dtype == DPC_BF16 && din % 8 == 0 && dout % 8 == 0 &&
+         ((size_t)T + kGramTile) * dmax * 2 < ((size_t)1 << 31);
+}
+// What a bias-free layer's norms use at most.
+static size_t gram_layer_bytes(int B, int T, int din, int dout, int dtype) {
+  return gram_slots_at(B, T, !gram_mfma_shape(T, din, dout, dtype) &&
+                                 gram_f64_route(B, T, din, dout, dtype) == F64Route::kMfma32);
 }
 
 extern "C" size_t dpc_gram_workspace_bytes(int B, int T) {
   if (B <= 0 || T <= 0) return 0;
-  return gram_bias_slots_offset(B, T) + (size_t)B * kBiasSlots * sizeof(double);
+  return gram_slots_at(B, T, T <= kF64FineMaxT) + (size_t)B * kBiasSlots * sizeof(double);
 }
 
 // The column norms of a bias into `out` ([B, n_slots] words); clears n_zero
@@ -2310,14 +2323,10 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
   if (B > 65535) return DPC_ENOTSUP;
   if (ws_bytes < gram_min_bytes(B, T)) return DPC_ENOSPC;
   hipStream_t s = (hipStream_t)stream;
-  const bool full_ws = ws_bytes >= dpc_gram_workspace_bytes(B, T);
   double* records = (double*)ws;
   int nt;
-  // Buffer offsets are 32-bit: one example's rows (plus a tile of padding)
-  // must stay below 2 GiB for the MFMA path.
-  const size_t dmax = (size_t)(din > dout ? din : dout);
-  const bool fits = ((size_t)T + kGramTile) * dmax * 2 < ((size_t)1 << 31);
-  const bool mfma = dtype == DPC_BF16 && din % 8 == 0 && dout % 8 == 0 && fits;
+  bool fine = false;
+  const bool mfma = gram_mfma_shape(T, din, dout, dtype);
   if (mfma && split_shape(T)) {
     // One operand per work item; the tickets start at zero.
     nt = ceil_div(T, kGramTile);
@@ -2352,8 +2361,10 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
                        (const uint16_t*)G, T, din, dout, npairs, items, nblocks, records);
   } else {
     F64Route route = gram_f64_route(B, T, din, dout, dtype);
-    if (route == F64Route::kMfma32 && !full_ws) route = F64Route::kMfma64;
-    const int subs = route == F64Route::kMfma32 ? 1 : kGenTile / kF64Rows;
+    if (route == F64Route::kMfma32 && ws_bytes < gram_slots_at(B, T, true))
+      route = F64Route::kMfma64;
+    fine = route == F64Route::kMfma32;
+    const int subs = fine ? 1 : kGenTile / kF64Rows;
     nt = ceil_div(T, kF64Rows * subs);
     // A launch holds less than 2^32 threads: more tile pairs of the MFMA kernel
     // go out as several launches of whole examples.
@@ -2393,9 +2404,10 @@ static int gram_sqnorms_run(const void* A, const void* G, int B, int T, int din,
   double* bias = nullptr;
   int n_slots = 1;
   if (with_bias) {
-    if (full_ws) {
+    const size_t at = gram_slots_at(B, T, fine);
+    if (ws_bytes >= at + (size_t)B * kBiasSlots * sizeof(double)) {
       n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
-      bias = (double*)((uint8_t*)ws + gram_bias_slots_offset(B, T));
+      bias = (double*)((uint8_t*)ws + at);
     } else {
       bias = records + (size_t)nt * (nt + 1) / 2 * (size_t)B * DPC_GRAM_REC_WORDS;
     }
@@ -2613,13 +2625,9 @@ namespace {
 // The split-mode shape of dpc_gram_sqnorms_multi: bf16, T an even number of
 // 128-row blocks, B a multiple of 8, every layer on the MFMA path.
 bool split_multi_shape(int n, const int* din, const int* dout, int B, int T, int dtype) {
-  if (n < 2 || n > kSplitMaxLayers || dtype != DPC_BF16 || B % kXcds != 0 || !split_shape(T))
-    return false;
-  for (int i = 0; i < n; ++i) {
-    const size_t dmax = (size_t)(din[i] > dout[i] ? din[i] : dout[i]);
-    if (din[i] % 8 != 0 || dout[i] % 8 != 0 || ((size_t)T + kGramTile) * dmax * 2 >= ((size_t)1 << 31))
-      return false;
-  }
+  if (n < 2 || n > kSplitMaxLayers || B % kXcds != 0 || !split_shape(T)) return false;
+  for (int i = 0; i < n; ++i)
+    if (!gram_mfma_shape(T, din[i], dout[i], dtype)) return false;
   return true;
 }
 size_t split_multi_bytes(int n, int B, int T) {
@@ -2631,13 +2639,26 @@ size_t split_multi_bytes(int n, int B, int T) {
 }
 }  // namespace
 
-extern "C" size_t dpc_gram_sqnorms_multi_workspace_bytes(int n, const int* din, const int* dout,
-                                                        int B, int T, int dtype) {
-  if (n <= 0 || B <= 0 || T <= 0 || !din || !dout) return 0;
+// The smallest workspace dpc_gram_sqnorms_multi takes: one layer's smallest, or
+// the shared launch's.
+static size_t gram_multi_min_bytes(int n, const int* din, const int* dout, int B, int T, int dtype) {
   const size_t one = gram_min_bytes(B, T);
   if (!split_multi_shape(n, din, dout, B, T, dtype)) return one;
   const size_t multi = split_multi_bytes(n, B, T);
   return multi > one ? multi : one;
+}
+
+// Layer by layer, each takes the kernel and tiles of its own call.
+extern "C" size_t dpc_gram_sqnorms_multi_workspace_bytes(int n, const int* din, const int* dout,
+                                                        int B, int T, int dtype) {
+  if (n <= 0 || B <= 0 || T <= 0 || !din || !dout) return 0;
+  size_t bytes = gram_multi_min_bytes(n, din, dout, B, T, dtype);
+  if (!split_multi_shape(n, din, dout, B, T, dtype))
+    for (int i = 0; i < n; ++i) {
+      const size_t layer = gram_layer_bytes(B, T, din[i], dout[i], dtype);
+      if (layer > bytes) bytes = layer;
+    }
+  return bytes;
 }
 
 extern "C" int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* const* G,
@@ -2651,8 +2672,7 @@ extern "C" int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* c
   for (int i = 0; i < n; ++i)
     if (!A[i] || !G[i] || din[i] <= 0 || dout[i] <= 0) return DPC_EINVAL;
   if (B > 65535) return DPC_ENOTSUP;
-  if (ws_bytes < dpc_gram_sqnorms_multi_workspace_bytes(n, din, dout, B, T, dtype))
-    return DPC_ENOSPC;
+  if (ws_bytes < gram_multi_min_bytes(n, din, dout, B, T, dtype)) return DPC_ENOSPC;
   if (!split_multi_shape(n, din, dout, B, T, dtype)) {
     // Layer by layer, each accumulating into the previous layers' sums.
     for (int i = 0; i < n; ++i) {
@@ -2707,12 +2727,10 @@ extern "C" int dpc_gram_sqnorms_multi(int n, const void* const* A, const void* c
 
 namespace {
 bool gram_clip_one_launch(int B, int T, int din, int dout, int dtype) {
-  const size_t dmax = (size_t)(din > dout ? din : dout);
   // The tail's LDS holds one example's records, then B flag words.
   const size_t nt = (size_t)ceil_div(T, kGramTile), np = nt * (nt + 1) / 2;
   const size_t lds_doubles = (size_t)(4 * 3 * kGTileBytes) / sizeof(double);
-  return dtype == DPC_BF16 && din % 8 == 0 && dout % 8 == 0 && split_shape(T) &&
-         B <= kSplitTailMaxB && ((size_t)T + kGramTile) * dmax * 2 < ((size_t)1 << 31) &&
+  return gram_mfma_shape(T, din, dout, dtype) && split_shape(T) && B <= kSplitTailMaxB &&
          np * DPC_GRAM_REC_WORDS <= lds_doubles && (size_t)B <= 2 * lds_doubles;
 }
 }  // namespace
@@ -2805,7 +2823,7 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   tail.job = job;
   if (with_bias) {
     tail.n_slots = min(kBiasSlots, ceil_div(dout, kBiasCols));
-    double* slots = (double*)(base + gram_bias_slots_offset(B, T));
+    double* slots = (double*)(base + gram_slots_at(B, T, false));
     tail.bias = slots;
     r = launch_bias_sqnorm(G, B, T, dout, dtype, tail.n_slots, slots, counters,
                            (int)(dpc_gram_clip_counter_bytes(B, T) / sizeof(int32_t)), s);

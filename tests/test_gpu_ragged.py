@@ -217,6 +217,22 @@ def test_gram_f64(dev, dtype, B, T, din, dout):
     assert (err <= 1.001 * (gammas + (T * T + 256) * 2.0**-52) * rows).all()
 
 
+# Layers in one call, layer by layer off the bf16 MFMA path: FMA kernel, 32- and
+# 64-row tiles, each as in the layer's own call.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T", [(16, 256), (6, 200), (3, 1100)])
+def test_gram_multi_matches_consecutive_calls(dev, dtype, B, T):
+    g = torch.Generator().manual_seed(B + T)
+    dims = [(65, 33), (9, 20), (260, 516), (100, 601)]
+    As = [torch.randn(B, T, din, generator=g).to(dtype).to(dev) for din, _ in dims]
+    Gs = [torch.randn(B, T, dout, generator=g).to(dtype).to(dev) for _, dout in dims]
+    want, want_err = ops.gram_sqnorms(As[0], Gs[0], return_error=True)
+    for a, x in zip(As[1:], Gs[1:]):
+        ops.gram_sqnorms(a, x, out=want, err=want_err)
+    got, err = ops.gram_sqnorms_multi(As, Gs, return_error=True)
+    assert torch.equal(got, want) and torch.equal(err, want_err)
+
+
 def _kernels(fn):
     fn()
     torch.cuda.synchronize()
