@@ -86,11 +86,14 @@ int dpc_write_words(void* dst, const uint32_t* host_words, int n, void* stream);
  * rounding or truncation of at most one fp32 ulp per addend of an MFMA
  * instruction, and flushed subnormals; generic path: fp64) and the fp64
  * inner product.  A layer bias adds ||sum_t G_i[t]||^2 (and its bound) when
- * with_bias != 0.  ws: dpc_gram_workspace_bytes(B, T) bytes; less is taken
- * down to the records of 64-row tiles, DPC_ENOSPC below that.  Examples whose A_i or G_i hold NaN/Inf produce a
+ * with_bias != 0.  ws: dpc_gram_workspace_bytes(B, T) bytes, enough for any
+ * layer, or dpc_gram_layer_workspace_bytes, what this layer uses (also in
+ * dpc_gram_clip_factors); less is taken down to the records of 64-row tiles,
+ * DPC_ENOSPC below that.  Examples whose A_i or G_i hold NaN/Inf produce a
  * non-finite value (their clip factor becomes 0).
  * -------------------------------------------------------------------------*/
 size_t dpc_gram_workspace_bytes(int B, int T);
+size_t dpc_gram_layer_workspace_bytes(int B, int T, int din, int dout, int dtype, int with_bias);
 int dpc_gram_sqnorms(const void* A, const void* G, int B, int T, int din, int dout, int dtype,
                      int with_bias, int accumulate, double* sqnorm, double* sqerr, void* ws,
                      size_t ws_bytes, void* stream);

@@ -53,6 +53,7 @@ SIGNATURES = {
     "dpc_last_error": (ctypes.c_char_p, []),
     "dpc_write_words": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p]),
     "dpc_gram_workspace_bytes": (_c_size_t, [_c_int, _c_int]),
+    "dpc_gram_layer_workspace_bytes": (_c_size_t, [_c_int] * 6),
     "dpc_gram_sqnorms": (
         _c_int,
         [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,

@@ -2256,8 +2256,8 @@ static F64Route gram_f64_route(int B, int T, int din, int dout, int dtype) {
   return pairs <= 128 || hi >= depth ? F64Route::kMfma32 : F64Route::kMfma64;
 }
 
-// The smallest workspace dpc_gram_sqnorms takes.  What dpc_gram_workspace_bytes
-// adds: the records of 32-row tiles of the fp64 path (in place of the 64-row
+// The smallest workspace dpc_gram_sqnorms takes.  What the workspace queries
+// add: the records of 32-row tiles of the fp64 path (in place of the 64-row
 // ones; without the room that path keeps 64-row tiles), and kBiasSlots words
 // per example (a bias norm's columns shared by several workgroups per
 // example, without them by one).
@@ -2742,10 +2742,26 @@ extern "C" size_t dpc_gram_clip_counter_bytes(int B, int T) {
   return (size_t)(3 * (size_t)B * nsets + (size_t)B + 1) * sizeof(int32_t);
 }
 
-// The norms' workspace and a biased layer's own counters.
+// A biased layer's own counters (see dpc_gram_clip_factors): after the bias words
+// of a layer on the MFMA path.
+static size_t gram_bias_counters_at(int B, int T) {
+  return align256(gram_slots_at(B, T, false) + (size_t)B * kBiasSlots * sizeof(double));
+}
+
 extern "C" size_t dpc_gram_clip_workspace_bytes(int B, int T) {
   if (B <= 0 || T <= 0) return 0;
-  return align256(dpc_gram_workspace_bytes(B, T)) + dpc_gram_clip_counter_bytes(B, T);
+  const size_t norms = dpc_gram_workspace_bytes(B, T);
+  const size_t bias = gram_bias_counters_at(B, T) + dpc_gram_clip_counter_bytes(B, T);
+  return norms > bias ? norms : bias;
+}
+
+extern "C" size_t dpc_gram_layer_workspace_bytes(int B, int T, int din, int dout, int dtype,
+                                                 int with_bias) {
+  if (B <= 0 || T <= 0 || din <= 0 || dout <= 0) return 0;
+  if (with_bias && gram_clip_one_launch(B, T, din, dout, dtype))
+    return gram_bias_counters_at(B, T) + dpc_gram_clip_counter_bytes(B, T);
+  return gram_layer_bytes(B, T, din, dout, dtype) +
+         (with_bias ? (size_t)B * kBiasSlots * sizeof(double) : 0);
 }
 
 extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din,
@@ -2773,7 +2789,9 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   // workspace holds its column norms and the counters, which the column norms'
   // launch clears: a biased call does not touch the caller's counter buffer, so
   // it may overlap with a call that uses it.
-  const bool bias_fits = !with_bias || ws_bytes >= dpc_gram_clip_workspace_bytes(B, T);
+  const size_t counters_at = gram_bias_counters_at(B, T);
+  const bool bias_fits =
+      !with_bias || ws_bytes >= counters_at + dpc_gram_clip_counter_bytes(B, T);
   if (!gram_clip_one_launch(B, T, din, dout, dtype) || !bias_fits) {
     // The norms, then (in their last launch, for a small batch) the clip
     // factors; the counters are not used.
@@ -2787,7 +2805,7 @@ extern "C" int dpc_gram_clip_factors(const void* A, const void* G, int B, int T,
   }
   uint8_t* base = (uint8_t*)ws;
   if (with_bias) {
-    counters = (int32_t*)(base + align256(dpc_gram_workspace_bytes(B, T)));
+    counters = (int32_t*)(base + counters_at);
   } else {
     if (!counters) return DPC_EINVAL;
     if (counter_bytes < dpc_gram_clip_counter_bytes(B, T)) return DPC_ENOSPC;

@@ -88,7 +88,8 @@ def gram_sqnorms(
     if with_err:
         err = _error_out(err, B, dev, accumulate)
     if B > 0:
-        ws_bytes = nat.load().dpc_gram_workspace_bytes(B, T)
+        ws_bytes = nat.load().dpc_gram_layer_workspace_bytes(
+            B, T, din, dout, nat.dtype_code(A.dtype), int(with_bias))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         nat.call(
             "dpc_gram_sqnorms", nat.ptr(A), nat.ptr(G), B, T, din, dout,
@@ -382,7 +383,8 @@ def gram_clip_factors(
     if B > 0:
         stream = nat.stream_handle(dev)
         lib = nat.load()
-        ws_bytes = lib.dpc_gram_clip_workspace_bytes(B, T)
+        ws_bytes = lib.dpc_gram_layer_workspace_bytes(
+            B, T, din, dout, nat.dtype_code(A.dtype), int(with_bias))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         counters = _gram_clip_counters(dev, stream, lib.dpc_gram_clip_counter_bytes(B, T))
         nat.call(

@@ -44,6 +44,40 @@ def test_version_and_size_queries():
     assert lib.dpc_gram_workspace_bytes(2, 128) > 0
 
 
+def test_gram_workspace_of_a_layer():
+    """Only layers off the bf16 MFMA path are given records of 32-row tile pairs (12
+    float64 words each): the others keep to those of 64 rows, and two words an example."""
+    if not _native.LIB_PATH.exists():
+        pytest.skip("native library not built")
+    lib = _native.load()
+
+    def query(B, T, din, dout, dtype, bias=0):
+        return lib.dpc_gram_layer_workspace_bytes(B, T, din, dout, dtype, bias)
+
+    def records(B, T, rows):
+        n = -(-T // rows)
+        return n * (n + 1) // 2 * B * 96
+
+    def up(n):
+        return -(-n // 256) * 256
+
+    f32, bf16 = _native.DPC_F32, _native.DPC_BF16
+    for B, T in ((8, 300), (4, 4160), (2, 32640)):  # odd numbers of 128-row blocks
+        assert query(B, T, 4096, 4096, bf16) == up(records(B, T, 64) + 16 * B)
+        assert query(B, T, 4096, 4096, bf16, 1) == up(records(B, T, 64) + 16 * B) + 256 * B
+    assert query(8, 300, 4096, 4096, f32) == up(records(8, 300, 32))
+    assert query(8, 300, 4095, 4096, bf16) == up(records(8, 300, 32))
+    assert query(8, 4160, 4096, 4096, f32) == up(records(8, 4160, 64) + 128)
+    # A biased layer of the one-launch path also holds its counters.
+    assert (query(6, 256, 128, 264, bf16, 1)
+            == up(query(6, 256, 128, 264, bf16) + 6 * 256) + lib.dpc_gram_clip_counter_bytes(6, 256))
+    # The queries without a layer hold any of them.
+    for B, T, din, dout, dtype, bias in ((6, 256, 128, 264, bf16, 1), (8, 300, 4096, 4096, f32, 1),
+                                         (8, 4160, 33, 9, bf16, 1), (1, 70, 8, 8, f32, 0)):
+        assert query(B, T, din, dout, dtype, bias) <= lib.dpc_gram_clip_workspace_bytes(B, T)
+        assert query(B, T, din, dout, dtype) <= lib.dpc_gram_workspace_bytes(B, T)
+
+
 def test_tables_used_under_keep_alive_survive_eviction():
     # A graph owner holds the tables its capture used: filling the content
     # cache past its bound afterwards evicts the cache's entries but not the
