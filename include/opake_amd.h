@@ -239,9 +239,15 @@ int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, i
  * z comes from `noise` (float32 [dout, din], mode INJECTED; bit-exact with a
  * host-drawn tensor) or from the Philox stream (mode PHILOX) keyed by
  * (seed, leaf_id).  `plan` is the dpc_clip_factors plan built from the same
- * `scale` (nullable: bf16 layers of 1.5 GFLOP and more then take the generic kernel,
- * which scans every example).  On the bf16 MFMA path (T > 1; widths that are
- * not multiples of 8 are copied into padded rows in ws) the products of
+ * `scale` (nullable).  The kernel goes by type, size and what is given:
+ *   fp32 MFMA   widths of at least 4; fp32, and bf16 of one token per example or of
+ *               less than 1.5 GFLOP (2 B T din dout);
+ *   bf16 MFMA   other bf16 layers of T > 1 with a plan; widths that are not
+ *               multiples of 8 are copied into padded rows in ws;
+ *   generic     (4 x 4 FMA blocks) the rest, fp32 layers whose K slices and bf16
+ *               layers whose padded copies ws is too small for.
+ * With ws NULL and a plan, bf16 layers of T > 1 and widths that are multiples of 8
+ * take the bf16 MFMA kernel at any size.  On that kernel the products of
  * the given bf16 values are summed in fp32 and each example's scale is
  * applied to the fp32 accumulators (the plan's first list); examples of the
  * plan's second list have G multiplied by the power of two of their scale
@@ -250,9 +256,8 @@ int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, i
  * sum_i scale[i] * sum_t G[i, t, m], its noise keyed by (seed, bias_leaf_id)
  * under the [dout, 1] view.  ws (dpc_clipped_sum_workspace_bytes) holds the
  * bias partials, the padded operand copies and, for layers of few output
- * tiles, the fp32 K-slices of a split-K launch (summed in a fixed order); with
- * a smaller ws (or none, without bias) the layer takes one pass or the generic
- * kernel.
+ * tiles, the fp32 K-slices of a split-K launch (summed in a fixed order; on the
+ * bf16 MFMA kernel a smaller ws takes one pass).
  * -------------------------------------------------------------------------*/
 size_t dpc_clipped_sum_workspace_bytes(int B, int T, int din, int dout, int dtype);
 int dpc_clipped_sum(const void* A, const void* G, const float* scale, const void* plan, int B,

@@ -1225,9 +1225,10 @@ int fast_splits(int B, int T, int din, int dout) {
 
 #undef DPC_WAIT_VMCNT
 
-// Generic path (calls without the workspace of the paths above and below, or
-// of widths below 4): any T, float32 or bf16 operands; 64 x 64 tiles with a 4 x 4
-// FMA block per thread.  K is walked in chunks of at most 16 rows that never
+// Generic path (float32 and one-token bf16 layers of widths below 4, larger bf16
+// layers without a plan or past the bf16 kernel's buffer offsets, and layers whose
+// workspace does not hold the K slices or padded copies of the paths above and
+// below): any T; 64 x 64 tiles with a 4 x 4 FMA block per thread.  K is walked in chunks of at most 16 rows that never
 // straddle two examples: G is staged multiplied by the power of two of its
 // example's scale (exact) and the accumulators carry the mantissa (they hold
 // the partial sum divided by the current mantissa, rescaled where it
@@ -2065,7 +2066,10 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
   const size_t pad_a = pad_bytes(B, T, din), pad_g = pad_bytes(B, T, dout);
   const size_t pad_at = bias_ws_bytes(dout), split_at = pad_at + pad_a + pad_g;
   const size_t f32_ws = f32_bytes(B, T, din, dout);
-  const bool f32 = f32_shape(B, T, din, dout, dtype) &&
+  // Without a workspace a layer that the bf16 kernel takes as it is stays there
+  // at any size: a layer of dpc_clipped_sum_multi's shared launch, bit for bit.
+  const bool as_shared = !ws && plan && pad_a + pad_g == 0 && fast_shape(B, T, din, dout, dtype);
+  const bool f32 = !as_shared && f32_shape(B, T, din, dout, dtype) &&
                    (f32_ws == 0 || (ws && ws_bytes >= pad_at + f32_ws));
   const bool fast =
       !f32 && fast_shape(B, T, din, dout, dtype) && plan != nullptr &&

@@ -481,8 +481,10 @@ def clipped_sum_multi(
     layer i's noise (None: none); the specs must share one mode and seed.
     Returns one [dout, din] tensor per layer.  When every layer takes the
     MFMA path (bf16, T > 1, widths % 8 == 0, a plan) and their tiles fill
-    launches, each result equals its own ``clipped_sum`` call without a split-K
-    workspace; otherwise the layers run as their own ``clipped_sum`` calls."""
+    launches, each result equals its own ``dpc_clipped_sum`` call without a
+    workspace (``clipped_sum``, which gives one, may take another kernel and
+    split K: equal up to the order of fp32 sums); otherwise the layers run as
+    their own ``clipped_sum`` calls."""
     n = len(A_list)
     if n == 0 or len(G_list) != n:
         raise ConfigurationError("expected matching, non-empty lists of A and G")

@@ -3,6 +3,8 @@ widths that are not multiples of 8 (GPU tests, called through the C ABI)."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -113,6 +115,38 @@ def test_clipped_sum_multi_ragged_matches_single_layers(dev):
         assert torch.equal(w, ops.clipped_sum_multi([As[i]], [Gs[i]], cf.scale[0], **kw)[0])
         want = _exact(*ops_[i], cf.scale[0].cpu().double())
         assert _rel(w.cpu(), want) < 1e-5
+
+
+# One call for several layers and each layer's own call without a workspace:
+# small layers and large ones, more tiles than CUs, full and ragged steps; padded
+# widths, one token and float32 go layer by layer.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,dims", [
+    (3, 128, [(256, 264), (8, 8), (64, 520)]), (3, 70, [(256, 264), (8, 8), (4104, 264)]),
+    (2, 64, [(4096, 2304), (520, 2304), (2304, 2304)]), (3, 70, [(256, 264), (33, 8)]),
+    (40, 1, [(256, 264), (8, 8)])])
+def test_clipped_sum_multi_equals_calls_without_a_workspace(dev, dtype, B, T, dims):
+    pairs = [_operands(B, T, din, dout, din + dout) for din, dout in dims]
+    As, Gs = [a.to(dev, dtype) for a, _ in pairs], [g.to(dev, dtype) for _, g in pairs]
+    sq = (4 * torch.rand(B, dtype=torch.float64, generator=torch.Generator().manual_seed(B))).to(dev)
+    cf = ops.clip_factors(sq, 1.0, [guard_for_linear(dtype, *dims[0], False)], count_threshold=1.0)
+    n, code, seed = len(dims), nat.dtype_code(dtype), 77
+    outs = [torch.empty(dout, din, device=dev) for din, dout in dims]
+    vp, ci = ctypes.c_void_p * n, ctypes.c_int * n
+    sigmas, leaves = [0.0] + [0.25] * (n - 1), list(range(n))
+    nat.call("dpc_clipped_sum_multi", n, vp(*[a.data_ptr() for a in As]),
+             vp(*[g.data_ptr() for g in Gs]), ci(*[d[0] for d in dims]), ci(*[d[1] for d in dims]),
+             nat.ptr(cf.scale[0]), nat.ptr(cf.plan[0]), B, T, code, 2.0, nat.NOISE_PHILOX, None,
+             seed, (ctypes.c_uint32 * n)(*leaves), (ctypes.c_double * n)(*sigmas),
+             nat.dtype_code(torch.float32), vp(*[o.data_ptr() for o in outs]),
+             nat.stream_handle(dev))
+    for a, g, out, sigma, leaf in zip(As, Gs, outs, sigmas, leaves):
+        one = torch.empty_like(out)
+        nat.call("dpc_clipped_sum", nat.ptr(a), nat.ptr(g), nat.ptr(cf.scale[0]),
+                 nat.ptr(cf.plan[0]), B, T, a.shape[2], g.shape[2], code, 2.0, nat.NOISE_PHILOX,
+                 None, None, seed, leaf, 0, sigma, nat.dtype_code(torch.float32), nat.ptr(one), 0,
+                 None, None, 0, nat.stream_handle(dev))
+        assert torch.equal(out, one)
 
 
 # Row groups of the bias column sums: fewer rows than groups, one more than a
