@@ -86,7 +86,9 @@ int dpc_write_words(void* dst, const uint32_t* host_words, int n, void* stream);
  * rounding or truncation of at most one fp32 ulp per addend of an MFMA
  * instruction, and flushed subnormals; generic path: fp64) and the fp64
  * inner product.  A layer bias adds ||sum_t G_i[t]||^2 (and its bound) when
- * with_bias != 0.  ws: dpc_gram_workspace_bytes(B, T) bytes, enough for any
+ * with_bias != 0.  bf16 operands of widths that are multiples of 8 start at a
+ * 16-byte boundary (the package copies views that do not; so for the grouped
+ * norms and sums).  ws: dpc_gram_workspace_bytes(B, T) bytes, enough for any
  * layer, or dpc_gram_layer_workspace_bytes, what this layer uses (also in
  * dpc_gram_clip_factors); less is taken down to the records of 64-row tiles,
  * DPC_ENOSPC below that.  Examples whose A_i or G_i hold NaN/Inf produce a
@@ -246,6 +248,8 @@ int dpc_gram_clip_factors(const void* A, const void* G, int B, int T, int din, i
  *               multiples of 8 are copied into padded rows in ws;
  *   generic     (4 x 4 FMA blocks) the rest, fp32 layers whose K slices and bf16
  *               layers whose padded copies ws is too small for.
+ * bf16 operands of widths that are multiples of 8 but that do not start at a
+ * 16-byte boundary take the fp32 MFMA kernel (unsplit where ws is too small).
  * With ws NULL and a plan, bf16 layers of T > 1 and widths that are multiples of 8
  * take the bf16 MFMA kernel at any size.  On that kernel the products of
  * the given bf16 values are summed in fp32 and each example's scale is

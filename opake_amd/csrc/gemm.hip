@@ -1643,8 +1643,11 @@ __global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args<In
 // 24 and 26, 16, 100, 1023, 511 (1.7) 33 and 38, but 32, 100, 768, 768 (3.8) 66
 // and 35; 256 tokens of one example each, 512 x 512, 18, and 1024 of 2048 x 2048
 // 101 (15 and 580 in the generic kernel).
+bool f32_widths(int B, int din, int dout) {
+  return B > 0 && din >= 4 && dout >= 4 && din < (1 << 26) && dout < (1 << 26);
+}
 bool f32_shape(int B, int T, int din, int dout, int dtype) {
-  if (B <= 0 || din < 4 || dout < 4 || din >= (1 << 26) || dout >= (1 << 26)) return false;
+  if (!f32_widths(B, din, dout)) return false;
   if (dtype == DPC_F32 || T == 1) return true;
   return 2.0 * B * T * (double)din * dout < kF32MaxBf16Flops;
 }
@@ -1940,6 +1943,7 @@ bool fast_shape(int B, int T, int din, int dout, int dtype) {
 size_t pad_bytes(int B, int T, int d) {
   return d % 8 == 0 ? 0 : align256((size_t)B * (size_t)T * (size_t)padded_width(d) * 2);
 }
+bool starts_at_16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 bool split_planes(int splits, int din) { return splits > 1 || din % 2 != 0; }
 size_t split_bytes(int splits, int din, int dout) {
   if (!split_planes(splits, din)) return 0;
@@ -2066,13 +2070,20 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
   const size_t pad_a = pad_bytes(B, T, din), pad_g = pad_bytes(B, T, dout);
   const size_t pad_at = bias_ws_bytes(dout), split_at = pad_at + pad_a + pad_g;
   const size_t f32_ws = f32_bytes(B, T, din, dout);
+  const bool f32_fits = f32_ws == 0 || (ws && ws_bytes >= pad_at + f32_ws);
+  // The bf16 kernel's transfers are of 16 aligned bytes: operands that start
+  // elsewhere and are not copied go to the fp32 kernel, which loads at any element
+  // boundary, unsplit where ws does not hold its slices.
+  const bool off16 =
+      dtype == DPC_BF16 && ((pad_a == 0 && !starts_at_16(A)) || (pad_g == 0 && !starts_at_16(G)));
   // Without a workspace a layer that the bf16 kernel takes as it is stays there
   // at any size: a layer of dpc_clipped_sum_multi's shared launch, bit for bit.
-  const bool as_shared = !ws && plan && pad_a + pad_g == 0 && fast_shape(B, T, din, dout, dtype);
-  const bool f32 = !as_shared && f32_shape(B, T, din, dout, dtype) &&
-                   (f32_ws == 0 || (ws && ws_bytes >= pad_at + f32_ws));
+  const bool as_shared =
+      !ws && plan && !off16 && pad_a + pad_g == 0 && fast_shape(B, T, din, dout, dtype);
+  const bool f32 = off16 ? f32_widths(B, din, dout)
+                         : !as_shared && f32_shape(B, T, din, dout, dtype) && f32_fits;
   const bool fast =
-      !f32 && fast_shape(B, T, din, dout, dtype) && plan != nullptr &&
+      !f32 && !off16 && fast_shape(B, T, din, dout, dtype) && plan != nullptr &&
       (pad_a + pad_g == 0 || (ws && ws_bytes >= split_at + split_bytes(1, din, dout)));
   if (fast) {
     const long long rows = (long long)B * T;
@@ -2115,7 +2126,7 @@ extern "C" int dpc_clipped_sum(const void* A, const void* G, const float* scale,
       bias.blocks = 0;
     }
   } else if (f32) {
-    const int splits = f32_splits(B, T, din, dout);
+    const int splits = f32_fits ? f32_splits(B, T, din, dout) : 1;
     const int prows = f32_plane_rows(dout), pld = f32_plane_ld(din);
     float* partial = splits > 1 ? (float*)((uint8_t*)ws + pad_at) : nullptr;
     const long long blocks =
@@ -2215,7 +2226,8 @@ extern "C" int dpc_clipped_sum_multi(int n, const void* const* A, const void* co
     if (sigmas[i] != 0.0 && noise_mode == DPC_NOISE_NONE) return DPC_EINVAL;
     if (sigmas[i] != 0.0 && noise_mode == DPC_NOISE_INJECTED && (!noise || !noise[i]))
       return DPC_EINVAL;
-    fast = fast && fast_shape(B, T, din[i], dout[i], dtype) && din[i] % 8 == 0 && dout[i] % 8 == 0;
+    fast = fast && fast_shape(B, T, din[i], dout[i], dtype) && din[i] % 8 == 0 &&
+           dout[i] % 8 == 0 && starts_at_16(A[i]) && starts_at_16(G[i]);
   }
   hipStream_t s = (hipStream_t)stream;
   if (!fast) {

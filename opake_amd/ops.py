@@ -23,6 +23,22 @@ def _contig(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous and 16-byte aligned (kernels that read rows with aligned vector
+    loads)."""
+    if t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
+def _operand(t: torch.Tensor) -> torch.Tensor:
+    """A layer's activations or output gradients, contiguous; bfloat16 rows of
+    whole 16-byte chunks, which the MFMA kernels move as such, start at one."""
+    if t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0:
+        return _aligned(t)
+    return _contig(t)
+
+
 def _wants_error(out, err, return_error):
     """Whether a norm call writes its error bound.  Accumulating into ``out``
     without ``err`` drops the bound of the sum (``out + err`` would no longer
@@ -78,7 +94,7 @@ def gram_sqnorms(
         raise ConfigurationError("A and G must share a dtype")
     B, T, din = A.shape
     dout = G.shape[2]
-    A, G = _contig(A), _contig(G)
+    A, G = _operand(A), _operand(G)
     accumulate = out is not None
     with_err = _wants_error(out, err, return_error)
     if out is None:
@@ -132,8 +148,8 @@ def gram_sqnorms_multi(
     if with_err:
         err = _error_out(err, B, dev, accumulate)
     if B > 0:
-        As = [_contig(A) for A in A_list]
-        Gs = [_contig(G) for G in G_list]
+        As = [_operand(A) for A in A_list]
+        Gs = [_operand(G) for G in G_list]
         c_din = (ctypes.c_int * n)(*[A.shape[2] for A in As])
         c_dout = (ctypes.c_int * n)(*[G.shape[2] for G in Gs])
         ws_bytes = nat.load().dpc_gram_sqnorms_multi_workspace_bytes(
@@ -372,7 +388,7 @@ def gram_clip_factors(
         return sq, err, cf
     B, T, din = A.shape
     dout = G.shape[2]
-    A, G = _contig(A), _contig(G)
+    A, G = _operand(A), _operand(G)
     n = len(guards)
     rel = (ctypes.c_double * n)(*[g[0] for g in guards])
     abs_ = (ctypes.c_double * n)(*[g[1] for g in guards])
@@ -440,7 +456,7 @@ def clipped_sum(
     if scale.dtype != torch.float32 or scale.numel() < B:
         raise ConfigurationError("scale must be float32 with B entries")
     out_dtype = out_dtype or A.dtype
-    A, G = _contig(A), _contig(G)
+    A, G = _operand(A), _operand(G)
     out = torch.empty((dout, din), dtype=out_dtype, device=dev)
     bias_out = torch.empty(dout, dtype=out_dtype, device=dev) if with_bias else None
     ws_bytes = nat.load().dpc_clipped_sum_workspace_bytes(B, T, din, dout, nat.dtype_code(A.dtype))
@@ -530,8 +546,8 @@ def clipped_sum_multi(
     if not mfma:
         return [clipped_sum(A, G, scale, plan=plan, normalize_by=normalize_by, noise=sp,
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]
-    As = [_contig(A) for A in A_list]
-    Gs = [_contig(G) for G in G_list]
+    As = [_operand(A) for A in A_list]
+    Gs = [_operand(G) for G in G_list]
     dins = [A.shape[2] for A in As]
     douts = [G.shape[2] for G in Gs]
     outs = [torch.empty((o, i), dtype=out_dtype, device=dev) for i, o in zip(dins, douts)]
@@ -803,6 +819,7 @@ def grouped_gram_sqnorms(A_list, G_list, layout: SegmentLayout, *, return_error:
         raise ConfigurationError("at most 64 problems per grouped Gram call")
     if not layout.has_gram:
         raise ConfigurationError("the layout was built without its Gram schedules (gram=False)")
+    A_list, G_list = [_operand(A) for A in A_list], [_operand(G) for G in G_list]
     dims = (ctypes.c_int * (2 * layout.E))(
         *[v for A, G in zip(A_list, G_list) for v in (A.shape[1], G.shape[1])])
     seg_sq = torch.empty((layout.E, layout.K), dtype=torch.float64, device=dev)
@@ -867,6 +884,7 @@ def grouped_clipped_sum(
     if seg_scale.dtype != torch.float32 or tuple(seg_scale.shape) != (layout.E, layout.K):
         raise ConfigurationError("seg_scale must be float32 [E, K]")
     seg_scale = _contig(seg_scale)
+    A_list, G_list = [_operand(A) for A in A_list], [_operand(G) for G in G_list]
     out_dtype = out_dtype or dtype
     E = layout.E
     out = torch.empty((E, dout, din), dtype=out_dtype, device=dev)
@@ -928,25 +946,13 @@ def per_example_grads(A: torch.Tensor, G: torch.Tensor, *,
     out = torch.empty((B, dout, din), dtype=out_dtype, device=dev)
     if B == 0:
         return out
-    # The kernel reads rows with aligned vector loads.
-    A = A.contiguous() if (A.is_contiguous() and A.data_ptr() % 16 == 0) else A.clone(
-        memory_format=torch.contiguous_format)
-    G = G.contiguous() if (G.is_contiguous() and G.data_ptr() % 16 == 0) else G.clone(
-        memory_format=torch.contiguous_format)
+    A, G = _aligned(A), _aligned(G)
     ws_bytes = nat.load().dpc_per_example_grads_workspace_bytes(B, T, din, dout)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     nat.call("dpc_per_example_grads", nat.ptr(A), nat.ptr(G), B, T, din, dout,
              nat.dtype_code(A.dtype), nat.ptr(out), nat.dtype_code(out_dtype), nat.ptr(ws),
              ws_bytes, nat.stream_handle(dev))
     return out
-
-
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    """Contiguous and 16-byte aligned (the kernels read rows with aligned
-    vector loads)."""
-    if t.is_contiguous() and t.data_ptr() % 16 == 0:
-        return t
-    return t.clone(memory_format=torch.contiguous_format)
 
 
 def per_example_grads_grouped(A_list, G_list, *,

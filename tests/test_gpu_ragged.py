@@ -149,6 +149,69 @@ def test_clipped_sum_multi_equals_calls_without_a_workspace(dev, dtype, B, T, di
         assert torch.equal(out, one)
 
 
+def _in_flat_buffer(t, first):
+    """``t`` as a view of a flat buffer from element `first` on."""
+    flat = torch.empty(t.numel() + first, dtype=t.dtype, device=t.device)
+    view = flat[first:].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+# Views that start 2, 4 and 8 bytes past a 16-byte boundary: small and large
+# layers, full and ragged steps, padded widths, one token, a bias; each operand.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,din,dout", [(3, 70, 64, 72), (24, 97, 520, 640), (24, 128, 520, 640),
+                                          (16, 100, 1023, 511), (40, 1, 64, 72), (8, 256, 64, 136)])
+def test_operands_at_any_element(dev, dtype, B, T, din, dout):
+    A, G = (x.to(dtype) for x in _operands(B, T, din, dout, B + T))
+    A_d, G_d = A.to(dev), G.to(dev)
+    guards = [guard_for_linear(dtype, din, dout, True)]
+
+    def outputs(a, g):
+        sq, err, cf = ops.gram_clip_factors(a, g, 1.0, guards, with_bias=True, count_threshold=1.0)
+        kw = dict(plan=cf.plan[0], out_dtype=torch.float32)
+        w, b = ops.clipped_sum(a, g, cf.scale[0], with_bias=True, **kw)
+        lay = ops.SegmentLayout([[T] * B], dev)
+        flat = [a.view(B * T, din)], [g.view(B * T, dout)], lay
+        return [sq, err, cf.scale, w, b, *ops.gram_sqnorms(a, g, with_bias=True, return_error=True),
+                *ops.gram_sqnorms_multi([a, a], [g, g], return_error=True),
+                *ops.clipped_sum_multi([a, a], [g, g], cf.scale[0], **kw),
+                *ops.grouped_gram_sqnorms(*flat, return_error=True),
+                ops.grouped_clipped_sum(*flat, cf.scale[:1], out_dtype=torch.float32)]
+
+    want = outputs(A_d, G_d)
+    # Copied to the boundary: the same bits.  Else the bias columns are summed in other
+    # row groups, T addends in fp32, and the clip factor follows.
+    rtol = 0 if dtype == torch.bfloat16 and din % 8 == 0 else T * 2.0**-23
+    for fa, fg in ((1, 0), (0, 2), (4, 1)):
+        a, g = _in_flat_buffer(A_d, fa), _in_flat_buffer(G_d, fg)
+        for x, y in zip(outputs(a, g), want):
+            torch.testing.assert_close(x, y, rtol=rtol, atol=rtol * float(y.abs().max()))
+    # The C entry points take them as they are.
+    cf = ops.clip_factors(want[0], 1.0, guards, err=want[1], count_threshold=1.0)
+    lib, code, f32 = nat.load(), nat.dtype_code(dtype), nat.dtype_code(torch.float32)
+    a, g = _in_flat_buffer(A_d, 1), _in_flat_buffer(G_d, 1)
+    exact = _exact(A, G, cf.scale[0].cpu().double())
+    full = lib.dpc_clipped_sum_workspace_bytes(B, T, din, dout, code)
+    for ws_bytes in (full, 0):
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        for plan in (cf.plan[0], None):
+            w = torch.empty(dout, din, device=dev)
+            nat.call("dpc_clipped_sum", nat.ptr(a), nat.ptr(g), nat.ptr(cf.scale[0]), nat.ptr(plan),
+                     B, T, din, dout, code, 1.0, nat.NOISE_NONE, None, None, 0, 0, 0, 0.0, f32,
+                     nat.ptr(w), 0, None, nat.ptr(ws), ws_bytes, nat.stream_handle(dev))
+            assert _rel(w.cpu(), exact) < 1e-5
+    outs = [torch.empty(dout, din, device=dev) for _ in range(2)]
+    vp, ci = ctypes.c_void_p * 2, ctypes.c_int * 2
+    nat.call("dpc_clipped_sum_multi", 2, vp(A_d.data_ptr(), a.data_ptr()),
+             vp(G_d.data_ptr(), g.data_ptr()), ci(din, din), ci(dout, dout),
+             nat.ptr(cf.scale[0]), nat.ptr(cf.plan[0]), B, T, code, 1.0, nat.NOISE_NONE, None, 0,
+             None, (ctypes.c_double * 2)(), f32, vp(*[o.data_ptr() for o in outs]),
+             nat.stream_handle(dev))
+    for w in outs:
+        assert _rel(w.cpu(), exact) < 1e-5
+
+
 # Row groups of the bias column sums: fewer rows than groups, one more than a
 # full turn of them, the unrolled part and its remainder; 16-byte rows and
 # rows of any alignment; one and several column blocks and slots, and a
