@@ -1932,8 +1932,12 @@ size_t bias_ws_bytes(int dout) {
 }
 int padded_width(int d) { return (d + 7) & ~7; }
 // The bf16 MFMA path: any T of at least two tokens (T % 64 != 0: the ragged
-// body; its out-of-range offset must lie past the operands).
+// body; its out-of-range offset must lie past the operands); odd output rows
+// that the launch of split_reduce_kernel, which finishes them, covers (less than
+// 2^32 threads, some of them the bias's).
 bool fast_shape(int B, int T, int din, int dout, int dtype) {
+  if (din % 2 != 0 && (size_t)ceil_div(din, 2) * (size_t)ceil_div(dout, 2) >= (size_t)7 << 29)
+    return false;
   const size_t rows = (size_t)B * (size_t)T;
   const size_t limit = T % kBK == 0 ? (size_t)1 << 31 : (size_t)kOutOfRange;
   return dtype == DPC_BF16 && T > 1 && B > 0 &&

@@ -78,6 +78,19 @@ def test_gram_workspace_of_a_layer():
         assert query(B, T, din, dout, dtype) <= lib.dpc_gram_workspace_bytes(B, T)
 
 
+def test_clipped_sum_workspace_of_huge_odd_outputs():
+    """Odd output rows of the bf16 MFMA path are finished by a launch of a thread per 2 x 2
+    values: outputs of more than it covers (2^32 threads) keep to the generic path, which
+    needs no float32 plane of the output."""
+    if not _native.LIB_PATH.exists():
+        pytest.skip("native library not built")
+    lib = _native.load()
+    bias = 32 * 131072 * 4
+    assert lib.dpc_clipped_sum_workspace_bytes(2, 64, 131073, 131072, _native.DPC_BF16) == bias
+    plane = 131072 * 65544 * 4
+    assert lib.dpc_clipped_sum_workspace_bytes(2, 64, 65537, 131072, _native.DPC_BF16) > plane
+
+
 def test_tables_used_under_keep_alive_survive_eviction():
     # A graph owner holds the tables its capture used: filling the content
     # cache past its bound afterwards evicts the cache's entries but not the
