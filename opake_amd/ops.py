@@ -34,9 +34,11 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 def _operand(t: torch.Tensor) -> torch.Tensor:
     """A layer's activations or output gradients, contiguous; bfloat16 rows of
     whole 16-byte chunks, which the MFMA kernels move as such, start at one."""
-    if t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0:
-        return _aligned(t)
-    return _contig(t)
+    if not t.is_contiguous():
+        return t.contiguous()
+    if t.data_ptr() % 16 and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0:
+        return t.clone(memory_format=torch.contiguous_format)
+    return t
 
 
 def _wants_error(out, err, return_error):
@@ -104,13 +106,13 @@ def gram_sqnorms(
     if with_err:
         err = _error_out(err, B, dev, accumulate)
     if B > 0:
-        ws_bytes = nat.load().dpc_gram_layer_workspace_bytes(
-            B, T, din, dout, nat.dtype_code(A.dtype), int(with_bias))
+        code, bias = nat.dtype_code(A.dtype), int(with_bias)
+        ws_bytes = nat.load().dpc_gram_layer_workspace_bytes(B, T, din, dout, code, bias)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         nat.call(
-            "dpc_gram_sqnorms", nat.ptr(A), nat.ptr(G), B, T, din, dout,
-            nat.dtype_code(A.dtype), int(with_bias), int(accumulate), nat.ptr(out),
-            nat.ptr(err if with_err else None), nat.ptr(ws), ws_bytes, nat.stream_handle(dev),
+            "dpc_gram_sqnorms", nat.ptr(A), nat.ptr(G), B, T, din, dout, code, bias,
+            int(accumulate), nat.ptr(out), nat.ptr(err if with_err else None), nat.ptr(ws),
+            ws_bytes, nat.stream_handle(dev),
         )
     return (out, err) if with_err else out
 
@@ -399,13 +401,13 @@ def gram_clip_factors(
     if B > 0:
         stream = nat.stream_handle(dev)
         lib = nat.load()
-        ws_bytes = lib.dpc_gram_layer_workspace_bytes(
-            B, T, din, dout, nat.dtype_code(A.dtype), int(with_bias))
+        code, bias = nat.dtype_code(A.dtype), int(with_bias)
+        ws_bytes = lib.dpc_gram_layer_workspace_bytes(B, T, din, dout, code, bias)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         counters = _gram_clip_counters(dev, stream, lib.dpc_gram_clip_counter_bytes(B, T))
         nat.call(
-            "dpc_gram_clip_factors", nat.ptr(A), nat.ptr(G), B, T, din, dout,
-            nat.dtype_code(A.dtype), int(with_bias), float(clipping_norm), kind, float(gamma),
+            "dpc_gram_clip_factors", nat.ptr(A), nat.ptr(G), B, T, din, dout, code,
+            bias, float(clipping_norm), kind, float(gamma),
             rel, abs_, mult, n, float(count_threshold), nat.ptr(sq), nat.ptr(err),
             nat.ptr(cf.scale), nat.ptr(cf.scale64), nat.ptr(cf.norms), nat.ptr(cf.nclipped),
             nat.ptr(cf.plan), nat.ptr(nonfinite), nat.ptr(ws), ws_bytes, nat.ptr(counters),
@@ -526,9 +528,9 @@ def clipped_sum_multi(
     # The MFMA kernel's 32-bit buffer offsets (with T % 64 != 0 one of them
     # marks the rows past an example's end).
     limit = 2 ** 31 if T % 64 == 0 else 0x7FF00000
+    dins, douts = [A.shape[2] for A in A_list], [G.shape[2] for G in G_list]
     mfma = plan is not None and B > 0 and dtype == torch.bfloat16 and T > 1 and all(
-        A.shape[2] % 8 == 0 and G.shape[2] % 8 == 0
-        and B * T * max(A.shape[2], G.shape[2]) * 2 < limit for A, G in zip(A_list, G_list))
+        i % 8 == 0 and o % 8 == 0 and B * T * max(i, o) * 2 < limit for i, o in zip(dins, douts))
     # Layers of few output tiles (256 x 256) and a long K leave most CUs idle for
     # the whole of it in a shared launch, which does not split K. Their own calls
     # do, for some 25 us more a layer; a K step is about 1.6 us. A transformer
@@ -537,8 +539,9 @@ def clipped_sum_multi(
     # 82 tiles at [23, 640] (230) 614 -> 549 us and 96 tiles at [112, 100] (224)
     # 628 -> 558 us; width 384 at [22, 192] (66) would lose, 261 -> 319 us, and
     # stays shared.
-    tiles = sum(-(-A.shape[2] // 256) * -(-G.shape[2] // 256) for A, G in zip(A_list, G_list))
-    if mfma and n > 1 and tiles <= 96 and B * -(-T // 64) >= 32 * n:
+    steps = B * -(-T // 64)
+    if mfma and n > 1 and steps >= 32 * n and sum(
+            -(-i // 256) * -(-o // 256) for i, o in zip(dins, douts)) <= 96:
         mfma = False
         noises = [None if sp is None or sp.sigma == 0.0
                   else replace(sp, noise=None if sp.noise is None else _contig(sp.noise))
@@ -548,8 +551,6 @@ def clipped_sum_multi(
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]
     As = [_operand(A) for A in A_list]
     Gs = [_operand(G) for G in G_list]
-    dins = [A.shape[2] for A in As]
-    douts = [G.shape[2] for G in Gs]
     outs = [torch.empty((o, i), dtype=out_dtype, device=dev) for i, o in zip(dins, douts)]
     sig = [sp.sigma if sp is not None else 0.0 for sp in noises]
     zs = []
