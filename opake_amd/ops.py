@@ -538,15 +538,20 @@ def clipped_sum_multi(
     # 830 -> 490 us, width 512 at [24, 1000] (384) 989 -> 700 us; at the line,
     # 82 tiles at [23, 640] (230) 614 -> 549 us and 96 tiles at [112, 100] (224)
     # 628 -> 558 us; width 384 at [22, 192] (66) would lose, 261 -> 319 us, and
-    # stays shared.
+    # stays shared.  Layers of under 0.3 GFLOP take some 22 us each in their own
+    # calls (the fp32 kernel, in which a short example does not fill a 64-row
+    # step): 14 of 24 x 48 at [330, 6] (330 steps) 609 -> 306 us, of 16 x 2048
+    # 626 -> 350 us, 2 of 24 x 48 at [40, 6] (40) 51 -> 38 us; 7 of 24 x 48 at
+    # [110, 6] (110) would lose by a factor of 1.4.
     steps = B * -(-T // 64)
-    if mfma and n > 1 and steps >= 32 * n and sum(
-            -(-i // 256) * -(-o // 256) for i, o in zip(dins, douts)) <= 96:
-        mfma = False
+    if mfma and n > 1 and steps >= 16 * n:
+        small = all(2 * B * T * i * o < 3e8 for i, o in zip(dins, douts))
+        tiles = sum(-(-i // 256) * -(-o // 256) for i, o in zip(dins, douts))
+        mfma = not small and (tiles > 96 or steps < 32 * n)
+    if not mfma:
         noises = [None if sp is None or sp.sigma == 0.0
                   else replace(sp, noise=None if sp.noise is None else _contig(sp.noise))
                   for sp in noises]
-    if not mfma:
         return [clipped_sum(A, G, scale, plan=plan, normalize_by=normalize_by, noise=sp,
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]
     As = [_operand(A) for A in A_list]

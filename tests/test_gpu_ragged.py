@@ -473,6 +473,19 @@ def test_clipped_sum_multi_few_tiles_long_k(dev):
         assert _rel((w - noise).cpu(), _exact(*pair, cf.scale[0].cpu().double())) < 1e-5
 
 
+# Many short examples: a shared launch would walk a nearly empty 64-row step for each.
+@pytest.mark.parametrize("B,T,own", [(230, 6, True), (150, 6, False)])
+def test_short_examples_of_small_layers_take_their_own_calls(dev, B, T, own):
+    pairs = [_operands(B, T, 24, 48, i) for i in range(14)]
+    As, Gs = [a.to(dev) for a, _ in pairs], [g.to(dev) for _, g in pairs]
+    cf = _factors(dev, As[0], Gs[0])
+    kw = dict(plan=cf.plan[0], out_dtype=torch.float32)
+    names = _kernels(lambda: ops.clipped_sum_multi(As, Gs, cf.scale[0], **kw))
+    assert any("clipped_sum_bf16_kernel" in n for n in names) != own
+    for w, pair in zip(ops.clipped_sum_multi(As, Gs, cf.scale[0], **kw), pairs):
+        assert _rel(w.cpu(), _exact(*pair, cf.scale[0].cpu().double())) < 1e-5
+
+
 # bf16 tile pairs of 128 rows: 45 and 66 records an example.
 @pytest.mark.parametrize("B,T,one", [(32, 1152, True), (16, 1408, True), (32, 1408, False)])
 def test_one_workgroup_finishes_few_records_only(dev, B, T, one):
