@@ -792,6 +792,16 @@ def _ptr_table(tensors, device) -> torch.Tensor:
     return pointer_table(tensors, device)
 
 
+def _operand_table(tensors, device):
+    """The pointer table of grouped operands (already contiguous) and the tensors it
+    points into: copies of those that :func:`_operand` copies."""
+    ptrs = [t.data_ptr() for t in tensors]
+    if any(p % 16 for p in ptrs):
+        tensors = [_operand(t) for t in tensors]
+        ptrs = [t.data_ptr() for t in tensors]
+    return device_table(ptrs, np.int64, device), tensors
+
+
 def _check_grouped(A_list, G_list, layout: SegmentLayout, *, same_shape: bool):
     if len(A_list) != layout.E or len(G_list) != layout.E:
         raise ConfigurationError("one A and one G per problem of the layout are required")
@@ -825,7 +835,6 @@ def grouped_gram_sqnorms(A_list, G_list, layout: SegmentLayout, *, return_error:
         raise ConfigurationError("at most 64 problems per grouped Gram call")
     if not layout.has_gram:
         raise ConfigurationError("the layout was built without its Gram schedules (gram=False)")
-    A_list, G_list = [_operand(A) for A in A_list], [_operand(G) for G in G_list]
     dims = (ctypes.c_int * (2 * layout.E))(
         *[v for A, G in zip(A_list, G_list) for v in (A.shape[1], G.shape[1])])
     seg_sq = torch.empty((layout.E, layout.K), dtype=torch.float64, device=dev)
@@ -846,7 +855,7 @@ def grouped_gram_sqnorms(A_list, G_list, layout: SegmentLayout, *, return_error:
     n_records = layout.n_items
     nbytes = nat.load().dpc_grouped_gram_workspace_bytes(n_records, n_sets)
     ws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=dev)
-    a_ptrs, g_ptrs = _ptr_table(A_list, dev), _ptr_table(G_list, dev)
+    (a_ptrs, A_list), (g_ptrs, G_list) = _operand_table(A_list, dev), _operand_table(G_list, dev)
     nat.call(
         "dpc_grouped_gram_sqnorms", nat.ptr(a_ptrs), nat.ptr(g_ptrs), dims, layout.E,
         nat.dtype_code(dtype), nat.ptr(items), n_items, layout.max_rows, nat.ptr(sets),
@@ -890,7 +899,6 @@ def grouped_clipped_sum(
     if seg_scale.dtype != torch.float32 or tuple(seg_scale.shape) != (layout.E, layout.K):
         raise ConfigurationError("seg_scale must be float32 [E, K]")
     seg_scale = _contig(seg_scale)
-    A_list, G_list = [_operand(A) for A in A_list], [_operand(G) for G in G_list]
     out_dtype = out_dtype or dtype
     E = layout.E
     out = torch.empty((E, dout, din), dtype=out_dtype, device=dev)
@@ -921,7 +929,7 @@ def grouped_clipped_sum(
         raise ConfigurationError("one leaf id per problem is required")
     leaf_dev = device_table([v & 0xFFFFFFFF for v in leaf_ids], np.uint32, dev)
     sig_dev = device_table([float(v) for v in spec.sigmas], np.float32, dev)
-    a_ptrs, g_ptrs = _ptr_table(A_list, dev), _ptr_table(G_list, dev)
+    (a_ptrs, A_list), (g_ptrs, G_list) = _operand_table(A_list, dev), _operand_table(G_list, dev)
     out_ptrs = _ptr_table([out[e] for e in range(E)], dev)
     nat.call(
         "dpc_grouped_clipped_sum", nat.ptr(a_ptrs), nat.ptr(g_ptrs), nat.ptr(layout.rows_dev),
