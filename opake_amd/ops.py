@@ -31,14 +31,17 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t.clone(memory_format=torch.contiguous_format)
 
 
-def _operand(t: torch.Tensor) -> torch.Tensor:
-    """A layer's activations or output gradients, contiguous; bfloat16 rows of
-    whole 16-byte chunks, which the MFMA kernels move as such, start at one."""
+def _operand(t: torch.Tensor):
+    """A layer's activations or output gradients, contiguous, and their address;
+    bfloat16 rows of whole 16-byte chunks, which the MFMA kernels move as such,
+    start at one."""
     if not t.is_contiguous():
-        return t.contiguous()
-    if t.data_ptr() % 16 and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0:
-        return t.clone(memory_format=torch.contiguous_format)
-    return t
+        t = t.contiguous()
+    ptr = t.data_ptr()
+    if ptr % 16 and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0:
+        t = _aligned(t)
+        ptr = t.data_ptr()
+    return t, ptr
 
 
 def _wants_error(out, err, return_error):
@@ -96,7 +99,7 @@ def gram_sqnorms(
         raise ConfigurationError("A and G must share a dtype")
     B, T, din = A.shape
     dout = G.shape[2]
-    A, G = _operand(A), _operand(G)
+    (A, a_ptr), (G, g_ptr) = _operand(A), _operand(G)
     accumulate = out is not None
     with_err = _wants_error(out, err, return_error)
     if out is None:
@@ -110,7 +113,7 @@ def gram_sqnorms(
         ws_bytes = nat.load().dpc_gram_layer_workspace_bytes(B, T, din, dout, code, bias)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         nat.call(
-            "dpc_gram_sqnorms", nat.ptr(A), nat.ptr(G), B, T, din, dout, code, bias,
+            "dpc_gram_sqnorms", a_ptr, g_ptr, B, T, din, dout, code, bias,
             int(accumulate), nat.ptr(out), nat.ptr(err if with_err else None), nat.ptr(ws),
             ws_bytes, nat.stream_handle(dev),
         )
@@ -150,8 +153,8 @@ def gram_sqnorms_multi(
     if with_err:
         err = _error_out(err, B, dev, accumulate)
     if B > 0:
-        As = [_operand(A) for A in A_list]
-        Gs = [_operand(G) for G in G_list]
+        As, a_ptrs = zip(*[_operand(A) for A in A_list])
+        Gs, g_ptrs = zip(*[_operand(G) for G in G_list])
         c_din = (ctypes.c_int * n)(*[A.shape[2] for A in As])
         c_dout = (ctypes.c_int * n)(*[G.shape[2] for G in Gs])
         ws_bytes = nat.load().dpc_gram_sqnorms_multi_workspace_bytes(
@@ -159,10 +162,9 @@ def gram_sqnorms_multi(
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         vp = ctypes.c_void_p * n
         nat.call(
-            "dpc_gram_sqnorms_multi", n, vp(*[t.data_ptr() for t in As]),
-            vp(*[t.data_ptr() for t in Gs]), c_din, c_dout, B, T, nat.dtype_code(dtype),
-            int(accumulate), nat.ptr(out), nat.ptr(err if with_err else None), nat.ptr(ws),
-            ws_bytes, nat.stream_handle(dev),
+            "dpc_gram_sqnorms_multi", n, vp(*a_ptrs), vp(*g_ptrs), c_din, c_dout, B, T,
+            nat.dtype_code(dtype), int(accumulate), nat.ptr(out),
+            nat.ptr(err if with_err else None), nat.ptr(ws), ws_bytes, nat.stream_handle(dev),
         )
     return (out, err) if with_err else out
 
@@ -390,7 +392,7 @@ def gram_clip_factors(
         return sq, err, cf
     B, T, din = A.shape
     dout = G.shape[2]
-    A, G = _operand(A), _operand(G)
+    (A, a_ptr), (G, g_ptr) = _operand(A), _operand(G)
     n = len(guards)
     rel = (ctypes.c_double * n)(*[g[0] for g in guards])
     abs_ = (ctypes.c_double * n)(*[g[1] for g in guards])
@@ -406,7 +408,7 @@ def gram_clip_factors(
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         counters = _gram_clip_counters(dev, stream, lib.dpc_gram_clip_counter_bytes(B, T))
         nat.call(
-            "dpc_gram_clip_factors", nat.ptr(A), nat.ptr(G), B, T, din, dout, code,
+            "dpc_gram_clip_factors", a_ptr, g_ptr, B, T, din, dout, code,
             bias, float(clipping_norm), kind, float(gamma),
             rel, abs_, mult, n, float(count_threshold), nat.ptr(sq), nat.ptr(err),
             nat.ptr(cf.scale), nat.ptr(cf.scale64), nat.ptr(cf.norms), nat.ptr(cf.nclipped),
@@ -458,7 +460,7 @@ def clipped_sum(
     if scale.dtype != torch.float32 or scale.numel() < B:
         raise ConfigurationError("scale must be float32 with B entries")
     out_dtype = out_dtype or A.dtype
-    A, G = _operand(A), _operand(G)
+    (A, a_ptr), (G, g_ptr) = _operand(A), _operand(G)
     out = torch.empty((dout, din), dtype=out_dtype, device=dev)
     bias_out = torch.empty(dout, dtype=out_dtype, device=dev) if with_bias else None
     ws_bytes = nat.load().dpc_clipped_sum_workspace_bytes(B, T, din, dout, nat.dtype_code(A.dtype))
@@ -473,7 +475,7 @@ def clipped_sum(
             if t is None or t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_cuda:
                 raise ConfigurationError(f"injected noise must be float32 {shape} on the device")
     nat.call(
-        "dpc_clipped_sum", nat.ptr(A), nat.ptr(G), nat.ptr(_contig(scale)), nat.ptr(plan), B, T,
+        "dpc_clipped_sum", a_ptr, g_ptr, nat.ptr(_contig(scale)), nat.ptr(plan), B, T,
         din, dout, nat.dtype_code(A.dtype), float(normalize_by), spec.mode,
         nat.ptr(spec.noise), nat.ptr(spec.bias_noise), spec.seed & ((1 << 64) - 1),
         spec.leaf_id & 0xFFFFFFFF, spec.bias_leaf_id & 0xFFFFFFFF, float(spec.sigma), nat.dtype_code(out_dtype), nat.ptr(out),
@@ -554,8 +556,8 @@ def clipped_sum_multi(
                   for sp in noises]
         return [clipped_sum(A, G, scale, plan=plan, normalize_by=normalize_by, noise=sp,
                             out_dtype=out_dtype)[0] for A, G, sp in zip(A_list, G_list, noises)]
-    As = [_operand(A) for A in A_list]
-    Gs = [_operand(G) for G in G_list]
+    As, a_ptrs = zip(*[_operand(A) for A in A_list])
+    Gs, g_ptrs = zip(*[_operand(G) for G in G_list])
     outs = [torch.empty((o, i), dtype=out_dtype, device=dev) for i, o in zip(dins, douts)]
     sig = [sp.sigma if sp is not None else 0.0 for sp in noises]
     zs = []
@@ -569,7 +571,7 @@ def clipped_sum_multi(
         zs.append(z)
     vp = ctypes.c_void_p * n
     nat.call(
-        "dpc_clipped_sum_multi", n, vp(*[t.data_ptr() for t in As]), vp(*[t.data_ptr() for t in Gs]),
+        "dpc_clipped_sum_multi", n, vp(*a_ptrs), vp(*g_ptrs),
         (ctypes.c_int * n)(*dins), (ctypes.c_int * n)(*douts), nat.ptr(_contig(scale)),
         nat.ptr(plan), B, T, nat.dtype_code(dtype), float(normalize_by), mode,
         vp(*[z.data_ptr() if z is not None else None for z in zs]), seed & ((1 << 64) - 1),
@@ -797,8 +799,7 @@ def _operand_table(tensors, device):
     points into: copies of those that :func:`_operand` copies."""
     ptrs = [t.data_ptr() for t in tensors]
     if any(p % 16 for p in ptrs):
-        tensors = [_operand(t) for t in tensors]
-        ptrs = [t.data_ptr() for t in tensors]
+        tensors, ptrs = zip(*[_operand(t) for t in tensors])
     return device_table(ptrs, np.int64, device), tensors
 
 
