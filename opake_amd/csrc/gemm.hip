@@ -1640,8 +1640,8 @@ __global__ void __launch_bounds__(kThreads, 2) clipped_sum_f32_kernel(F32Args<In
 // split-K are worth (its matrix rate is 16 times higher): B, T, din, dout = 4,
 // 24, 64, 96 takes 10 us here and 20 there (both with their launches), 8, 20,
 // 63, 65 12 and 28, 64, 2, 1024, 1024 22 and 40, 16, 128, 512, 512 (1.1 GFLOP)
-// 24 and 26, 16, 100, 1023, 511 (1.7) 33 and 38, but 32, 100, 768, 768 (3.8) 66
-// and 35; 256 tokens of one example each, 512 x 512, 18, and 1024 of 2048 x 2048
+// 24 and 26, but 32, 100, 768, 768 (3.8) 66 and 35 (padded copies move the
+// crossing up: 16, 100, 1023, 511 (1.7) 33 and 38, past the line all the same); 256 tokens of one example each, 512 x 512, 18, and 1024 of 2048 x 2048
 // 101 (15 and 580 in the generic kernel).
 bool f32_widths(int B, int din, int dout) {
   return B > 0 && din >= 4 && dout >= 4 && din < (1 << 26) && dout < (1 << 26);
@@ -1653,7 +1653,8 @@ bool f32_shape(int B, int T, int din, int dout, int dtype) {
 }
 
 // Workgroups per tile of the fp32 path: enough for two on every CU, each of a
-// wave's slices at least 64 rows.
+// wave's slices at least 64 rows.  Rounds are not counted: the 576 tiles of 1536 x
+// 1536 go unsplit to 512 places.
 int f32_splits(int B, int T, int din, int dout) {
   const long long tiles = (long long)ceil_div(din, kF32Tile) * ceil_div(dout, kF32Tile);
   const long long K = (long long)B * T;

@@ -1776,8 +1776,8 @@ gram_generic_kernel(const In* __restrict__ A, const In* __restrict__ G, int T, i
 }
 
 // Dense fp64 MFMA path (fp32 operands, and bf16 shapes off the bf16 MFMA path,
-// where gram_f64_route takes it): products of fp32 values are exact in fp64, and the 16x16x4 fp64 MFMA
-// sums them, so the error model is that of a fp64 chain.
+// where gram_f64_route takes it): products of fp32 values are exact in fp64, and
+// the 16x16x4 fp64 MFMA sums them, so the error model is that of a fp64 chain.
 //
 // A workgroup computes one pair (p, q) of 32-row tiles of both Gram matrices:
 // waves 0, 1 the tile of A A^T, waves 2, 3 that of G G^T, as 2 x 2 blocks of

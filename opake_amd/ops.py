@@ -544,7 +544,9 @@ def clipped_sum_multi(
     # calls (the fp32 kernel, in which a short example does not fill a 64-row
     # step): 14 of 24 x 48 at [330, 6] (330 steps) 609 -> 306 us, of 16 x 2048
     # 626 -> 350 us, 2 of 24 x 48 at [40, 6] (40) 51 -> 38 us; 7 of 24 x 48 at
-    # [110, 6] (110) would lose by a factor of 1.4.
+    # [110, 6] (110) would lose by a factor of 1.4.  Both lines lie on the safe
+    # side: 14 of 512 x 512 at [8, 2000] (256) share in 744 us, their own calls
+    # take 546; 7 of 1024 x 1024 at [64, 500] (112 tiles) 716 and 556.
     steps = B * -(-T // 64)
     if mfma and n > 1 and steps >= 16 * n:
         small = all(2 * B * T * i * o < 3e8 for i, o in zip(dins, douts))

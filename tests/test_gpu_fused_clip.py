@@ -3,9 +3,10 @@ layer in one launch (the split Gram kernel's last work item folds the
 records and computes the clip factors).  Against the two-call path
 (``dpc_gram_sqnorms`` then ``dpc_clip_factors``), bit for bit, on call after
 call on one workspace (each call must leave its tickets zero for the next),
-for fixed and AUTO-S scales, several guards, and the shapes that take the
-separate launches inside the entry point (a bias, an odd number of 128-row
-blocks, float32) interleaved with one-launch calls.
+for fixed and AUTO-S scales, several guards, a bias (its column sums in a launch
+before, its counters in the workspace), and the shapes that take the separate
+launches inside the entry point (an odd number of 128-row blocks, float32)
+interleaved with one-launch calls.
 """
 
 from __future__ import annotations
@@ -49,11 +50,11 @@ def _two_calls(A, G, C, guards, bias, kind, gamma):
 
 
 CASES = [
-    # B, T, din, dout, dtype, bias: one launch, then the separate launches
+    # B, T, din, dout, dtype, bias
     (32, 512, 512, 384, torch.bfloat16, False),
     (8, 256, 256, 256, torch.bfloat16, False),
     (4, 384, 128, 256, torch.bfloat16, False),   # odd block count: separate launches
-    (6, 256, 128, 64, torch.bfloat16, True),     # bias: separate launches
+    (6, 256, 128, 64, torch.bfloat16, True),     # bias: column sums, then one launch
     (5, 130, 72, 40, torch.float32, False),      # float32: separate launches
     (32, 512, 512, 384, torch.bfloat16, False),  # one launch again on the same workspace
     (16, 1024, 256, 512, torch.bfloat16, False),

@@ -1,5 +1,9 @@
-"""The bf16 clipped sum at token counts that no 64-row step divides and at
-widths that are not multiples of 8 (GPU tests, called through the C ABI)."""
+"""Layers off the usual shapes (GPU tests): token counts that no 64-row step
+divides, widths that are not multiples of 8, operands that start at any element,
+float32, few tiles over a long K, narrow layers, biases, small batches; clipped
+sums, Gram norms and clip factors, one layer and several, and materialised leaves
+of any alignment.  Through the package's wrappers and, where they hide the choice,
+the C ABI."""
 
 from __future__ import annotations
 
